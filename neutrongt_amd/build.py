@@ -40,8 +40,11 @@ HIPCC_FLAGS = [
 # (masked keys are -inf, every tile's running maximum is finite), so they run
 # with the IEEE-mode bit off: fmaxf then needs no canonicalising v_max of each
 # MFMA result (9 of the forward's 77 VALU instructions per 32 x 32 score tile).
+# The fp32 ones take the same flags for the same reason; a NaN input still goes
+# through their arithmetic to the outputs that depend on it.
 FILE_FLAGS = {
     "ngt_dense_mfma.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
+    "ngt_dense_f32.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
 }
 
 

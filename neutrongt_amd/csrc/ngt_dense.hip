@@ -41,6 +41,19 @@ int mfma_dense_bwd(int d, const void* q, const void* k, const void* v, const voi
                    const void* out, const float* out32, const float* lse, float* dsum, int n_q,
                    int n_k, int H, float scale, const DropoutMask* dm, void* gq, void* gk, void* gv,
                    MfSplit sq, float* part_dq, int fused_blocks, hipStream_t st);
+// fp32 matrix-core kernels (ngt_dense_f32.hip).
+MfSplit f32_fwd_split(int n_q, int n_k, int H, int d, bool node_scores);
+MfSplit f32_dq_split(int n_q, int n_k, int H, int d);
+size_t f32_fwd_image_bytes(int n_q, int n_k, int H, int d);
+size_t f32_bwd_image_bytes(int n_q, int n_k, int H, int d);
+int f32_dense_fwd(int d, const float* q, const float* k, const float* v, int n_q, int n_k, int H,
+                  float scale, const DropoutMask* dm, float* out, float* out32, float* lse,
+                  float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
+                  hipStream_t st);
+int f32_dense_bwd(int d, const float* q, const float* k, const float* v, const float* go,
+                  const float* out, const float* lse, float* dsum, int n_q, int n_k, int H,
+                  float scale, const DropoutMask* dm, float* gq, float* gk, float* gv, MfSplit sq,
+                  float* part_dq, char* images, hipStream_t st);
 
 namespace {
 
@@ -842,39 +855,6 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* out, con
   return NGT_OK;
 }
 
-template <typename T, int DH>
-struct FwdOp {
-  template <typename... A>
-  static int run(A&&... a) {
-    return launch_fwd<T, DH>(std::forward<A>(a)...);
-  }
-};
-template <typename T, int DH>
-struct BwdOp {
-  template <typename... A>
-  static int run(A&&... a) {
-    return launch_bwd<T, DH>(std::forward<A>(a)...);
-  }
-};
-
-template <template <typename, int> class F, typename... Args>
-int dispatch(int dtype, int d, Args&&... args) {
-#define NGT_CASE(DH)                                                         \
-  case DH:                                                                   \
-    return dtype == NGT_F32 ? F<float, DH>::run(std::forward<Args>(args)...) \
-                            : F<bf16_t, DH>::run(std::forward<Args>(args)...);
-  switch (d) {
-    NGT_CASE(8)
-    NGT_CASE(16)
-    NGT_CASE(24)
-    NGT_CASE(32)
-    NGT_CASE(64)
-    default:
-      return set_error(NGT_ERR_UNSUPPORTED, "dense: head_dim=%d has no kernel", d);
-  }
-#undef NGT_CASE
-}
-
 int check_args(const char* fn, int dtype, int n_q, int n_k, int H, int d) {
   if (dtype != NGT_F32 && dtype != NGT_BF16)
     return set_error(NGT_ERR_ARG, "%s: unknown dtype %d", fn, dtype);
@@ -885,26 +865,25 @@ int check_args(const char* fn, int dtype, int n_q, int n_k, int H, int d) {
   return NGT_OK;
 }
 
-// The bf16 path runs on the matrix cores (ngt_dense_mfma.hip) for d <= 32;
-// NGT_DENSE_VALU=1 selects the vector-ALU kernels instead (for comparison).
+// fp32 runs on ngt_dense_f32.hip, bf16 with d <= 32 on ngt_dense_mfma.hip,
+// bf16 with d = 64 on the vector-ALU kernels of this file.
 bool use_mfma(int dtype, int d) {
-  static const bool valu = getenv("NGT_DENSE_VALU") != nullptr;
-  return dtype == NGT_BF16 && mfma_dense_supported(d) && !valu;
+  return dtype == NGT_F32 || mfma_dense_supported(d);
 }
 
-// Forward workspace: the matrix-core path needs H * n_k floats of node-score
-// partials (only with node scores); the vector-ALU path needs per-block
-// node-score partials (only with node scores) and, when it splits the keys,
-// the split states behind them.
-// The matrix-core path: [node-score partials H * n_k (with node scores)]
-// [split states (m, l) and unnormalised outputs (with a key split)].
+// Forward workspace of the matrix-core paths: [node-score partials H * n_k
+// (with node scores)][split states (m, l) and unnormalised outputs (with a
+// key split)][the operands' bf16 pieces (fp32)].  The vector-ALU path needs per-block node-score partials (only
+// with node scores) and, when it splits the keys, the split states behind them.
 struct MfFwdLayout {
-  size_t ml, acc, total;
+  size_t ml, acc, images, total;
   MfSplit sp;
 };
-MfFwdLayout mf_fwd_layout(int32_t n_q, int32_t n_k, int32_t H, int32_t d, bool node_scores) {
+MfFwdLayout mf_fwd_layout(int dtype, int32_t n_q, int32_t n_k, int32_t H, int32_t d,
+                          bool node_scores) {
   MfFwdLayout L{};
-  L.sp = mfma_fwd_split(n_q, n_k, H, node_scores);
+  L.sp = dtype == NGT_F32 ? f32_fwd_split(n_q, n_k, H, d, node_scores)
+                          : mfma_fwd_split(n_q, n_k, H, node_scores);
   size_t off = node_scores ? align256(size_t(H) * n_k * 4) : 0;
   if (L.sp.n_split > 1) {
     L.ml = off;
@@ -912,12 +891,14 @@ MfFwdLayout mf_fwd_layout(int32_t n_q, int32_t n_k, int32_t H, int32_t d, bool n
     L.acc = off;
     off += align256(size_t(L.sp.n_split) * n_q * H * d * 4);
   }
+  L.images = off;
+  if (dtype == NGT_F32) off += f32_fwd_image_bytes(n_q, n_k, H, d);
   L.total = off;
   return L;
 }
 
 size_t fwd_need(int dtype, int32_t n_q, int32_t n_k, int32_t H, int32_t d, bool node_scores) {
-  if (use_mfma(dtype, d)) return mf_fwd_layout(n_q, n_k, H, d, node_scores).total;
+  if (use_mfma(dtype, d)) return mf_fwd_layout(dtype, n_q, n_k, H, d, node_scores).total;
   return node_scores || key_split(n_q, n_k, H).n_split > 1 ? fwd_ws(n_q, n_k, H, d) : 0;
 }
 
@@ -927,21 +908,34 @@ size_t fwd_need(int dtype, int32_t n_q, int32_t n_k, int32_t H, int32_t d, bool 
 size_t bwd_need(int dtype, int32_t n_q, int32_t n_k, int32_t H, int32_t d) {
   size_t need = bwd_ws(n_q, H);
   if (use_mfma(dtype, d) && n_q > 0) {
-    const int fb = mfma_fused_blocks(n_q, n_k, H, d);
-    const MfSplit sq = mfma_dq_split(n_q, n_k, H);
+    const int fb = dtype == NGT_F32 ? 0 : mfma_fused_blocks(n_q, n_k, H, d);
+    const MfSplit sq = dtype == NGT_F32 ? f32_dq_split(n_q, n_k, H, d) : mfma_dq_split(n_q, n_k, H);
     const int parts = fb > 0 ? fb : (sq.n_split > 1 ? sq.n_split : 0);
     if (parts > 0) need += align256(size_t(parts) * n_q * H * d * 4);
   }
+  if (dtype == NGT_F32) need += f32_bwd_image_bytes(n_q, n_k, H, d);
   return need;
 }
 
-template <int DH>
-void launch_mf_combine(const float* part_ml, const float* part_acc, int n_split, int n_q, int H,
-                       void* out, float* out32, float* lse, hipStream_t st) {
+template <typename T>
+int launch_combine(int d, const float* part_ml, const float* part_acc, int n_split, int n_q, int H,
+                   void* out, float* out32, float* lse, hipStream_t st) {
+  KernelTimer timer_("dense_combine", st);
   int64_t blocks = (int64_t(n_q) * H + kBlock - 1) / kBlock;
   if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL((k_dense_combine<bf16_t, DH>), dim3(int(blocks)), dim3(kBlock), 0, st,
-                     part_ml, part_acc, n_split, n_q, H, static_cast<bf16_t*>(out), out32, lse);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(int(blocks)), dim3(kBlock), 0, st, part_ml, part_acc, n_split,
+                       n_q, H, static_cast<T*>(out), out32, lse);
+  };
+  switch (d) {
+    case 8: run(k_dense_combine<T, 8>); break;
+    case 16: run(k_dense_combine<T, 16>); break;
+    case 24: run(k_dense_combine<T, 24>); break;
+    case 32: run(k_dense_combine<T, 32>); break;
+    default: run(k_dense_combine<T, 64>); break;
+  }
+  NGT_HIP_CHECK(hipGetLastError());
+  return NGT_OK;
 }
 
 __global__ void k_fill_zero(float* __restrict__ p, int64_t n) {
@@ -993,31 +987,31 @@ extern "C" int ngt_dense_fwd(int dtype, const void* q, const void* k, const void
   if (use_mfma(dtype, head_dim)) {
     if (n_q == 0) return NGT_OK;
     float* part = node_score ? static_cast<float*>(workspace) : nullptr;
-    const MfFwdLayout L = mf_fwd_layout(n_q, n_k, n_heads, head_dim, node_score != nullptr);
+    const MfFwdLayout L =
+        mf_fwd_layout(dtype, n_q, n_k, n_heads, head_dim, node_score != nullptr);
     char* ws = static_cast<char*>(workspace);
     float* part_ml = L.sp.n_split > 1 ? reinterpret_cast<float*>(ws + L.ml) : nullptr;
     float* part_acc = L.sp.n_split > 1 ? reinterpret_cast<float*>(ws + L.acc) : nullptr;
-    rc = mfma_dense_fwd(head_dim, q, k, v, n_q, n_k, n_heads, scale, dm, out, out_f32, lse, part,
-                        L.sp, part_ml, part_acc, st);
+    if (dtype == NGT_F32)
+      rc = f32_dense_fwd(head_dim, static_cast<const float*>(q), static_cast<const float*>(k),
+                         static_cast<const float*>(v), n_q, n_k, n_heads, scale, dm,
+                         static_cast<float*>(out), out_f32, lse, part, L.sp, part_ml, part_acc,
+                         ws + L.images, st);
+    else
+      rc = mfma_dense_fwd(head_dim, q, k, v, n_q, n_k, n_heads, scale, dm, out, out_f32, lse, part,
+                          L.sp, part_ml, part_acc, st);
     if (rc != NGT_OK) return rc;
-    if (L.sp.n_split > 1) {
-      KernelTimer timer_("dense_combine", st);
-      switch (head_dim) {
-        case 8: launch_mf_combine<8>(part_ml, part_acc, L.sp.n_split, n_q, n_heads, out, out_f32, lse, st); break;
-        case 16: launch_mf_combine<16>(part_ml, part_acc, L.sp.n_split, n_q, n_heads, out, out_f32, lse, st); break;
-        case 24: launch_mf_combine<24>(part_ml, part_acc, L.sp.n_split, n_q, n_heads, out, out_f32, lse, st); break;
-        default: launch_mf_combine<32>(part_ml, part_acc, L.sp.n_split, n_q, n_heads, out, out_f32, lse, st); break;
-      }
-      NGT_HIP_CHECK(hipGetLastError());
-    }
+    if (L.sp.n_split > 1)
+      NGT_CHECK_OK((dtype == NGT_F32 ? launch_combine<float> : launch_combine<bf16_t>)(
+          head_dim, part_ml, part_acc, L.sp.n_split, n_q, n_heads, out, out_f32, lse, st));
     if (!node_score || n_k == 0) return NGT_OK;
     hipLaunchKernelGGL(k_dense_scores, dim3((n_k + kWave - 1) / kWave), dim3(kScoreThreads), 0, st,
                        part, n_heads, n_k, n_heads, node_score);
     NGT_HIP_CHECK(hipGetLastError());
     return NGT_OK;
   }
-  return dispatch<FwdOp>(dtype, head_dim, q, k, v, int(n_q), int(n_k), int(n_heads), scale, dm,
-                         out, out_f32, lse, node_score, static_cast<char*>(workspace), st);
+  return launch_fwd<bf16_t, 64>(q, k, v, n_q, n_k, n_heads, scale, dm, out, out_f32, lse,
+                                node_score, static_cast<char*>(workspace), st);
 }
 
 extern "C" int ngt_dense_bwd(int dtype, const void* q, const void* k, const void* v,
@@ -1045,15 +1039,26 @@ extern "C" int ngt_dense_bwd(int dtype, const void* q, const void* k, const void
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (use_mfma(dtype, head_dim)) {
     float* dsum = static_cast<float*>(workspace);  // written by the dQ pass
-    const MfSplit sq = n_q > 0 ? mfma_dq_split(n_q, n_k, n_heads) : MfSplit{1, 1};
-    const int fb = mfma_fused_blocks(n_q, n_k, n_heads, head_dim);
+    const bool f32 = dtype == NGT_F32;
+    const MfSplit sq = n_q == 0 ? MfSplit{1, 1}
+                       : f32    ? f32_dq_split(n_q, n_k, n_heads, head_dim)
+                                : mfma_dq_split(n_q, n_k, n_heads);
+    const int fb = f32 ? 0 : mfma_fused_blocks(n_q, n_k, n_heads, head_dim);
     float* part_dq = sq.n_split > 1 || fb > 0
                          ? reinterpret_cast<float*>(static_cast<char*>(workspace) + bwd_ws(n_q, n_heads))
                          : nullptr;
+    if (f32) {
+      char* images = static_cast<char*>(workspace) + need - f32_bwd_image_bytes(n_q, n_k, n_heads, head_dim);
+      return f32_dense_bwd(head_dim, static_cast<const float*>(q), static_cast<const float*>(k),
+                           static_cast<const float*>(v), static_cast<const float*>(grad_out),
+                           out_f32 ? out_f32 : static_cast<const float*>(out), lse, dsum, n_q, n_k,
+                           n_heads, scale, dm, static_cast<float*>(grad_q),
+                           static_cast<float*>(grad_k), static_cast<float*>(grad_v), sq, part_dq,
+                           images, st);
+    }
     return mfma_dense_bwd(head_dim, q, k, v, grad_out, out, out_f32, lse, dsum, n_q, n_k,
                           n_heads, scale, dm, grad_q, grad_k, grad_v, sq, part_dq, fb, st);
   }
-  return dispatch<BwdOp>(dtype, head_dim, q, k, v, out, out_f32, grad_out, lse, int(n_q), int(n_k),
-                         int(n_heads), scale, dm, grad_q, grad_k, grad_v,
-                         static_cast<char*>(workspace), st);
+  return launch_bwd<bf16_t, 64>(q, k, v, out, out_f32, grad_out, lse, n_q, n_k, n_heads, scale, dm,
+                                grad_q, grad_k, grad_v, static_cast<char*>(workspace), st);
 }

@@ -1,0 +1,1297 @@
+// Dense full-window attention in fp32 on the matrix cores, head_dim d in
+// {8, 16, 24, 32, 64}.
+//
+// Products.  An fp32 value is the sum of three bf16 pieces h + m + l (each the
+// round-to-nearest of what is left, so the last remainder is zero or below
+// 2^-24 of the value).  A product of two such values is hh + (hm + mh) +
+// (mm + hl + lh) up to 2^-24, and v_mfma_f32_16x16x32_bf16 multiplies pieces
+// exactly, adds 8 products at a time exactly and rounds to fp32 once per 8
+// (checked on gfx950), so a contraction loses less than an fp32 FMA chain.
+// At d = 8 a 32 x 32 tile of S takes 128 cycles of bf16 MFMAs where fp32 ones
+// take 256, and they leave the vector ALU to the exponentials: the fp32 MFMAs
+// do not overlap with vector instructions here (dK/dV at 16,000 nodes, 8
+// heads, d = 8: 1,536 MFMA cycles and 800 of vector work per tile ran 2,330
+// cycles).  What bounds the kernels is the vector work per score (dK/dV: 320
+// vector instructions per tile): the exponential, the split of P (and dS) into
+// pieces and, with dropout, the hash.
+// Measured (us per launch, forward with node scores / dK/dV / dQ; the earlier
+// one-row-per-lane vector kernels -> these): 16,000 nodes, 8 heads, d = 8
+// 1,720 / 2,490 / 1,680 -> 1,060 / 1,780 / 1,030, with dropout 0.5 2,150 /
+// 2,810 / 1,980 -> 1,400 / 2,215 / 1,370; all-fp32 MFMAs 1,390 / 1,900 /
+// 1,300.  5,000 nodes, 8 heads, d = 64: 8,400 in all -> 650 / 1,210 / 555.
+//
+// A preparation kernel (k_fx_prep) writes the pieces of q * scale, k, v and dO
+// once per call, in the layout the LDS stages have:
+//   row image: per row 3 pieces x d / 8 blocks of 8 columns (16 bytes each),
+//     read as A and B operands of S and dP;
+//   transposed image: per 32 rows, one line per (piece, column) with the 32
+//     rows in the order a lane needs them, read as A operands of the products
+//     over rows.
+// Lane layouts (g = lane / 16, l = lane % 16; checked on gfx950):
+//   A (16 x 32): lane holds A[l][8 g + j], B (32 x 16): B[8 g + j][l], j < 8;
+//   D (16 x 16): lane holds D[4 g + i][l], i < 4.
+// A contraction's index order is free as long as A and B share it: two score
+// tiles (32 streamed rows) give lane (l, g) the rows 4 g + i of both, and those
+// 8 values, split, are the B operand of the next product as they stand.
+//
+// The lanes' side (queries in the forward and dQ pass, keys in the dK/dV
+// pass) is the tiles' column, so per-row state (running maximum, sum, lse, D)
+// sits in one register per lane; the other side is staged in LDS with line
+// lengths that are odd multiples of 16 bytes (16 lanes on 16 bank groups).
+// Outputs come out transposed, 4 consecutive columns of a lane's row.
+//
+// Pieces of an infinity or a NaN would turn products with zero pieces into
+// NaN, so a head whose inputs hold one (or a value past 2^125) runs the same
+// kernels' other body, with v_mfma_f32_16x16x4_f32: plain fp32 FMA chains.
+#include "ngt_common.h"
+
+#include <math.h>
+#include <stdlib.h>
+
+#include <algorithm>
+
+namespace ngt {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Ids as register reads: this file is built with the IEEE mode bit off, and
+// the device library's functions behind threadIdx / blockIdx are not inlined
+// across that difference (each use would be a call).
+__device__ __forceinline__ int tid_x() { return static_cast<int>(__builtin_amdgcn_workitem_id_x()); }
+__device__ __forceinline__ int wg_x() { return static_cast<int>(__builtin_amdgcn_workgroup_id_x()); }
+__device__ __forceinline__ int wg_y() { return static_cast<int>(__builtin_amdgcn_workgroup_id_y()); }
+__device__ __forceinline__ int wg_z() { return static_cast<int>(__builtin_amdgcn_workgroup_id_z()); }
+
+constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / kWave;
+constexpr int kT = 16;     // MFMA tile edge
+constexpr int kStep = 32;  // streamed rows per step of a wave (two tiles)
+constexpr int kPadRows = 64;  // the images' rows come in multiples of this
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
+constexpr float kRebase = 5.5f;  // forward: P entries stay below e^5.5 (fp32 sums)
+constexpr float kHuge = 4.2535296e37f;  // 2^125: values past it take the fp32 MFMAs
+
+// Rows (queries or keys) a block owns with G tiles per wave.
+constexpr int block_rows(int G) { return kWaves * kT * G; }
+constexpr int out_tiles(int dh) { return (dh + 15) / 16; }
+// Row image: bytes per row (3 pieces x blocks of 8 columns, d = 24 padded to
+// 4 blocks, the line length an odd multiple of 16).
+constexpr int col_blocks(int dh) { return dh == 24 ? 4 : dh / 8; }
+constexpr int row_bytes(int dh) {
+  const int units = 3 * col_blocks(dh);
+  return 16 * (units % 2 ? units : units + 1);
+}
+// Transposed image: lines per 32 rows, one per (piece, column) in whole
+// 16-line tiles; at d = 8 the first tile holds pieces h and m, the second l.
+constexpr int t_lines(int dh) { return dh == 8 ? 32 : 3 * 16 * out_tiles(dh); }
+constexpr int kTLine = 80;  // 32 bf16 and 16 bytes of padding
+constexpr int t_bytes(int dh) { return t_lines(dh) * kTLine; }
+__host__ __device__ inline int padded(int n) { return (n + kPadRows - 1) / kPadRows * kPadRows; }
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 zero4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
+__device__ __forceinline__ float exp_nat(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
+
+// x combined over the four 16-lane rows of the wave (the lanes of one column).
+__device__ __forceinline__ float sum_halves(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+__device__ __forceinline__ float sum_rows(float x) {
+  x = sum_halves(x);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ float max_rows(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// The dropout word of lane ^ 1 (DPP quad_perm 1,0,3,2).
+__device__ __forceinline__ uint32_t swap_pair(uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0xB1, 0xF, 0xF, true));
+}
+
+// Two floats' next pieces, packed; x0, x1 become the remainders (exact).
+// NEAREST: pieces rounded to nearest (the operands, once per call), so that
+// the products left out are signed and below 2^-24.  Else the leading 16 bits
+// (P and dS, per score): a mask and a subtraction at the vector ALU's double
+// rate (2.5 cycles each; conversions and shifts take 4.4).  Either way three
+// pieces hold all 24 bits.
+template <bool NEAREST>
+__device__ __forceinline__ uint32_t peel2(float& x0, float& x1) {
+  if constexpr (NEAREST) {
+    const uint32_t w = pack2_bf16(x0, x1);
+    x0 -= __uint_as_float(w << 16);
+    x1 -= __uint_as_float(w & 0xffff0000u);
+    return w;
+  } else {
+    const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+    x0 -= __uint_as_float(u0 & 0xffff0000u);
+    x1 -= __uint_as_float(u1 & 0xffff0000u);
+    return __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the two upper halves
+  }
+}
+struct Split {
+  bf16x8 h, m, l;
+};
+template <bool NEAREST>
+__device__ __forceinline__ Split split8(float (&x)[8]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[n][j] = peel2<NEAREST>(x[2 * j], x[2 * j + 1]);
+  return {__builtin_bit_cast(bf16x8, make_uint4(w[0][0], w[0][1], w[0][2], w[0][3])),
+          __builtin_bit_cast(bf16x8, make_uint4(w[1][0], w[1][1], w[1][2], w[1][3])),
+          __builtin_bit_cast(bf16x8, make_uint4(w[2][0], w[2][1], w[2][2], w[2][3]))};
+}
+
+// Dropout: 1 / (1 - p) rides in the staged V (forward) and dO (backward), so a
+// score only keeps or clears its value.  bits: the 16-bit draw in the upper
+// half (the lower half is the other key's and cannot change the comparison
+// with thr << 16).
+__device__ __forceinline__ bool kept(uint32_t bits, uint32_t thr16) { return bits >= thr16; }
+
+// One operand matrix [n, H, d]: its fp32 rows and, per head, the images.
+struct Mat {
+  const float* x;
+  const char* row_img;  // [H][padded(n)][row_bytes]
+  const char* t_img;    // [H][padded(n) / 32][t_bytes]
+  const uint32_t* flag; // [H][padded(n) / 32]: nonzero where a value takes the fp32 body
+  int32_t n;
+  float scale;          // applied to x before anything else
+};
+
+// -------------------------------------------------------------- preparation
+struct PrepJob {
+  const float* x;
+  char* row_img;
+  char* t_img;  // null: not wanted
+  uint32_t* flag;
+  int32_t n;
+  float scale;
+};
+struct PrepJobs {
+  PrepJob j[4];
+};
+
+// Block (step of 32 rows, head, matrix): both images of the step's rows and
+// the flag word.  Rows past n are zero.
+template <int DH>
+__global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t H) {
+  const PrepJob job = jobs.j[wg_z()];
+  const int step = wg_x(), h = wg_y();
+  const int n_pad = padded(job.n);
+  if (step * kStep >= n_pad) return;
+  __shared__ float xs[kStep][DH + 1];
+  int bad = 0;
+  for (int e = tid_x(); e < kStep * DH; e += kBlock) {
+    const int r = e / DH, c = e - r * DH;
+    const int64_t row = int64_t(step) * kStep + r;
+    const float v = row < job.n ? job.x[(row * H + h) * DH + c] * job.scale : 0.f;
+    xs[r][c] = v;
+    // (an unordered compare on the bits: this file does not honour NaNs)
+    bad |= (__float_as_uint(v) & 0x7fffffffu) > __float_as_uint(kHuge);
+  }
+  bad = __syncthreads_or(bad);
+  if (tid_x() == 0) job.flag[int64_t(h) * (n_pad / kStep) + step] = bad ? 1u : 0u;
+  constexpr int NB = col_blocks(DH);
+  for (int e = tid_x(); e < kStep * NB; e += kBlock) {
+    const int r = e / NB, cb = e - r * NB;
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = 8 * cb + j < DH ? xs[r][(8 * cb + j) % DH] : 0.f;
+    const Split sp = split8<true>(x);
+    char* p = job.row_img + (int64_t(h) * n_pad + step * kStep + r) * row_bytes(DH) + 16 * cb;
+    *reinterpret_cast<bf16x8*>(p) = sp.h;
+    *reinterpret_cast<bf16x8*>(p + 16 * NB) = sp.m;
+    *reinterpret_cast<bf16x8*>(p + 32 * NB) = sp.l;
+  }
+  if (!job.t_img) return;
+  constexpr int PL = DH == 8 ? 8 : 16 * out_tiles(DH);  // lines per piece
+  char* t = job.t_img + (int64_t(h) * (n_pad / kStep) + step) * t_bytes(DH);
+  for (int e = tid_x(); e < 4 * PL; e += kBlock) {
+    const int c = e / 4, gg = e - 4 * c;
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      x[j] = c < DH ? xs[kT * (j / 4) + 4 * gg + j % 4][c < DH ? c : 0] : 0.f;
+    const Split sp = split8<true>(x);
+    char* p = t + c * kTLine + 16 * gg;
+    *reinterpret_cast<bf16x8*>(p) = sp.h;
+    *reinterpret_cast<bf16x8*>(p + PL * kTLine) = sp.m;
+    *reinterpret_cast<bf16x8*>(p + 2 * PL * kTLine) = sp.l;
+    if constexpr (DH == 8)  // the last 8 lines of the second tile
+      *reinterpret_cast<uint4*>(p + 3 * PL * kTLine) = make_uint4(0u, 0u, 0u, 0u);
+  }
+}
+
+// Whether any step of head h of these matrices takes the fp32 body (the same
+// answer in every thread of the block).
+__device__ __forceinline__ bool any_flag(const Mat& a, const Mat& b, const Mat& c, int h) {
+  int bad = 0;
+  const Mat* m[3] = {&a, &b, &c};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int steps = padded(m[i]->n) / kStep;
+    for (int t = tid_x(); t < steps; t += kBlock) bad |= int(m[i]->flag[int64_t(h) * steps + t]);
+  }
+  return __syncthreads_or(bad) != 0;
+}
+
+// ------------------------------------------------------- fp32 MFMA products
+// A lane's d / 4 floats of row p, columns (d / 4) g ..
+template <int DH>
+__device__ __forceinline__ void load_quarter(const float* p, float (&x)[DH / 4]) {
+  constexpr int KC = DH / 4;
+  if constexpr (KC % 4 == 0) {
+#pragma unroll
+    for (int j = 0; j < KC; j += 4) {
+      const float4 w = *reinterpret_cast<const float4*>(p + j);
+      x[j] = w.x, x[j + 1] = w.y, x[j + 2] = w.z, x[j + 3] = w.w;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < KC; j += 2) {
+      const float2 w = *reinterpret_cast<const float2*>(p + j);
+      x[j] = w.x, x[j + 1] = w.y;
+    }
+  }
+}
+
+// Rows are staged as they are, LD floats apart, and serve both kinds of
+// product (an A operand of the products over rows is a column of 4 rows).  At
+// d = 8 and 24 the last tile's columns past d read the floats that follow and
+// end in registers that nothing stores.
+template <int DH, int G>
+struct Fp32Ops {
+  static constexpr int SB = DH > 32 ? 32 : 64;
+  static constexpr int LD = DH + 4;
+  static constexpr int MT = out_tiles(DH);
+  struct Rows {
+    float x[G][DH / 4];
+  };
+  static __device__ __forceinline__ void load_rows(Rows& r, int u, const Mat& m, int64_t row, int h,
+                                                   int H, int g) {
+#pragma unroll
+    for (int j = 0; j < DH / 4; ++j) r.x[u][j] = 0.f;
+    if (row < m.n) load_quarter<DH>(m.x + (row * H + h) * DH + (DH / 4) * g, r.x[u]);
+#pragma unroll
+    for (int j = 0; j < DH / 4; ++j) r.x[u][j] *= m.scale;
+  }
+  template <bool ROW, bool COL>
+  struct Staged {
+    static constexpr int BYTES = (SB * LD + 16) * 4;
+    static constexpr int VPR = DH / 4;
+    static constexpr int NV = (SB * VPR + kBlock - 1) / kBlock;
+    float* lds;
+    float4 w[NV];
+    __device__ __forceinline__ void load(const Mat& m, int row0, int h, int H) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = tid_x() + i * kBlock;
+        const int r = e / VPR, c = e - r * VPR;
+        w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (e < SB * VPR && row0 + r < m.n)
+          w[i] = *reinterpret_cast<const float4*>(m.x + (int64_t(row0 + r) * H + h) * DH + 4 * c);
+        w[i] = make_float4(w[i].x * m.scale, w[i].y * m.scale, w[i].z * m.scale, w[i].w * m.scale);
+      }
+    }
+    __device__ __forceinline__ void store() const {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int e = tid_x() + i * kBlock;
+        const int r = e / VPR, c = e - r * VPR;
+        if (e < SB * VPR) *reinterpret_cast<float4*>(lds + r * LD + 4 * c) = w[i];
+      }
+    }
+    // X[t][u] = M R[u]^T for the 16-row tiles t at LDS row r0; chains of two
+    // MFMAs meet in a tree
+    __device__ __forceinline__ void products(int r0, int g, int l16, const Rows& rows,
+                                             f32x4 (&x)[2][G]) const {
+      constexpr int NCH = DH / 8;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float a[DH / 4];
+        load_quarter<DH>(lds + (r0 + kT * t + l16) * LD + (DH / 4) * g, a);
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          f32x4 c[NCH];
+#pragma unroll
+          for (int n = 0; n < NCH; ++n)
+            c[n] = mfma4(a[2 * n + 1], rows.x[u][2 * n + 1],
+                         mfma4(a[2 * n], rows.x[u][2 * n], zero4()));
+#pragma unroll
+          for (int v = 1; v < NCH; v *= 2)
+#pragma unroll
+            for (int n = 0; n + v < NCH; n += 2 * v) c[n] += c[n + v];
+          x[t][u] = c[0];
+        }
+      }
+    }
+    // acc[u] (columns x lanes, transposed) += M^T X[u] over 32 rows
+    __device__ __forceinline__ void accumulate(int r0, int g, int l16, const f32x4 (&x)[2][G],
+                                               f32x4 (&acc)[G][MT]) const {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) {
+            const float a = lds[(r0 + kT * t + 4 * g + i) * LD + kT * m + l16];
+#pragma unroll
+            for (int u = 0; u < G; ++u) acc[u][m] = mfma4(a, x[t][u][i], acc[u][m]);
+          }
+    }
+  };
+  static __device__ __forceinline__ void finish(f32x4 (&)[G][MT]) {}
+};
+
+// ------------------------------------------------------ bf16-piece products
+// S and dP contract the columns of two rows' pieces.  A lane's operand is 16
+// bytes of a row image, its 16-byte unit chosen by (operand number, g): the
+// MFMAs of a tile pair A and B operands so that, over the four g, every piece
+// product down to 2^-16 is there once; the smallest come first.
+template <int DH>
+struct Pairs {
+  static constexpr int NA = DH == 8 ? 2 : DH == 64 ? 6 : 3;   // A operands
+  static constexpr int NB = DH <= 16 ? 2 : DH == 64 ? 6 : 3;  // B operands
+  static constexpr int N = DH == 8 ? 2 : DH == 16 ? 3 : DH == 64 ? 12 : 6;
+  // the N MFMAs, smallest products first
+  static constexpr __host__ __device__ int a_of(int n) {
+    if constexpr (DH == 8) return 1 - n;        // [h l m l] x [l h l m], [h h m m] x [h m h m]
+    else if constexpr (DH == 16) return 2 - n;  // [h l] x [l h], [m m] x [h m], [h h] x [h m]
+    else {
+      constexpr int a[6] = {2, 0, 1, 1, 0, 0};
+      return DH == 64 ? 2 * a[n / 2] + n % 2 : a[n];
+    }
+  }
+  static constexpr __host__ __device__ int b_of(int n) {
+    if constexpr (DH == 8) return 1 - n;
+    else if constexpr (DH == 16) return n == 0 ? 1 : 0;
+    else {
+      constexpr int b[6] = {0, 2, 1, 0, 1, 0};
+      return DH == 64 ? 2 * b[n / 2] + n % 2 : b[n];
+    }
+  }
+  // byte offset of operand k of a lane's row
+  static __device__ __forceinline__ int unit(bool b, int k, int g) {
+    constexpr int CB = col_blocks(DH);
+    if constexpr (DH == 8) {
+      const int first = b ? (g & 1) : (g >> 1);                              // hmhm / hhmm
+      const int second = b ? (g == 1 ? 0 : g == 3 ? 1 : 2) : (g == 0 ? 0 : g == 2 ? 1 : 2);
+      return 16 * (k == 0 ? first : second);
+    } else if constexpr (DH == 16) {
+      const int hi = g >> 1;  // the second two lane groups
+      const int piece = b ? (k == 0 ? hi : (hi ? 0 : 2))                      // hm / lh
+                          : (k == 0 ? 0 : k == 1 ? 1 : (hi ? 2 : 0));         // hh / mm / hl
+      return 16 * (piece * CB + (g & 1));
+    } else if constexpr (DH == 64) {
+      return 16 * ((k / 2) * CB + 4 * (k % 2) + g);
+    } else {
+      return 16 * (k * CB + g);
+    }
+  }
+};
+
+template <int DH, int G>
+struct PieceOps {
+  static constexpr int SB = DH <= 16 ? 64 : 32;
+  static constexpr int MT = out_tiles(DH);
+  using P = Pairs<DH>;
+  struct Rows {
+    bf16x8 x[G][P::NB];
+  };
+  static __device__ __forceinline__ void load_rows(Rows& r, int u, const Mat& m, int64_t row, int h,
+                                                   int H, int g) {
+    const int n_pad = padded(m.n);
+    const char* p = m.row_img + (int64_t(h) * n_pad + row) * row_bytes(DH);
+#pragma unroll
+    for (int k = 0; k < P::NB; ++k) {
+      uint4 w = make_uint4(0u, 0u, 0u, 0u);
+      if (row < n_pad) w = *reinterpret_cast<const uint4*>(p + P::unit(true, k, g));
+      r.x[u][k] = __builtin_bit_cast(bf16x8, w);
+    }
+  }
+  template <bool ROW, bool COL>
+  struct Staged {
+    static constexpr int RB = ROW ? SB * row_bytes(DH) : 0;
+    static constexpr int TB = COL ? SB / kStep * t_bytes(DH) : 0;
+    static constexpr int BYTES = RB + TB;
+    static constexpr int NR = (RB / 16 + kBlock - 1) / kBlock, NT = (TB / 16 + kBlock - 1) / kBlock;
+    static constexpr int NV = NR + NT;
+    char* lds;
+    uint4 w[NV];
+    __device__ __forceinline__ void load(const Mat& m, int row0, int h, int H) {
+      const int n_pad = padded(m.n);
+      const char* r = m.row_img + (int64_t(h) * n_pad + row0) * row_bytes(DH);
+      const char* t = m.t_img + (int64_t(h) * (n_pad / kStep) + row0 / kStep) * t_bytes(DH);
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const int e = 16 * (tid_x() + i * kBlock);
+        w[i] = *reinterpret_cast<const uint4*>(r + min(e, RB - 16));
+      }
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int e = 16 * (tid_x() + i * kBlock);
+        w[NR + i] = *reinterpret_cast<const uint4*>(t + min(e, TB - 16));
+      }
+    }
+    __device__ __forceinline__ void store() const {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const int e = 16 * (tid_x() + i * kBlock);
+        if (e < RB) *reinterpret_cast<uint4*>(lds + e) = w[i];
+      }
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int e = 16 * (tid_x() + i * kBlock);
+        if (e < TB) *reinterpret_cast<uint4*>(lds + RB + e) = w[NR + i];
+      }
+    }
+    __device__ __forceinline__ void products(int r0, int g, int l16, const Rows& rows,
+                                             f32x4 (&x)[2][G]) const {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const char* p = lds + (r0 + kT * t + l16) * row_bytes(DH);
+        bf16x8 a[P::NA];
+#pragma unroll
+        for (int k = 0; k < P::NA; ++k)
+          a[k] = *reinterpret_cast<const bf16x8*>(p + P::unit(false, k, g));
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          x[t][u] = zero4();
+#pragma unroll
+          for (int n = 0; n < P::N; ++n)
+            x[t][u] = mfma32(a[P::a_of(n)], rows.x[u][P::b_of(n)], x[t][u]);
+        }
+      }
+    }
+    __device__ __forceinline__ void accumulate(int r0, int g, int l16, const f32x4 (&x)[2][G],
+                                               f32x4 (&acc)[G][MT]) const {
+      const char* p = lds + RB + (r0 / kStep) * t_bytes(DH) + l16 * kTLine + 16 * g;
+      auto line = [&](int tile) {
+        return *reinterpret_cast<const bf16x8*>(p + tile * kT * kTLine);
+      };
+      Split sp[G];
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = x[j / 4][u][j % 4];
+        sp[u] = split8<false>(v);
+      }
+      if constexpr (DH == 8) {  // rows 0-7: h (then l), rows 8-15: m of M
+        const bf16x8 hm = line(0), l = line(1);
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          acc[u][0] = mfma32(l, sp[u].h, acc[u][0]);
+          acc[u][0] = mfma32(hm, sp[u].l, acc[u][0]);
+          acc[u][0] = mfma32(hm, sp[u].m, acc[u][0]);
+          acc[u][0] = mfma32(hm, sp[u].h, acc[u][0]);
+        }
+      } else {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const bf16x8 ah = line(m), am = line(MT + m), al = line(2 * MT + m);
+#pragma unroll
+          for (int u = 0; u < G; ++u) {
+            acc[u][m] = mfma32(al, sp[u].h, acc[u][m]);
+            acc[u][m] = mfma32(ah, sp[u].l, acc[u][m]);
+            acc[u][m] = mfma32(am, sp[u].m, acc[u][m]);
+            acc[u][m] = mfma32(am, sp[u].h, acc[u][m]);
+            acc[u][m] = mfma32(ah, sp[u].m, acc[u][m]);
+            acc[u][m] = mfma32(ah, sp[u].h, acc[u][m]);
+          }
+        }
+      }
+    }
+  };
+  // d = 8: a column's two piece rows meet (lanes g and g + 2)
+  static __device__ __forceinline__ void finish(f32x4 (&acc)[G][MT]) {
+    if constexpr (DH == 8) {
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[u][0][i] = sum_halves(acc[u][0][i]);
+    }
+  }
+};
+
+// A stage's sums (at most 64 rows) start from zero and are added to the total
+// at its end: one accumulator over 16,000 rows had moved the outputs by 6e-6,
+// three times the error of the two levels' sum.
+template <int G, int MT>
+__device__ __forceinline__ void zero_acc(f32x4 (&x)[G][MT]) {
+#pragma unroll
+  for (int u = 0; u < G; ++u)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) x[u][t] = zero4();
+}
+template <int G, int MT>
+__device__ __forceinline__ void add_acc(const f32x4 (&x)[G][MT], f32x4 (&acc)[G][MT]) {
+#pragma unroll
+  for (int u = 0; u < G; ++u)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[u][t] += x[u][t];
+}
+template <int DH, int G>
+__device__ __forceinline__ void store_acc(float* __restrict__ row, int u, int g, float f,
+                                          const f32x4 (&acc)[G][out_tiles(DH)]) {
+#pragma unroll
+  for (int m = 0; m < out_tiles(DH); ++m)
+    if (kT * m + 4 * g < DH)
+      *reinterpret_cast<float4*>(row + kT * m + 4 * g) = make_float4(
+          acc[u][m][0] * f, acc[u][m][1] * f, acc[u][m][2] * f, acc[u][m][3] * f);
+}
+
+// LDS of a kernel whose two bodies share one buffer.
+constexpr int max_of(int a, int b) { return a > b ? a : b; }
+
+// ------------------------------------------------------------------ forward
+struct FwdArgs {
+  Mat q, k, v;
+  int32_t H;
+  DropoutMask dm;
+  uint32_t thr16;
+  float *out, *out32, *lse;
+  int32_t split_keys;
+  float *part_ml, *part_acc;
+  int32_t n_split, fwd_bx, score_bx;
+  float* part;
+};
+
+// One block: block_rows(G) queries of head h, keys of split z.  S^T = K Q^T
+// (rows = keys), online softmax per lane's query, O^T += V^T P^T.  The base m
+// moves only when some score exceeds it by more than kRebase, so after the
+// first step a wave rarely rescales; the column maximum over the lanes that
+// share a query is taken only then.
+template <class Ops, int DH, int G, bool DROP>
+__device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z, char* lds) {
+  constexpr int SB = Ops::SB, MT = out_tiles(DH);
+  const int lane = tid_x() & (kWave - 1);
+  const int wave = tid_x() >> 6;
+  const int g = lane >> 4, l16 = lane & 15;
+  const int n_q = a.q.n, H = a.H;
+  DropoutMask dm = a.dm;
+  if constexpr (DROP) dm = drop_for_head(dm, h);
+  int qi[G];
+  typename Ops::Rows qf;
+  float m[G], l[G], thr[G];
+  f32x4 acc[G][MT];
+  zero_acc(acc);
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    qi[u] = bx * block_rows(G) + (wave * G + u) * kT + l16;
+    Ops::load_rows(qf, u, a.q, qi[u], h, H, g);
+    m[u] = thr[u] = -INFINITY;
+    l[u] = 0.f;
+  }
+  const int k_begin = z * a.split_keys;
+  const int k_end = min(a.k.n, k_begin + a.split_keys);
+  typename Ops::template Staged<true, false> sk;
+  typename Ops::template Staged<false, true> sv;
+  sk.lds = reinterpret_cast<decltype(sk.lds)>(lds);
+  sv.lds = reinterpret_cast<decltype(sv.lds)>(lds + sk.BYTES);
+  if (k_begin < k_end) {
+    sk.load(a.k, k_begin, h, H);
+    sv.load(a.v, k_begin, h, H);
+  }
+  for (int kb = k_begin; kb < k_end; kb += SB) {
+    __syncthreads();
+    sk.store();
+    sv.store();
+    __syncthreads();
+    if (kb + SB < k_end) {
+      sk.load(a.k, kb + SB, h, H);
+      sv.load(a.v, kb + SB, h, H);
+    }
+    f32x4 stage[G][MT];  // this stage's share of acc and l
+    float lst[G];
+    zero_acc(stage);
+#pragma unroll
+    for (int u = 0; u < G; ++u) lst[u] = 0.f;
+    for (int r0 = 0; r0 < SB && kb + r0 < k_end; r0 += kStep) {
+      f32x4 s[2][G];  // S^T tiles: rows = keys kb + r0 + 16 t + 4 g + i
+      sk.products(r0, g, l16, qf, s);
+      if (kb + r0 + kStep > k_end) {  // keys past the end drop out
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb + r0 + kT * t + 4 * g + i >= k_end)
+#pragma unroll
+              for (int u = 0; u < G; ++u) s[t][u][i] = -INFINITY;
+      }
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[t][u][i]);
+        if (__any(mx > thr[u])) {
+          const float m_new = fmaxf(m[u], max_rows(mx));
+          const float alpha = m[u] == -INFINITY ? 0.f : exp_nat(m[u] - m_new);
+          l[u] *= alpha;
+          lst[u] *= alpha;
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            acc[u][t] *= alpha;
+            stage[u][t] *= alpha;
+          }
+          m[u] = m_new;
+          thr[u] = m_new + kRebase;
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const uint32_t key = uint32_t(kb + r0 + kT * t + 4 * g);
+          uint32_t w[2] = {0u, 0u};  // keys +0, +1 and +2, +3
+          if constexpr (DROP) {
+            w[0] = drop_word(dm, uint32_t(qi[u]), key);
+            w[1] = drop_word(dm, uint32_t(qi[u]), key + 2);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float p = exp_nat(s[t][u][i] - m[u]);
+            lst[u] += p;  // the softmax normaliser uses every key
+            if constexpr (DROP) {
+              const uint32_t bits = i & 1 ? w[i / 2] : w[i / 2] << 16;
+              s[t][u][i] = kept(bits, a.thr16) ? p : 0.f;
+            } else {
+              s[t][u][i] = p;
+            }
+          }
+        }
+      }
+      sv.accumulate(r0, g, l16, s, stage);
+    }
+    add_acc(stage, acc);
+#pragma unroll
+    for (int u = 0; u < G; ++u) l[u] += lst[u];
+  }
+  Ops::finish(acc);
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    const float lsum = sum_rows(l[u]);
+    if (qi[u] >= n_q) continue;
+    const int64_t row = int64_t(qi[u]) * H + h;
+    if (a.part_ml) {  // this split's softmax state, merged in split order later
+      store_acc<DH, G>(a.part_acc + (int64_t(z) * n_q * H + row) * DH, u, g, 1.f, acc);
+      if (g == 0) {
+        const int64_t r = (int64_t(z) * H + h) * n_q + qi[u];
+        a.part_ml[2 * r] = m[u];
+        a.part_ml[2 * r + 1] = lsum;
+      }
+      continue;
+    }
+    const float inv = a.k.n > 0 ? 1.0f / lsum : 0.f;
+    store_acc<DH, G>(a.out + row * DH, u, g, inv, acc);
+    if (a.out32) store_acc<DH, G>(a.out32 + row * DH, u, g, inv, acc);
+    if (g == 0)
+      a.lse[int64_t(h) * n_q + qi[u]] =
+          a.k.n > 0 ? m[u] + __builtin_amdgcn_logf(lsum) * kLn2 : -INFINITY;
+  }
+}
+
+// Column scores part[h][j] = sum_i |S[h, i, j]|: rows = queries (staged),
+// lanes = keys.  Each stage's sum is added to the total, so a long column is
+// summed in two levels.
+template <class Ops, int DH, int G>
+__device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, char* lds) {
+  constexpr int SB = Ops::SB;
+  const int lane = tid_x() & (kWave - 1);
+  const int wave = tid_x() >> 6;
+  const int g = lane >> 4, l16 = lane & 15;
+  const int n_q = a.q.n;
+  int kj[G];
+  typename Ops::Rows kf;
+  float sum[G];
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    kj[u] = bx * block_rows(G) + (wave * G + u) * kT + l16;
+    sum[u] = 0.f;
+    Ops::load_rows(kf, u, a.k, kj[u], h, a.H, g);
+  }
+  typename Ops::template Staged<true, false> sq;
+  sq.lds = reinterpret_cast<decltype(sq.lds)>(lds);
+  sq.load(a.q, 0, h, a.H);
+  for (int qb = 0; qb < n_q; qb += SB) {
+    __syncthreads();
+    sq.store();
+    __syncthreads();
+    if (qb + SB < n_q) sq.load(a.q, qb + SB, h, a.H);
+    float st[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) st[u] = 0.f;
+    for (int r0 = 0; r0 < SB && qb + r0 < n_q; r0 += kStep) {  // rows past n_q are zero
+      f32x4 s[2][G];
+      sq.products(r0, g, l16, kf, s);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[u] += fabsf(s[t][u][i]);
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u) sum[u] += st[u];
+  }
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    const float t = sum_rows(sum[u]);
+    if (g == 0 && kj[u] < a.k.n) a.part[int64_t(h) * a.k.n + kj[u]] = t;
+  }
+}
+
+template <class Ops>
+constexpr int fwd_lds() {
+  return Ops::template Staged<true, false>::BYTES + Ops::template Staged<false, true>::BYTES;
+}
+
+// The forward and the column scores in one launch: grid z < n_split are
+// forward blocks, the last slice holds the score blocks, which fill the CUs
+// that the forward's last round leaves idle.
+template <int DH, int G, bool DROP>
+__global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
+  using F = Fp32Ops<DH, G>;
+  using P = PieceOps<DH, G>;
+  __shared__ __align__(16) char lds[max_of(fwd_lds<F>(), fwd_lds<P>())];
+  const int bx = wg_x(), h = wg_y(), z = wg_z();
+  if (bx >= (z == a.n_split ? a.score_bx : a.fwd_bx)) return;  // block-uniform, before any barrier
+  const bool plain = any_flag(a.q, a.k, a.v, h);
+  if (z == a.n_split) {
+    if (plain)
+      scores_body<F, DH, G>(a, bx, h, lds);
+    else
+      scores_body<P, DH, G>(a, bx, h, lds);
+  } else if (plain) {
+    fwd_body<F, DH, G, DROP>(a, bx, h, z, lds);
+  } else {
+    fwd_body<P, DH, G, DROP>(a, bx, h, z, lds);
+  }
+}
+
+// ----------------------------------------------------------------- backward
+struct BwdArgs {
+  Mat q, k, v, g;
+  int32_t H;
+  DropoutMask dm;
+  uint32_t thr16;
+  const float *out, *lse;
+  float* dsum;
+  float scale;
+  float *grad_q, *grad_k, *grad_v;
+  int32_t split_keys;
+  float* part_dq;
+  int32_t n_split, kv_bx, comb_bx;
+};
+
+// Query-major: dQ^T += K^T dS^T over the keys of split z, S and dP recomputed
+// as in the forward.  D = dO . out per query is formed here and stored (split
+// 0) for the dK/dV pass.
+template <class Ops, int DH, int G, bool DROP>
+__device__ __forceinline__ void bwd_q_body(const BwdArgs& a, int bx, int h, int z, char* lds) {
+  constexpr int SB = Ops::SB, MT = out_tiles(DH);
+  const int lane = tid_x() & (kWave - 1);
+  const int wave = tid_x() >> 6;
+  const int g = lane >> 4, l16 = lane & 15;
+  const int n_q = a.q.n, H = a.H;
+  DropoutMask dm = a.dm;
+  if constexpr (DROP) dm = drop_for_head(dm, h);
+  int qi[G];
+  typename Ops::Rows qf, gf;
+  float L[G], D[G];
+  f32x4 acc[G][MT];
+  zero_acc(acc);
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    qi[u] = bx * block_rows(G) + (wave * G + u) * kT + l16;
+    const bool ok = qi[u] < n_q;
+    Ops::load_rows(qf, u, a.q, qi[u], h, H, g);
+    Ops::load_rows(gf, u, a.g, qi[u], h, H, g);
+    float d = 0.f;
+    if (ok) {
+      const int64_t o = (int64_t(qi[u]) * H + h) * DH + (DH / 4) * g;
+      float gq[DH / 4], oq[DH / 4];
+      load_quarter<DH>(a.g.x + o, gq);
+      load_quarter<DH>(a.out + o, oq);
+#pragma unroll
+      for (int j = 0; j < DH / 4; ++j) d = fmaf(gq[j], oq[j], d);
+    }
+    D[u] = sum_rows(d);
+    L[u] = ok ? a.lse[int64_t(h) * n_q + qi[u]] : INFINITY;
+    if (ok && z == 0 && g == 0) a.dsum[int64_t(h) * n_q + qi[u]] = D[u];
+  }
+  const int k_begin = z * a.split_keys;
+  const int k_end = min(a.k.n, k_begin + a.split_keys);
+  typename Ops::template Staged<true, true> sk;
+  typename Ops::template Staged<true, false> sv;
+  sk.lds = reinterpret_cast<decltype(sk.lds)>(lds);
+  sv.lds = reinterpret_cast<decltype(sv.lds)>(lds + sk.BYTES);
+  if (k_begin < k_end) {
+    sk.load(a.k, k_begin, h, H);
+    sv.load(a.v, k_begin, h, H);
+  }
+  for (int kb = k_begin; kb < k_end; kb += SB) {
+    __syncthreads();
+    sk.store();
+    sv.store();
+    __syncthreads();
+    if (kb + SB < k_end) {
+      sk.load(a.k, kb + SB, h, H);
+      sv.load(a.v, kb + SB, h, H);
+    }
+    f32x4 stage[G][MT];
+    zero_acc(stage);
+    for (int r0 = 0; r0 < SB && kb + r0 < k_end; r0 += kStep) {
+      f32x4 s[2][G], dp[2][G];
+      sk.products(r0, g, l16, qf, s);
+      sv.products(r0, g, l16, gf, dp);
+      if (kb + r0 + kStep > k_end) {  // keys past the end: p = 0
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb + r0 + kT * t + 4 * g + i >= k_end)
+#pragma unroll
+              for (int u = 0; u < G; ++u) s[t][u][i] = -INFINITY;
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          const uint32_t key = uint32_t(kb + r0 + kT * t + 4 * g);
+          uint32_t w[2] = {0u, 0u};
+          if constexpr (DROP) {
+            w[0] = drop_word(dm, uint32_t(qi[u]), key);
+            w[1] = drop_word(dm, uint32_t(qi[u]), key + 2);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float p = exp_nat(s[t][u][i] - L[u]);
+            float x = dp[t][u][i];
+            if constexpr (DROP) {
+              const uint32_t bits = i & 1 ? w[i / 2] : w[i / 2] << 16;
+              x = kept(bits, a.thr16) ? x : 0.f;
+            }
+            s[t][u][i] = p * (x - D[u]);
+          }
+        }
+      sk.accumulate(r0, g, l16, s, stage);
+    }
+    add_acc(stage, acc);
+  }
+  Ops::finish(acc);
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    if (qi[u] >= n_q) continue;
+    const int64_t row = int64_t(qi[u]) * H + h;
+    if (a.part_dq)
+      store_acc<DH, G>(a.part_dq + (int64_t(z) * n_q * H + row) * DH, u, g, 1.f, acc);
+    else
+      store_acc<DH, G>(a.grad_q + row * DH, u, g, a.scale, acc);
+  }
+}
+
+template <class Ops>
+constexpr int bwd_q_lds() {
+  return Ops::template Staged<true, true>::BYTES + Ops::template Staged<true, false>::BYTES;
+}
+
+template <int DH, int G, bool DROP>
+__global__ __launch_bounds__(kBlock) void k_fx_bwd_q(const BwdArgs a) {
+  using F = Fp32Ops<DH, G>;
+  using P = PieceOps<DH, G>;
+  __shared__ __align__(16) char lds[max_of(bwd_q_lds<F>(), bwd_q_lds<P>())];
+  const int bx = wg_x(), h = wg_y(), z = wg_z();
+  if (any_flag(a.q, a.k, a.v, h) || any_flag(a.g, a.g, a.g, h))
+    bwd_q_body<F, DH, G, DROP>(a, bx, h, z, lds);
+  else
+    bwd_q_body<P, DH, G, DROP>(a, bx, h, z, lds);
+}
+
+// grad_q = scale * sum of the key splits' partial dQ, added in split order.
+__device__ __forceinline__ void dq_combine(const BwdArgs& a, int64_t n, int64_t b, int64_t nb) {
+  for (int64_t t = b * kBlock + tid_x(); t < n; t += nb * kBlock) {
+    float x = a.part_dq[t];
+    for (int s = 1; s < a.n_split; ++s) x += a.part_dq[int64_t(s) * n + t];
+    a.grad_q[t] = x * a.scale;
+  }
+}
+
+// Key-major: dV^T += dO^T P and dK^T += (Q scale)^T dS, rows = queries
+// (staged, Q already scaled), lanes = keys.
+template <class Ops, int DH, int G, bool DROP>
+__device__ __forceinline__ void bwd_kv_body(const BwdArgs& a, int bx, int h, char* lds, float* ls,
+                                            float* ds) {
+  constexpr int SB = Ops::SB, MT = out_tiles(DH);
+  const int lane = tid_x() & (kWave - 1);
+  const int wave = tid_x() >> 6;
+  const int g = lane >> 4, l16 = lane & 15;
+  const int n_q = a.q.n, H = a.H;
+  DropoutMask dm = a.dm;
+  if constexpr (DROP) dm = drop_for_head(dm, h);
+  int kj[G];
+  typename Ops::Rows kf, vf;
+  f32x4 dk[G][MT], dv[G][MT];
+  zero_acc(dk);
+  zero_acc(dv);
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    kj[u] = bx * block_rows(G) + (wave * G + u) * kT + l16;
+    Ops::load_rows(kf, u, a.k, kj[u], h, H, g);
+    Ops::load_rows(vf, u, a.v, kj[u], h, H, g);
+  }
+  typename Ops::template Staged<true, true> sq, sg;
+  sq.lds = reinterpret_cast<decltype(sq.lds)>(lds);
+  sg.lds = reinterpret_cast<decltype(sg.lds)>(lds + sq.BYTES);
+  float pl = 0.f, pd = 0.f;
+  auto prefetch = [&](int qb) {
+    sq.load(a.q, qb, h, H);
+    sg.load(a.g, qb, h, H);
+    if (tid_x() < SB) {
+      const bool ok = qb + tid_x() < n_q;  // padded rows: p = exp(-inf) = 0, dO = D = 0
+      pl = ok ? a.lse[int64_t(h) * n_q + qb + tid_x()] : INFINITY;
+      pd = ok ? a.dsum[int64_t(h) * n_q + qb + tid_x()] : 0.f;
+    }
+  };
+  const int shift = lane & 1 ? 0 : 16;  // this lane's key's half of a word (kj is odd where l16 is)
+  if (n_q > 0) prefetch(0);
+  for (int qb = 0; qb < n_q; qb += SB) {
+    __syncthreads();
+    sq.store();
+    sg.store();
+    if (tid_x() < SB) {
+      ls[tid_x()] = pl;
+      ds[tid_x()] = pd;
+    }
+    __syncthreads();
+    if (qb + SB < n_q) prefetch(qb + SB);
+    f32x4 sdk[G][MT], sdv[G][MT];
+    zero_acc(sdk);
+    zero_acc(sdv);
+    for (int r0 = 0; r0 < SB && qb + r0 < n_q; r0 += kStep) {
+      f32x4 s[2][G], dp[2][G];
+      sq.products(r0, g, l16, kf, s);
+      sg.products(r0, g, l16, vf, dp);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int r = r0 + kT * t + 4 * g;  // queries qb + r .. + 3
+        const f32x4 L = *reinterpret_cast<const f32x4*>(ls + r);
+        const f32x4 D = *reinterpret_cast<const f32x4*>(ds + r);
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          // the lanes of a key pair need the same four words (one per query):
+          // the even lane hashes the first two, the odd one the others
+          uint32_t w[4] = {0u, 0u, 0u, 0u};
+          if constexpr (DROP) {
+            const bool odd = (lane & 1) != 0;
+            const uint32_t qr = uint32_t(qb + r) + (odd ? 2u : 0u);
+            const uint32_t wa = drop_word(dm, qr, uint32_t(kj[u]));
+            const uint32_t wb = drop_word(dm, qr + 1, uint32_t(kj[u]));
+            const uint32_t wc = swap_pair(wa), wd = swap_pair(wb);
+            w[0] = odd ? wc : wa, w[1] = odd ? wd : wb, w[2] = odd ? wa : wc, w[3] = odd ? wb : wd;
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float p = exp_nat(s[t][u][i] - L[i]);
+            if constexpr (DROP) {
+              const bool keep = kept(w[i] << shift, a.thr16);
+              dp[t][u][i] = p * ((keep ? dp[t][u][i] : 0.f) - D[i]);
+              s[t][u][i] = keep ? p : 0.f;
+            } else {
+              dp[t][u][i] = p * (dp[t][u][i] - D[i]);
+              s[t][u][i] = p;
+            }
+          }
+        }
+      }
+      sg.accumulate(r0, g, l16, s, sdv);
+      sq.accumulate(r0, g, l16, dp, sdk);
+    }
+    add_acc(sdk, dk);
+    add_acc(sdv, dv);
+  }
+  Ops::finish(dk);
+  Ops::finish(dv);
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    if (kj[u] >= a.k.n) continue;
+    const int64_t o = (int64_t(kj[u]) * H + h) * DH;
+    store_acc<DH, G>(a.grad_k + o, u, g, 1.f, dk);
+    store_acc<DH, G>(a.grad_v + o, u, g, 1.f, dv);
+  }
+}
+
+template <class Ops>
+constexpr int bwd_kv_lds() {
+  return 2 * Ops::template Staged<true, true>::BYTES;
+}
+
+// Blocks at grid x >= kv_bx add the dQ splits' partials instead of taking
+// keys (that merge needs no launch of its own).
+template <int DH, int G, bool DROP>
+__global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
+  using F = Fp32Ops<DH, G>;
+  using P = PieceOps<DH, G>;
+  __shared__ __align__(16) char lds[max_of(bwd_kv_lds<F>(), bwd_kv_lds<P>())];
+  __shared__ __align__(16) float ls[64];
+  __shared__ __align__(16) float ds[64];
+  const int bx = wg_x(), h = wg_y();
+  if (bx >= a.kv_bx) {  // block-uniform
+    dq_combine(a, int64_t(a.q.n) * a.H * DH, int64_t(bx - a.kv_bx) * a.H + h,
+               int64_t(a.comb_bx) * a.H);
+    return;
+  }
+  if (any_flag(a.q, a.k, a.v, h) || any_flag(a.g, a.g, a.g, h))
+    bwd_kv_body<F, DH, G, DROP>(a, bx, h, lds, ls, ds);
+  else
+    bwd_kv_body<P, DH, G, DROP>(a, bx, h, lds, ls, ds);
+}
+
+// ------------------------------------------------------------------ host side
+inline int blocks_of(int n, int rows) { return (n + rows - 1) / rows; }
+inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
+
+// 16-row tiles per wave: 2 (each staged operand feeds two MFMAs) where the
+// grid still gives the 1,024 SIMDs two waves each, else 1; 1 at d = 64, whose
+// accumulators and operands of two tiles would leave one wave per SIMD.
+// NGT_DENSE_F32_TILES overrides the choice below d = 64.
+int tiles_per_wave(int n, int H, int d) {
+  if (d == 64) return 1;
+  if (const char* e = getenv("NGT_DENSE_F32_TILES")) return atoi(e) == 1 ? 1 : 2;
+  return int64_t(blocks_of(n, block_rows(2))) * H * kWaves >= 2048 ? 2 : 1;
+}
+
+MfSplit split_keys_for(int n_q, int n_k, int H, int d, int target_waves, int64_t shared_waves,
+                       const char* env) {
+  const int rows = block_rows(tiles_per_wave(n_q, H, d));
+  const int64_t base = int64_t(blocks_of(n_q, rows)) * H * kWaves;
+  const int64_t room = std::max<int64_t>(target_waves - shared_waves, 0);
+  int want = base > 0 ? int((room + base / 2) / base) : 1;
+  if (const char* e = getenv(env)) want = atoi(e);
+  want = std::max(1, std::min({want, 8, std::max(1, n_k / 256)}));
+  if (want <= 1 || n_k <= 0) return {1, std::max(n_k, 1)};
+  int keys = (n_k + want - 1) / want;
+  keys = (keys + kPadRows - 1) / kPadRows * kPadRows;
+  return {(n_k + keys - 1) / keys, keys};
+}
+
+constexpr int rt_row_bytes(int d) {
+  return d == 8 ? row_bytes(8) : d == 16 ? row_bytes(16) : d == 24 ? row_bytes(24)
+       : d == 32 ? row_bytes(32) : row_bytes(64);
+}
+constexpr int rt_t_bytes(int d) {
+  return d == 8 ? t_bytes(8) : d == 16 ? t_bytes(16) : d == 24 ? t_bytes(24)
+       : d == 32 ? t_bytes(32) : t_bytes(64);
+}
+size_t row_image_bytes(int n, int H, int d) {
+  return align256(size_t(padded(n)) * H * rt_row_bytes(d));
+}
+size_t t_image_bytes(int n, int H, int d) {
+  return align256(size_t(padded(n) / kStep) * H * rt_t_bytes(d));
+}
+size_t flag_bytes(int n, int H) { return align256(size_t(padded(n) / kStep) * H * 4); }
+
+// Assigns one matrix's images in the workspace and adds its preparation job.
+struct Images {
+  char* ws;
+  int H, d;
+  PrepJobs jobs{};
+  int n_jobs = 0, max_rows = 0;
+  Mat add(const float* x, int n, float scale, bool want_t) {
+    PrepJob& j = jobs.j[n_jobs++];
+    j.x = x;
+    j.row_img = ws;
+    ws += row_image_bytes(n, H, d);
+    j.t_img = nullptr;
+    if (want_t) {
+      j.t_img = ws;
+      ws += t_image_bytes(n, H, d);
+    }
+    j.flag = reinterpret_cast<uint32_t*>(ws);
+    ws += flag_bytes(n, H);
+    j.n = n;
+    j.scale = scale;
+    max_rows = std::max(max_rows, padded(n));
+    return Mat{x, j.row_img, j.t_img, j.flag, n, scale};
+  }
+};
+
+template <int DH>
+int run_prep(const Images& im, hipStream_t st) {
+  if (im.max_rows == 0) return NGT_OK;
+  KernelTimer timer_("dense_prep", st);
+  hipLaunchKernelGGL((k_fx_prep<DH>), dim3(im.max_rows / kStep, im.H, im.n_jobs), dim3(kBlock), 0,
+                     st, im.jobs, im.H);
+  NGT_HIP_CHECK(hipGetLastError());
+  return NGT_OK;
+}
+
+template <int DH, int G>
+int fx_fwd(FwdArgs a, const DropoutMask* dm, hipStream_t st) {
+  a.fwd_bx = blocks_of(a.q.n, block_rows(G));
+  a.score_bx = a.part && a.k.n > 0 ? blocks_of(a.k.n, block_rows(G)) : 0;
+  const dim3 grid(std::max(a.fwd_bx, a.score_bx), a.H, a.n_split + (a.score_bx > 0 ? 1 : 0));
+  KernelTimer timer_("dense_fwd", st);
+  if (dm)
+    hipLaunchKernelGGL((k_fx_fwd<DH, G, true>), grid, dim3(kBlock), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_fx_fwd<DH, G, false>), grid, dim3(kBlock), 0, st, a);
+  NGT_HIP_CHECK(hipGetLastError());
+  return NGT_OK;
+}
+
+template <int DH, int G>
+int fx_bwd_q(const BwdArgs& a, const DropoutMask* dm, hipStream_t st) {
+  KernelTimer timer_("dense_bwd_q", st);
+  const dim3 grid(blocks_of(a.q.n, block_rows(G)), a.H, a.n_split);
+  if (dm)
+    hipLaunchKernelGGL((k_fx_bwd_q<DH, G, true>), grid, dim3(kBlock), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_fx_bwd_q<DH, G, false>), grid, dim3(kBlock), 0, st, a);
+  NGT_HIP_CHECK(hipGetLastError());
+  return NGT_OK;
+}
+
+template <int DH, int G>
+int fx_bwd_kv(BwdArgs a, const DropoutMask* dm, hipStream_t st) {
+  KernelTimer timer_("dense_bwd_kv", st);
+  a.kv_bx = blocks_of(a.k.n, block_rows(G));
+  // merge blocks per head: about 4 elements per thread
+  const int64_t n_dq = int64_t(a.q.n) * a.H * DH;
+  const int64_t per = int64_t(4) * kBlock * a.H;
+  a.comb_bx = a.part_dq ? int((n_dq + per - 1) / per) : 0;
+  const dim3 grid(a.kv_bx + a.comb_bx, a.H);
+  if (dm)
+    hipLaunchKernelGGL((k_fx_bwd_kv<DH, G, true>), grid, dim3(kBlock), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_fx_bwd_kv<DH, G, false>), grid, dim3(kBlock), 0, st, a);
+  NGT_HIP_CHECK(hipGetLastError());
+  return NGT_OK;
+}
+
+template <int DH>
+int fx_forward(FwdArgs a, const Images& im, const DropoutMask* dm, hipStream_t st) {
+  NGT_CHECK_OK(run_prep<DH>(im, st));
+  if constexpr (DH == 64) return fx_fwd<DH, 1>(a, dm, st);
+  else
+    return tiles_per_wave(a.q.n, a.H, DH) == 2 ? fx_fwd<DH, 2>(a, dm, st) : fx_fwd<DH, 1>(a, dm, st);
+}
+
+template <int DH>
+int fx_backward(const BwdArgs& a, const Images& im, const DropoutMask* dm, hipStream_t st) {
+  NGT_CHECK_OK(run_prep<DH>(im, st));
+  if constexpr (DH == 64) {
+    if (a.q.n > 0) NGT_CHECK_OK((fx_bwd_q<DH, 1>(a, dm, st)));
+    return a.k.n > 0 ? fx_bwd_kv<DH, 1>(a, dm, st) : NGT_OK;
+  } else {
+    if (a.q.n > 0)
+      NGT_CHECK_OK((tiles_per_wave(a.q.n, a.H, DH) == 2 ? fx_bwd_q<DH, 2>(a, dm, st)
+                                                        : fx_bwd_q<DH, 1>(a, dm, st)));
+    if (a.k.n > 0)
+      return tiles_per_wave(a.k.n, a.H, DH) == 2 ? fx_bwd_kv<DH, 2>(a, dm, st)
+                                                 : fx_bwd_kv<DH, 1>(a, dm, st);
+    return NGT_OK;
+  }
+}
+
+}  // namespace
+
+MfSplit f32_fwd_split(int n_q, int n_k, int H, int d, bool node_scores) {
+  const int rows = block_rows(tiles_per_wave(n_k, H, d));
+  const int64_t score_waves = node_scores ? int64_t(blocks_of(n_k, rows)) * H * kWaves : 0;
+  return split_keys_for(n_q, n_k, H, d, 6144, score_waves, "NGT_DENSE_F32_FWD_SPLIT");
+}
+MfSplit f32_dq_split(int n_q, int n_k, int H, int d) {
+  return split_keys_for(n_q, n_k, H, d, 6144, 0, "NGT_DENSE_F32_DQ_SPLIT");
+}
+
+// Bytes of the images and flags that the two directions keep in the workspace.
+size_t f32_fwd_image_bytes(int n_q, int n_k, int H, int d) {
+  return row_image_bytes(n_q, H, d) + flag_bytes(n_q, H) + 2 * row_image_bytes(n_k, H, d) +
+         t_image_bytes(n_k, H, d) + 2 * flag_bytes(n_k, H);
+}
+size_t f32_bwd_image_bytes(int n_q, int n_k, int H, int d) {
+  return 2 * (row_image_bytes(n_q, H, d) + t_image_bytes(n_q, H, d) + flag_bytes(n_q, H)) +
+         2 * (row_image_bytes(n_k, H, d) + flag_bytes(n_k, H)) + t_image_bytes(n_k, H, d);
+}
+
+// (threshold << 16, scale) of a mask for kept(); a threshold of 2^16 (nothing
+// kept) becomes "all kept" with scale 0, as p = 1 is.
+static void drop_terms(const DropoutMask* dm, uint32_t* thr16, float* scale) {
+  const bool none = dm && dm->thr > 0xffffu;
+  *thr16 = dm && !none ? dm->thr << 16 : 0u;
+  *scale = !dm ? 1.f : none ? 0.f : dm->scale;
+}
+
+int f32_dense_fwd(int d, const float* q, const float* k, const float* v, int n_q, int n_k, int H,
+                  float scale, const DropoutMask* dm, float* out, float* out32, float* lse,
+                  float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
+                  hipStream_t st) {
+  Images im{images, H, d};
+  FwdArgs a{};
+  a.q = im.add(q, n_q, scale, false);
+  a.k = im.add(k, n_k, 1.f, false);
+  float vs;
+  drop_terms(dm, &a.thr16, &vs);
+  a.v = im.add(v, n_k, vs, true);
+  a.H = H;
+  if (dm) a.dm = *dm;
+  a.out = out, a.out32 = out32, a.lse = lse;
+  a.split_keys = sp.split_keys;
+  a.n_split = sp.n_split;
+  if (sp.n_split > 1) a.part_ml = part_ml, a.part_acc = part_acc;
+  a.part = part;
+  switch (d) {
+    case 8: return fx_forward<8>(a, im, dm, st);
+    case 16: return fx_forward<16>(a, im, dm, st);
+    case 24: return fx_forward<24>(a, im, dm, st);
+    case 32: return fx_forward<32>(a, im, dm, st);
+    case 64: return fx_forward<64>(a, im, dm, st);
+    default: return set_error(NGT_ERR_UNSUPPORTED, "fp32 dense: head_dim %d", d);
+  }
+}
+
+int f32_dense_bwd(int d, const float* q, const float* k, const float* v, const float* go,
+                  const float* out, const float* lse, float* dsum, int n_q, int n_k, int H,
+                  float scale, const DropoutMask* dm, float* gq, float* gk, float* gv, MfSplit sq,
+                  float* part_dq, char* images, hipStream_t st) {
+  Images im{images, H, d};
+  BwdArgs a{};
+  a.q = im.add(q, n_q, scale, true);
+  float gs;
+  drop_terms(dm, &a.thr16, &gs);
+  a.g = im.add(go, n_q, gs, true);
+  a.k = im.add(k, n_k, 1.f, true);
+  a.v = im.add(v, n_k, 1.f, false);
+  a.H = H;
+  if (dm) a.dm = *dm;
+  a.out = out, a.lse = lse, a.dsum = dsum, a.scale = scale;
+  a.grad_q = gq, a.grad_k = gk, a.grad_v = gv;
+  a.split_keys = sq.split_keys;
+  a.n_split = sq.n_split;
+  a.part_dq = n_q > 0 && sq.n_split > 1 ? part_dq : nullptr;
+  switch (d) {
+    case 8: return fx_backward<8>(a, im, dm, st);
+    case 16: return fx_backward<16>(a, im, dm, st);
+    case 24: return fx_backward<24>(a, im, dm, st);
+    case 32: return fx_backward<32>(a, im, dm, st);
+    case 64: return fx_backward<64>(a, im, dm, st);
+    default: return set_error(NGT_ERR_UNSUPPORTED, "fp32 dense: head_dim %d", d);
+  }
+}
+
+}  // namespace ngt
