@@ -44,7 +44,7 @@ HIPCC_FLAGS = [
 # through their arithmetic to the outputs that depend on it.
 FILE_FLAGS = {
     "ngt_dense_mfma.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
-    "ngt_dense_f32.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
+    "ngt_dense_fx.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
 }
 
 

@@ -1,5 +1,6 @@
-// Dense full-window attention in fp32 on the matrix cores, head_dim d in
-// {8, 16, 24, 32, 64}.
+// Dense full-window attention on the matrix cores with fp32 weights: fp32
+// inputs, head_dim d in {8, 16, 24, 32, 64}, and bf16 inputs at d = 64 (P and
+// dS keep their 24 bits; the bf16 operands are one piece each).
 //
 // Products.  An fp32 value is the sum of three bf16 pieces h + m + l (each the
 // round-to-nearest of what is left, so the last remainder is zero or below
@@ -18,7 +19,8 @@
 // one-row-per-lane vector kernels -> these): 16,000 nodes, 8 heads, d = 8
 // 1,720 / 2,490 / 1,680 -> 1,060 / 1,780 / 1,030, with dropout 0.5 2,150 /
 // 2,810 / 1,980 -> 1,400 / 2,215 / 1,370; all-fp32 MFMAs 1,390 / 1,900 /
-// 1,300.  5,000 nodes, 8 heads, d = 64: 8,400 in all -> 650 / 1,210 / 555.
+// 1,300.  5,000 nodes, 8 heads, d = 64: 8,400 in all -> 650 / 1,210 / 555; the
+// same in bf16 (one piece per operand) 1,570 / 5,870 / 2,970 -> 275 / 635 / 290.
 //
 // A preparation kernel (k_fx_prep) writes the pieces of q * scale, k, v and dO
 // once per call, in the layout the LDS stages have:
@@ -77,18 +79,23 @@ constexpr float kHuge = 4.2535296e37f;  // 2^125: values past it take the fp32 M
 // Rows (queries or keys) a block owns with G tiles per wave.
 constexpr int block_rows(int G) { return kWaves * kT * G; }
 constexpr int out_tiles(int dh) { return (dh + 15) / 16; }
-// Row image: bytes per row (3 pieces x blocks of 8 columns, d = 24 padded to
+// np: pieces per operand, 3 for fp32 inputs and 1 for bf16 ones.
+// Row image: bytes per row (np pieces x blocks of 8 columns, d = 24 padded to
 // 4 blocks, the line length an odd multiple of 16).
 constexpr int col_blocks(int dh) { return dh == 24 ? 4 : dh / 8; }
-constexpr int row_bytes(int dh) {
-  const int units = 3 * col_blocks(dh);
+constexpr int row_bytes(int dh, int np) {
+  const int units = np * col_blocks(dh);
   return 16 * (units % 2 ? units : units + 1);
 }
 // Transposed image: lines per 32 rows, one per (piece, column) in whole
 // 16-line tiles; at d = 8 the first tile holds pieces h and m, the second l.
-constexpr int t_lines(int dh) { return dh == 8 ? 32 : 3 * 16 * out_tiles(dh); }
+constexpr int t_lines(int dh, int np) { return dh == 8 ? 32 : np * 16 * out_tiles(dh); }
 constexpr int kTLine = 80;  // 32 bf16 and 16 bytes of padding
-constexpr int t_bytes(int dh) { return t_lines(dh) * kTLine; }
+constexpr int t_bytes(int dh, int np) { return t_lines(dh, np) * kTLine; }
+template <typename T>
+constexpr int pieces() {
+  return sizeof(T) == 4 ? 3 : 1;
+}
 __host__ __device__ inline int padded(int n) { return (n + kPadRows - 1) / kPadRows * kPadRows; }
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
@@ -165,17 +172,17 @@ __device__ __forceinline__ bool kept(uint32_t bits, uint32_t thr16) { return bit
 
 // One operand matrix [n, H, d]: its fp32 rows and, per head, the images.
 struct Mat {
-  const float* x;
+  const void* x;        // [n, H, d] of the element type
   const char* row_img;  // [H][padded(n)][row_bytes]
   const char* t_img;    // [H][padded(n) / 32][t_bytes]
   const uint32_t* flag; // [H][padded(n) / 32]: nonzero where a value takes the fp32 body
   int32_t n;
-  float scale;          // applied to x before anything else
+  float scale;          // of x (in the images of fp32 inputs already)
 };
 
 // -------------------------------------------------------------- preparation
 struct PrepJob {
-  const float* x;
+  const void* x;
   char* row_img;
   char* t_img;  // null: not wanted
   uint32_t* flag;
@@ -187,8 +194,9 @@ struct PrepJobs {
 };
 
 // Block (step of 32 rows, head, matrix): both images of the step's rows and
-// the flag word.  Rows past n are zero.
-template <int DH>
+// the flag word.  Rows past n are zero.  bf16 inputs are their own single
+// piece and stay unscaled.
+template <typename T, int DH>
 __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t H) {
   const PrepJob job = jobs.j[wg_z()];
   const int step = wg_x(), h = wg_y();
@@ -199,13 +207,16 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
   for (int e = tid_x(); e < kStep * DH; e += kBlock) {
     const int r = e / DH, c = e - r * DH;
     const int64_t row = int64_t(step) * kStep + r;
-    const float v = row < job.n ? job.x[(row * H + h) * DH + c] * job.scale : 0.f;
+    float v = 0.f;
+    if (row < job.n) v = elem<T>::load(static_cast<const T*>(job.x) + (row * H + h) * DH + c);
+    if constexpr (pieces<T>() == 3) v *= job.scale;
     xs[r][c] = v;
     // (an unordered compare on the bits: this file does not honour NaNs)
     bad |= (__float_as_uint(v) & 0x7fffffffu) > __float_as_uint(kHuge);
   }
   bad = __syncthreads_or(bad);
   if (tid_x() == 0) job.flag[int64_t(h) * (n_pad / kStep) + step] = bad ? 1u : 0u;
+  constexpr int NP = pieces<T>();
   constexpr int NB = col_blocks(DH);
   for (int e = tid_x(); e < kStep * NB; e += kBlock) {
     const int r = e / NB, cb = e - r * NB;
@@ -213,14 +224,16 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[j] = 8 * cb + j < DH ? xs[r][(8 * cb + j) % DH] : 0.f;
     const Split sp = split8<true>(x);
-    char* p = job.row_img + (int64_t(h) * n_pad + step * kStep + r) * row_bytes(DH) + 16 * cb;
+    char* p = job.row_img + (int64_t(h) * n_pad + step * kStep + r) * row_bytes(DH, NP) + 16 * cb;
     *reinterpret_cast<bf16x8*>(p) = sp.h;
-    *reinterpret_cast<bf16x8*>(p + 16 * NB) = sp.m;
-    *reinterpret_cast<bf16x8*>(p + 32 * NB) = sp.l;
+    if constexpr (NP == 3) {
+      *reinterpret_cast<bf16x8*>(p + 16 * NB) = sp.m;
+      *reinterpret_cast<bf16x8*>(p + 32 * NB) = sp.l;
+    }
   }
   if (!job.t_img) return;
   constexpr int PL = DH == 8 ? 8 : 16 * out_tiles(DH);  // lines per piece
-  char* t = job.t_img + (int64_t(h) * (n_pad / kStep) + step) * t_bytes(DH);
+  char* t = job.t_img + (int64_t(h) * (n_pad / kStep) + step) * t_bytes(DH, NP);
   for (int e = tid_x(); e < 4 * PL; e += kBlock) {
     const int c = e / 4, gg = e - 4 * c;
     float x[8];
@@ -230,8 +243,10 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
     const Split sp = split8<true>(x);
     char* p = t + c * kTLine + 16 * gg;
     *reinterpret_cast<bf16x8*>(p) = sp.h;
-    *reinterpret_cast<bf16x8*>(p + PL * kTLine) = sp.m;
-    *reinterpret_cast<bf16x8*>(p + 2 * PL * kTLine) = sp.l;
+    if constexpr (NP == 3) {
+      *reinterpret_cast<bf16x8*>(p + PL * kTLine) = sp.m;
+      *reinterpret_cast<bf16x8*>(p + 2 * PL * kTLine) = sp.l;
+    }
     if constexpr (DH == 8)  // the last 8 lines of the second tile
       *reinterpret_cast<uint4*>(p + 3 * PL * kTLine) = make_uint4(0u, 0u, 0u, 0u);
   }
@@ -251,11 +266,13 @@ __device__ __forceinline__ bool any_flag(const Mat& a, const Mat& b, const Mat& 
 }
 
 // ------------------------------------------------------- fp32 MFMA products
-// A lane's d / 4 floats of row p, columns (d / 4) g ..
-template <int DH>
-__device__ __forceinline__ void load_quarter(const float* p, float (&x)[DH / 4]) {
+// A lane's d / 4 elements of row p, columns (d / 4) g ..
+template <int DH, typename T>
+__device__ __forceinline__ void load_quarter(const T* p, float (&x)[DH / 4]) {
   constexpr int KC = DH / 4;
-  if constexpr (KC % 4 == 0) {
+  if constexpr (sizeof(T) == 2) {
+    load_row<T, KC>(p, x);
+  } else if constexpr (KC % 4 == 0) {
 #pragma unroll
     for (int j = 0; j < KC; j += 4) {
       const float4 w = *reinterpret_cast<const float4*>(p + j);
@@ -274,8 +291,9 @@ __device__ __forceinline__ void load_quarter(const float* p, float (&x)[DH / 4])
 // product (an A operand of the products over rows is a column of 4 rows).  At
 // d = 8 and 24 the last tile's columns past d read the floats that follow and
 // end in registers that nothing stores.
-template <int DH, int G>
+template <typename T, int DH, int G>
 struct Fp32Ops {
+  static constexpr bool SCALED = true;  // operands carry their Mat's scale
   static constexpr int SB = DH > 32 ? 32 : 64;
   static constexpr int LD = DH + 4;
   static constexpr int MT = out_tiles(DH);
@@ -286,7 +304,8 @@ struct Fp32Ops {
                                                    int H, int g) {
 #pragma unroll
     for (int j = 0; j < DH / 4; ++j) r.x[u][j] = 0.f;
-    if (row < m.n) load_quarter<DH>(m.x + (row * H + h) * DH + (DH / 4) * g, r.x[u]);
+    if (row < m.n)
+      load_quarter<DH>(static_cast<const T*>(m.x) + (row * H + h) * DH + (DH / 4) * g, r.x[u]);
 #pragma unroll
     for (int j = 0; j < DH / 4; ++j) r.x[u][j] *= m.scale;
   }
@@ -302,9 +321,18 @@ struct Fp32Ops {
       for (int i = 0; i < NV; ++i) {
         const int e = tid_x() + i * kBlock;
         const int r = e / VPR, c = e - r * VPR;
-        w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (e < SB * VPR && row0 + r < m.n)
-          w[i] = *reinterpret_cast<const float4*>(m.x + (int64_t(row0 + r) * H + h) * DH + 4 * c);
+        const bool ok = e < SB * VPR && row0 + r < m.n;  // else read the first piece, use zeros
+        const T* p = static_cast<const T*>(m.x) + (int64_t(row0 + (ok ? r : 0)) * H + h) * DH +
+                     4 * (ok ? c : 0);
+        float4 x;
+        if constexpr (sizeof(T) == 4) {
+          x = *reinterpret_cast<const float4*>(p);
+        } else {
+          const uint2 b = *reinterpret_cast<const uint2*>(p);
+          x = make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u),
+                          __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u));
+        }
+        w[i] = ok ? x : make_float4(0.f, 0.f, 0.f, 0.f);
         w[i] = make_float4(w[i].x * m.scale, w[i].y * m.scale, w[i].z * m.scale, w[i].w * m.scale);
       }
     }
@@ -363,8 +391,17 @@ struct Fp32Ops {
 // bytes of a row image, its 16-byte unit chosen by (operand number, g): the
 // MFMAs of a tile pair A and B operands so that, over the four g, every piece
 // product down to 2^-16 is there once; the smallest come first.
-template <int DH>
+// With one piece per operand (d = 64) they are the row's two halves.
+template <int DH, int NP>
 struct Pairs {
+  static_assert(DH == 64, "one piece per operand: d = 64 only");
+  static constexpr int NA = 2, NB = 2, N = 2;
+  static constexpr __host__ __device__ int a_of(int n) { return n; }
+  static constexpr __host__ __device__ int b_of(int n) { return n; }
+  static __device__ __forceinline__ int unit(bool, int k, int g) { return 16 * (4 * k + g); }
+};
+template <int DH>
+struct Pairs<DH, 3> {
   static constexpr int NA = DH == 8 ? 2 : DH == 64 ? 6 : 3;   // A operands
   static constexpr int NB = DH <= 16 ? 2 : DH == 64 ? 6 : 3;  // B operands
   static constexpr int N = DH == 8 ? 2 : DH == 16 ? 3 : DH == 64 ? 12 : 6;
@@ -405,18 +442,20 @@ struct Pairs {
   }
 };
 
-template <int DH, int G>
+template <typename T, int DH, int G>
 struct PieceOps {
-  static constexpr int SB = DH <= 16 ? 64 : 32;
+  static constexpr int NP = pieces<T>();
+  static constexpr bool SCALED = NP == 3;
+  static constexpr int SB = DH <= 16 || NP == 1 ? 64 : 32;
   static constexpr int MT = out_tiles(DH);
-  using P = Pairs<DH>;
+  using P = Pairs<DH, NP>;
   struct Rows {
     bf16x8 x[G][P::NB];
   };
   static __device__ __forceinline__ void load_rows(Rows& r, int u, const Mat& m, int64_t row, int h,
                                                    int H, int g) {
     const int n_pad = padded(m.n);
-    const char* p = m.row_img + (int64_t(h) * n_pad + row) * row_bytes(DH);
+    const char* p = m.row_img + (int64_t(h) * n_pad + row) * row_bytes(DH, NP);
 #pragma unroll
     for (int k = 0; k < P::NB; ++k) {
       uint4 w = make_uint4(0u, 0u, 0u, 0u);
@@ -426,8 +465,8 @@ struct PieceOps {
   }
   template <bool ROW, bool COL>
   struct Staged {
-    static constexpr int RB = ROW ? SB * row_bytes(DH) : 0;
-    static constexpr int TB = COL ? SB / kStep * t_bytes(DH) : 0;
+    static constexpr int RB = ROW ? SB * row_bytes(DH, NP) : 0;
+    static constexpr int TB = COL ? SB / kStep * t_bytes(DH, NP) : 0;
     static constexpr int BYTES = RB + TB;
     static constexpr int NR = (RB / 16 + kBlock - 1) / kBlock, NT = (TB / 16 + kBlock - 1) / kBlock;
     static constexpr int NV = NR + NT;
@@ -435,8 +474,8 @@ struct PieceOps {
     uint4 w[NV];
     __device__ __forceinline__ void load(const Mat& m, int row0, int h, int H) {
       const int n_pad = padded(m.n);
-      const char* r = m.row_img + (int64_t(h) * n_pad + row0) * row_bytes(DH);
-      const char* t = m.t_img + (int64_t(h) * (n_pad / kStep) + row0 / kStep) * t_bytes(DH);
+      const char* r = m.row_img + (int64_t(h) * n_pad + row0) * row_bytes(DH, NP);
+      const char* t = m.t_img + (int64_t(h) * (n_pad / kStep) + row0 / kStep) * t_bytes(DH, NP);
 #pragma unroll
       for (int i = 0; i < NR; ++i) {
         const int e = 16 * (tid_x() + i * kBlock);
@@ -464,7 +503,7 @@ struct PieceOps {
                                              f32x4 (&x)[2][G]) const {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const char* p = lds + (r0 + kT * t + l16) * row_bytes(DH);
+        const char* p = lds + (r0 + kT * t + l16) * row_bytes(DH, NP);
         bf16x8 a[P::NA];
 #pragma unroll
         for (int k = 0; k < P::NA; ++k)
@@ -480,7 +519,7 @@ struct PieceOps {
     }
     __device__ __forceinline__ void accumulate(int r0, int g, int l16, const f32x4 (&x)[2][G],
                                                f32x4 (&acc)[G][MT]) const {
-      const char* p = lds + RB + (r0 / kStep) * t_bytes(DH) + l16 * kTLine + 16 * g;
+      const char* p = lds + RB + (r0 / kStep) * t_bytes(DH, NP) + l16 * kTLine + 16 * g;
       auto line = [&](int tile) {
         return *reinterpret_cast<const bf16x8*>(p + tile * kT * kTLine);
       };
@@ -500,6 +539,17 @@ struct PieceOps {
           acc[u][0] = mfma32(hm, sp[u].l, acc[u][0]);
           acc[u][0] = mfma32(hm, sp[u].m, acc[u][0]);
           acc[u][0] = mfma32(hm, sp[u].h, acc[u][0]);
+        }
+      } else if constexpr (NP == 1) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const bf16x8 ah = line(m);
+#pragma unroll
+          for (int u = 0; u < G; ++u) {
+            acc[u][m] = mfma32(ah, sp[u].l, acc[u][m]);
+            acc[u][m] = mfma32(ah, sp[u].m, acc[u][m]);
+            acc[u][m] = mfma32(ah, sp[u].h, acc[u][m]);
+          }
         }
       } else {
 #pragma unroll
@@ -546,14 +596,28 @@ __device__ __forceinline__ void add_acc(const f32x4 (&x)[G][MT], f32x4 (&acc)[G]
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[u][t] += x[u][t];
 }
-template <int DH, int G>
-__device__ __forceinline__ void store_acc(float* __restrict__ row, int u, int g, float f,
+// Multiplies both tiles of a step by f (the scale that unscaled operands leave out).
+template <int G>
+__device__ __forceinline__ void times(f32x4 (&x)[2][G], float f) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int u = 0; u < G; ++u) x[t][u] *= f;
+}
+template <int DH, int G, typename T>
+__device__ __forceinline__ void store_acc(T* __restrict__ row, int u, int g, float f,
                                           const f32x4 (&acc)[G][out_tiles(DH)]) {
 #pragma unroll
   for (int m = 0; m < out_tiles(DH); ++m)
-    if (kT * m + 4 * g < DH)
-      *reinterpret_cast<float4*>(row + kT * m + 4 * g) = make_float4(
-          acc[u][m][0] * f, acc[u][m][1] * f, acc[u][m][2] * f, acc[u][m][3] * f);
+    if (kT * m + 4 * g < DH) {
+      const float4 w = make_float4(acc[u][m][0] * f, acc[u][m][1] * f, acc[u][m][2] * f,
+                                   acc[u][m][3] * f);
+      if constexpr (sizeof(T) == 4)
+        *reinterpret_cast<float4*>(row + kT * m + 4 * g) = w;
+      else
+        *reinterpret_cast<uint2*>(row + kT * m + 4 * g) =
+            make_uint2(pack2_bf16(w.x, w.y), pack2_bf16(w.z, w.w));
+    }
 }
 
 // LDS of a kernel whose two bodies share one buffer.
@@ -565,7 +629,9 @@ struct FwdArgs {
   int32_t H;
   DropoutMask dm;
   uint32_t thr16;
-  float *out, *out32, *lse;
+  float drop_scale;
+  void* out;
+  float *out32, *lse;
   int32_t split_keys;
   float *part_ml, *part_acc;
   int32_t n_split, fwd_bx, score_bx;
@@ -577,7 +643,7 @@ struct FwdArgs {
 // moves only when some score exceeds it by more than kRebase, so after the
 // first step a wave rarely rescales; the column maximum over the lanes that
 // share a query is taken only then.
-template <class Ops, int DH, int G, bool DROP>
+template <class Ops, typename T, int DH, int G, bool DROP>
 __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z, char* lds) {
   constexpr int SB = Ops::SB, MT = out_tiles(DH);
   const int lane = tid_x() & (kWave - 1);
@@ -625,6 +691,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     for (int r0 = 0; r0 < SB && kb + r0 < k_end; r0 += kStep) {
       f32x4 s[2][G];  // S^T tiles: rows = keys kb + r0 + 16 t + 4 g + i
       sk.products(r0, g, l16, qf, s);
+      if constexpr (!Ops::SCALED) times(s, a.q.scale);
       if (kb + r0 + kStep > k_end) {  // keys past the end drop out
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -682,13 +749,14 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     for (int u = 0; u < G; ++u) l[u] += lst[u];
   }
   Ops::finish(acc);
+  const float ds = DROP && !Ops::SCALED ? a.drop_scale : 1.f;
 #pragma unroll
   for (int u = 0; u < G; ++u) {
     const float lsum = sum_rows(l[u]);
     if (qi[u] >= n_q) continue;
     const int64_t row = int64_t(qi[u]) * H + h;
     if (a.part_ml) {  // this split's softmax state, merged in split order later
-      store_acc<DH, G>(a.part_acc + (int64_t(z) * n_q * H + row) * DH, u, g, 1.f, acc);
+      store_acc<DH, G>(a.part_acc + (int64_t(z) * n_q * H + row) * DH, u, g, ds, acc);
       if (g == 0) {
         const int64_t r = (int64_t(z) * H + h) * n_q + qi[u];
         a.part_ml[2 * r] = m[u];
@@ -696,8 +764,8 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
       }
       continue;
     }
-    const float inv = a.k.n > 0 ? 1.0f / lsum : 0.f;
-    store_acc<DH, G>(a.out + row * DH, u, g, inv, acc);
+    const float inv = a.k.n > 0 ? ds / lsum : 0.f;
+    store_acc<DH, G>(static_cast<T*>(a.out) + row * DH, u, g, inv, acc);
     if (a.out32) store_acc<DH, G>(a.out32 + row * DH, u, g, inv, acc);
     if (g == 0)
       a.lse[int64_t(h) * n_q + qi[u]] =
@@ -738,6 +806,7 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
     for (int r0 = 0; r0 < SB && qb + r0 < n_q; r0 += kStep) {  // rows past n_q are zero
       f32x4 s[2][G];
       sq.products(r0, g, l16, kf, s);
+      if constexpr (!Ops::SCALED) times(s, a.q.scale);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -763,10 +832,10 @@ constexpr int fwd_lds() {
 // The forward and the column scores in one launch: grid z < n_split are
 // forward blocks, the last slice holds the score blocks, which fill the CUs
 // that the forward's last round leaves idle.
-template <int DH, int G, bool DROP>
+template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
-  using F = Fp32Ops<DH, G>;
-  using P = PieceOps<DH, G>;
+  using F = Fp32Ops<T, DH, G>;
+  using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(fwd_lds<F>(), fwd_lds<P>())];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
   if (bx >= (z == a.n_split ? a.score_bx : a.fwd_bx)) return;  // block-uniform, before any barrier
@@ -777,9 +846,9 @@ __global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
     else
       scores_body<P, DH, G>(a, bx, h, lds);
   } else if (plain) {
-    fwd_body<F, DH, G, DROP>(a, bx, h, z, lds);
+    fwd_body<F, T, DH, G, DROP>(a, bx, h, z, lds);
   } else {
-    fwd_body<P, DH, G, DROP>(a, bx, h, z, lds);
+    fwd_body<P, T, DH, G, DROP>(a, bx, h, z, lds);
   }
 }
 
@@ -789,10 +858,13 @@ struct BwdArgs {
   int32_t H;
   DropoutMask dm;
   uint32_t thr16;
-  const float *out, *lse;
+  float drop_scale;
+  const void* out;     // of the element type
+  const float* out32;  // the forward's fp32 copy, or null
+  const float* lse;
   float* dsum;
   float scale;
-  float *grad_q, *grad_k, *grad_v;
+  void *grad_q, *grad_k, *grad_v;
   int32_t split_keys;
   float* part_dq;
   int32_t n_split, kv_bx, comb_bx;
@@ -801,7 +873,7 @@ struct BwdArgs {
 // Query-major: dQ^T += K^T dS^T over the keys of split z, S and dP recomputed
 // as in the forward.  D = dO . out per query is formed here and stored (split
 // 0) for the dK/dV pass.
-template <class Ops, int DH, int G, bool DROP>
+template <class Ops, typename T, int DH, int G, bool DROP>
 __device__ __forceinline__ void bwd_q_body(const BwdArgs& a, int bx, int h, int z, char* lds) {
   constexpr int SB = Ops::SB, MT = out_tiles(DH);
   const int lane = tid_x() & (kWave - 1);
@@ -825,8 +897,11 @@ __device__ __forceinline__ void bwd_q_body(const BwdArgs& a, int bx, int h, int 
     if (ok) {
       const int64_t o = (int64_t(qi[u]) * H + h) * DH + (DH / 4) * g;
       float gq[DH / 4], oq[DH / 4];
-      load_quarter<DH>(a.g.x + o, gq);
-      load_quarter<DH>(a.out + o, oq);
+      load_quarter<DH>(static_cast<const T*>(a.g.x) + o, gq);
+      if (a.out32)
+        load_quarter<DH>(a.out32 + o, oq);
+      else
+        load_quarter<DH>(static_cast<const T*>(a.out) + o, oq);
 #pragma unroll
       for (int j = 0; j < DH / 4; ++j) d = fmaf(gq[j], oq[j], d);
     }
@@ -859,6 +934,8 @@ __device__ __forceinline__ void bwd_q_body(const BwdArgs& a, int bx, int h, int 
       f32x4 s[2][G], dp[2][G];
       sk.products(r0, g, l16, qf, s);
       sv.products(r0, g, l16, gf, dp);
+      if constexpr (!Ops::SCALED) times(s, a.q.scale);
+      if constexpr (!Ops::SCALED && DROP) times(dp, a.drop_scale);
       if (kb + r0 + kStep > k_end) {  // keys past the end: p = 0
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -901,7 +978,7 @@ __device__ __forceinline__ void bwd_q_body(const BwdArgs& a, int bx, int h, int 
     if (a.part_dq)
       store_acc<DH, G>(a.part_dq + (int64_t(z) * n_q * H + row) * DH, u, g, 1.f, acc);
     else
-      store_acc<DH, G>(a.grad_q + row * DH, u, g, a.scale, acc);
+      store_acc<DH, G>(static_cast<T*>(a.grad_q) + row * DH, u, g, a.scale, acc);
   }
 }
 
@@ -910,30 +987,31 @@ constexpr int bwd_q_lds() {
   return Ops::template Staged<true, true>::BYTES + Ops::template Staged<true, false>::BYTES;
 }
 
-template <int DH, int G, bool DROP>
+template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_bwd_q(const BwdArgs a) {
-  using F = Fp32Ops<DH, G>;
-  using P = PieceOps<DH, G>;
+  using F = Fp32Ops<T, DH, G>;
+  using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(bwd_q_lds<F>(), bwd_q_lds<P>())];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
   if (any_flag(a.q, a.k, a.v, h) || any_flag(a.g, a.g, a.g, h))
-    bwd_q_body<F, DH, G, DROP>(a, bx, h, z, lds);
+    bwd_q_body<F, T, DH, G, DROP>(a, bx, h, z, lds);
   else
-    bwd_q_body<P, DH, G, DROP>(a, bx, h, z, lds);
+    bwd_q_body<P, T, DH, G, DROP>(a, bx, h, z, lds);
 }
 
 // grad_q = scale * sum of the key splits' partial dQ, added in split order.
+template <typename T>
 __device__ __forceinline__ void dq_combine(const BwdArgs& a, int64_t n, int64_t b, int64_t nb) {
   for (int64_t t = b * kBlock + tid_x(); t < n; t += nb * kBlock) {
     float x = a.part_dq[t];
     for (int s = 1; s < a.n_split; ++s) x += a.part_dq[int64_t(s) * n + t];
-    a.grad_q[t] = x * a.scale;
+    elem<T>::store(static_cast<T*>(a.grad_q) + t, x * a.scale);
   }
 }
 
 // Key-major: dV^T += dO^T P and dK^T += (Q scale)^T dS, rows = queries
 // (staged, Q already scaled), lanes = keys.
-template <class Ops, int DH, int G, bool DROP>
+template <class Ops, typename T, int DH, int G, bool DROP>
 __device__ __forceinline__ void bwd_kv_body(const BwdArgs& a, int bx, int h, char* lds, float* ls,
                                             float* ds) {
   constexpr int SB = Ops::SB, MT = out_tiles(DH);
@@ -986,6 +1064,8 @@ __device__ __forceinline__ void bwd_kv_body(const BwdArgs& a, int bx, int h, cha
       f32x4 s[2][G], dp[2][G];
       sq.products(r0, g, l16, kf, s);
       sg.products(r0, g, l16, vf, dp);
+      if constexpr (!Ops::SCALED) times(s, a.q.scale);
+      if constexpr (!Ops::SCALED && DROP) times(dp, a.drop_scale);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int r = r0 + kT * t + 4 * g;  // queries qb + r .. + 3
@@ -1030,8 +1110,9 @@ __device__ __forceinline__ void bwd_kv_body(const BwdArgs& a, int bx, int h, cha
   for (int u = 0; u < G; ++u) {
     if (kj[u] >= a.k.n) continue;
     const int64_t o = (int64_t(kj[u]) * H + h) * DH;
-    store_acc<DH, G>(a.grad_k + o, u, g, 1.f, dk);
-    store_acc<DH, G>(a.grad_v + o, u, g, 1.f, dv);
+    store_acc<DH, G>(static_cast<T*>(a.grad_k) + o, u, g, Ops::SCALED ? 1.f : a.scale, dk);
+    store_acc<DH, G>(static_cast<T*>(a.grad_v) + o, u, g,
+                     Ops::SCALED || !DROP ? 1.f : a.drop_scale, dv);
   }
 }
 
@@ -1042,23 +1123,23 @@ constexpr int bwd_kv_lds() {
 
 // Blocks at grid x >= kv_bx add the dQ splits' partials instead of taking
 // keys (that merge needs no launch of its own).
-template <int DH, int G, bool DROP>
+template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
-  using F = Fp32Ops<DH, G>;
-  using P = PieceOps<DH, G>;
+  using F = Fp32Ops<T, DH, G>;
+  using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(bwd_kv_lds<F>(), bwd_kv_lds<P>())];
   __shared__ __align__(16) float ls[64];
   __shared__ __align__(16) float ds[64];
   const int bx = wg_x(), h = wg_y();
   if (bx >= a.kv_bx) {  // block-uniform
-    dq_combine(a, int64_t(a.q.n) * a.H * DH, int64_t(bx - a.kv_bx) * a.H + h,
+    dq_combine<T>(a, int64_t(a.q.n) * a.H * DH, int64_t(bx - a.kv_bx) * a.H + h,
                int64_t(a.comb_bx) * a.H);
     return;
   }
   if (any_flag(a.q, a.k, a.v, h) || any_flag(a.g, a.g, a.g, h))
-    bwd_kv_body<F, DH, G, DROP>(a, bx, h, lds, ls, ds);
+    bwd_kv_body<F, T, DH, G, DROP>(a, bx, h, lds, ls, ds);
   else
-    bwd_kv_body<P, DH, G, DROP>(a, bx, h, lds, ls, ds);
+    bwd_kv_body<P, T, DH, G, DROP>(a, bx, h, lds, ls, ds);
 }
 
 // ------------------------------------------------------------------ host side
@@ -1089,37 +1170,29 @@ MfSplit split_keys_for(int n_q, int n_k, int H, int d, int target_waves, int64_t
   return {(n_k + keys - 1) / keys, keys};
 }
 
-constexpr int rt_row_bytes(int d) {
-  return d == 8 ? row_bytes(8) : d == 16 ? row_bytes(16) : d == 24 ? row_bytes(24)
-       : d == 32 ? row_bytes(32) : row_bytes(64);
+size_t row_image_bytes(int n, int H, int d, int np) {
+  return align256(size_t(padded(n)) * H * row_bytes(d, np));
 }
-constexpr int rt_t_bytes(int d) {
-  return d == 8 ? t_bytes(8) : d == 16 ? t_bytes(16) : d == 24 ? t_bytes(24)
-       : d == 32 ? t_bytes(32) : t_bytes(64);
-}
-size_t row_image_bytes(int n, int H, int d) {
-  return align256(size_t(padded(n)) * H * rt_row_bytes(d));
-}
-size_t t_image_bytes(int n, int H, int d) {
-  return align256(size_t(padded(n) / kStep) * H * rt_t_bytes(d));
+size_t t_image_bytes(int n, int H, int d, int np) {
+  return align256(size_t(padded(n) / kStep) * H * t_bytes(d, np));
 }
 size_t flag_bytes(int n, int H) { return align256(size_t(padded(n) / kStep) * H * 4); }
 
 // Assigns one matrix's images in the workspace and adds its preparation job.
 struct Images {
   char* ws;
-  int H, d;
+  int H, d, np;
   PrepJobs jobs{};
   int n_jobs = 0, max_rows = 0;
-  Mat add(const float* x, int n, float scale, bool want_t) {
+  Mat add(const void* x, int n, float scale, bool want_t) {
     PrepJob& j = jobs.j[n_jobs++];
     j.x = x;
     j.row_img = ws;
-    ws += row_image_bytes(n, H, d);
+    ws += row_image_bytes(n, H, d, np);
     j.t_img = nullptr;
     if (want_t) {
       j.t_img = ws;
-      ws += t_image_bytes(n, H, d);
+      ws += t_image_bytes(n, H, d, np);
     }
     j.flag = reinterpret_cast<uint32_t*>(ws);
     ws += flag_bytes(n, H);
@@ -1130,43 +1203,43 @@ struct Images {
   }
 };
 
-template <int DH>
+template <typename T, int DH>
 int run_prep(const Images& im, hipStream_t st) {
   if (im.max_rows == 0) return NGT_OK;
   KernelTimer timer_("dense_prep", st);
-  hipLaunchKernelGGL((k_fx_prep<DH>), dim3(im.max_rows / kStep, im.H, im.n_jobs), dim3(kBlock), 0,
+  hipLaunchKernelGGL((k_fx_prep<T, DH>), dim3(im.max_rows / kStep, im.H, im.n_jobs), dim3(kBlock), 0,
                      st, im.jobs, im.H);
   NGT_HIP_CHECK(hipGetLastError());
   return NGT_OK;
 }
 
-template <int DH, int G>
+template <typename T, int DH, int G>
 int fx_fwd(FwdArgs a, const DropoutMask* dm, hipStream_t st) {
   a.fwd_bx = blocks_of(a.q.n, block_rows(G));
   a.score_bx = a.part && a.k.n > 0 ? blocks_of(a.k.n, block_rows(G)) : 0;
   const dim3 grid(std::max(a.fwd_bx, a.score_bx), a.H, a.n_split + (a.score_bx > 0 ? 1 : 0));
   KernelTimer timer_("dense_fwd", st);
   if (dm)
-    hipLaunchKernelGGL((k_fx_fwd<DH, G, true>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_fx_fwd<T, DH, G, true>), grid, dim3(kBlock), 0, st, a);
   else
-    hipLaunchKernelGGL((k_fx_fwd<DH, G, false>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_fx_fwd<T, DH, G, false>), grid, dim3(kBlock), 0, st, a);
   NGT_HIP_CHECK(hipGetLastError());
   return NGT_OK;
 }
 
-template <int DH, int G>
+template <typename T, int DH, int G>
 int fx_bwd_q(const BwdArgs& a, const DropoutMask* dm, hipStream_t st) {
   KernelTimer timer_("dense_bwd_q", st);
   const dim3 grid(blocks_of(a.q.n, block_rows(G)), a.H, a.n_split);
   if (dm)
-    hipLaunchKernelGGL((k_fx_bwd_q<DH, G, true>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_fx_bwd_q<T, DH, G, true>), grid, dim3(kBlock), 0, st, a);
   else
-    hipLaunchKernelGGL((k_fx_bwd_q<DH, G, false>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_fx_bwd_q<T, DH, G, false>), grid, dim3(kBlock), 0, st, a);
   NGT_HIP_CHECK(hipGetLastError());
   return NGT_OK;
 }
 
-template <int DH, int G>
+template <typename T, int DH, int G>
 int fx_bwd_kv(BwdArgs a, const DropoutMask* dm, hipStream_t st) {
   KernelTimer timer_("dense_bwd_kv", st);
   a.kv_bx = blocks_of(a.k.n, block_rows(G));
@@ -1176,57 +1249,59 @@ int fx_bwd_kv(BwdArgs a, const DropoutMask* dm, hipStream_t st) {
   a.comb_bx = a.part_dq ? int((n_dq + per - 1) / per) : 0;
   const dim3 grid(a.kv_bx + a.comb_bx, a.H);
   if (dm)
-    hipLaunchKernelGGL((k_fx_bwd_kv<DH, G, true>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_fx_bwd_kv<T, DH, G, true>), grid, dim3(kBlock), 0, st, a);
   else
-    hipLaunchKernelGGL((k_fx_bwd_kv<DH, G, false>), grid, dim3(kBlock), 0, st, a);
+    hipLaunchKernelGGL((k_fx_bwd_kv<T, DH, G, false>), grid, dim3(kBlock), 0, st, a);
   NGT_HIP_CHECK(hipGetLastError());
   return NGT_OK;
 }
 
-template <int DH>
+template <typename T, int DH>
 int fx_forward(FwdArgs a, const Images& im, const DropoutMask* dm, hipStream_t st) {
-  NGT_CHECK_OK(run_prep<DH>(im, st));
-  if constexpr (DH == 64) return fx_fwd<DH, 1>(a, dm, st);
+  NGT_CHECK_OK((run_prep<T, DH>(im, st)));
+  if constexpr (DH == 64) return fx_fwd<T, DH, 1>(a, dm, st);
   else
-    return tiles_per_wave(a.q.n, a.H, DH) == 2 ? fx_fwd<DH, 2>(a, dm, st) : fx_fwd<DH, 1>(a, dm, st);
+    return tiles_per_wave(a.q.n, a.H, DH) == 2 ? fx_fwd<T, DH, 2>(a, dm, st) : fx_fwd<T, DH, 1>(a, dm, st);
 }
 
-template <int DH>
+template <typename T, int DH>
 int fx_backward(const BwdArgs& a, const Images& im, const DropoutMask* dm, hipStream_t st) {
-  NGT_CHECK_OK(run_prep<DH>(im, st));
+  NGT_CHECK_OK((run_prep<T, DH>(im, st)));
   if constexpr (DH == 64) {
-    if (a.q.n > 0) NGT_CHECK_OK((fx_bwd_q<DH, 1>(a, dm, st)));
-    return a.k.n > 0 ? fx_bwd_kv<DH, 1>(a, dm, st) : NGT_OK;
+    if (a.q.n > 0) NGT_CHECK_OK((fx_bwd_q<T, DH, 1>(a, dm, st)));
+    return a.k.n > 0 ? fx_bwd_kv<T, DH, 1>(a, dm, st) : NGT_OK;
   } else {
     if (a.q.n > 0)
-      NGT_CHECK_OK((tiles_per_wave(a.q.n, a.H, DH) == 2 ? fx_bwd_q<DH, 2>(a, dm, st)
-                                                        : fx_bwd_q<DH, 1>(a, dm, st)));
+      NGT_CHECK_OK((tiles_per_wave(a.q.n, a.H, DH) == 2 ? fx_bwd_q<T, DH, 2>(a, dm, st)
+                                                        : fx_bwd_q<T, DH, 1>(a, dm, st)));
     if (a.k.n > 0)
-      return tiles_per_wave(a.k.n, a.H, DH) == 2 ? fx_bwd_kv<DH, 2>(a, dm, st)
-                                                 : fx_bwd_kv<DH, 1>(a, dm, st);
+      return tiles_per_wave(a.k.n, a.H, DH) == 2 ? fx_bwd_kv<T, DH, 2>(a, dm, st)
+                                                 : fx_bwd_kv<T, DH, 1>(a, dm, st);
     return NGT_OK;
   }
 }
 
 }  // namespace
 
-MfSplit f32_fwd_split(int n_q, int n_k, int H, int d, bool node_scores) {
+MfSplit fx_fwd_split(int n_q, int n_k, int H, int d, bool node_scores) {
   const int rows = block_rows(tiles_per_wave(n_k, H, d));
   const int64_t score_waves = node_scores ? int64_t(blocks_of(n_k, rows)) * H * kWaves : 0;
   return split_keys_for(n_q, n_k, H, d, 6144, score_waves, "NGT_DENSE_F32_FWD_SPLIT");
 }
-MfSplit f32_dq_split(int n_q, int n_k, int H, int d) {
+MfSplit fx_dq_split(int n_q, int n_k, int H, int d) {
   return split_keys_for(n_q, n_k, H, d, 6144, 0, "NGT_DENSE_F32_DQ_SPLIT");
 }
 
 // Bytes of the images and flags that the two directions keep in the workspace.
-size_t f32_fwd_image_bytes(int n_q, int n_k, int H, int d) {
-  return row_image_bytes(n_q, H, d) + flag_bytes(n_q, H) + 2 * row_image_bytes(n_k, H, d) +
-         t_image_bytes(n_k, H, d) + 2 * flag_bytes(n_k, H);
+size_t fx_fwd_image_bytes(int dtype, int n_q, int n_k, int H, int d) {
+  const int np = dtype == NGT_F32 ? 3 : 1;
+  return row_image_bytes(n_q, H, d, np) + flag_bytes(n_q, H) + 2 * row_image_bytes(n_k, H, d, np) +
+         t_image_bytes(n_k, H, d, np) + 2 * flag_bytes(n_k, H);
 }
-size_t f32_bwd_image_bytes(int n_q, int n_k, int H, int d) {
-  return 2 * (row_image_bytes(n_q, H, d) + t_image_bytes(n_q, H, d) + flag_bytes(n_q, H)) +
-         2 * (row_image_bytes(n_k, H, d) + flag_bytes(n_k, H)) + t_image_bytes(n_k, H, d);
+size_t fx_bwd_image_bytes(int dtype, int n_q, int n_k, int H, int d) {
+  const int np = dtype == NGT_F32 ? 3 : 1;
+  return 2 * (row_image_bytes(n_q, H, d, np) + t_image_bytes(n_q, H, d, np) + flag_bytes(n_q, H)) +
+         2 * (row_image_bytes(n_k, H, d, np) + flag_bytes(n_k, H)) + t_image_bytes(n_k, H, d, np);
 }
 
 // (threshold << 16, scale) of a mask for kept(); a threshold of 2^16 (nothing
@@ -1237,17 +1312,16 @@ static void drop_terms(const DropoutMask* dm, uint32_t* thr16, float* scale) {
   *scale = !dm ? 1.f : none ? 0.f : dm->scale;
 }
 
-int f32_dense_fwd(int d, const float* q, const float* k, const float* v, int n_q, int n_k, int H,
-                  float scale, const DropoutMask* dm, float* out, float* out32, float* lse,
-                  float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
-                  hipStream_t st) {
-  Images im{images, H, d};
+int fx_dense_fwd(int dtype, int d, const void* q, const void* k, const void* v, int n_q, int n_k,
+                 int H, float scale, const DropoutMask* dm, void* out, float* out32, float* lse,
+                 float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
+                 hipStream_t st) {
+  Images im{images, H, d, dtype == NGT_F32 ? 3 : 1};
   FwdArgs a{};
+  drop_terms(dm, &a.thr16, &a.drop_scale);
   a.q = im.add(q, n_q, scale, false);
   a.k = im.add(k, n_k, 1.f, false);
-  float vs;
-  drop_terms(dm, &a.thr16, &vs);
-  a.v = im.add(v, n_k, vs, true);
+  a.v = im.add(v, n_k, a.drop_scale, true);
   a.H = H;
   if (dm) a.dm = *dm;
   a.out = out, a.out32 = out32, a.lse = lse;
@@ -1255,43 +1329,46 @@ int f32_dense_fwd(int d, const float* q, const float* k, const float* v, int n_q
   a.n_split = sp.n_split;
   if (sp.n_split > 1) a.part_ml = part_ml, a.part_acc = part_acc;
   a.part = part;
-  switch (d) {
-    case 8: return fx_forward<8>(a, im, dm, st);
-    case 16: return fx_forward<16>(a, im, dm, st);
-    case 24: return fx_forward<24>(a, im, dm, st);
-    case 32: return fx_forward<32>(a, im, dm, st);
-    case 64: return fx_forward<64>(a, im, dm, st);
-    default: return set_error(NGT_ERR_UNSUPPORTED, "fp32 dense: head_dim %d", d);
-  }
+  if (dtype == NGT_BF16 && d == 64) return fx_forward<bf16_t, 64>(a, im, dm, st);
+  if (dtype == NGT_F32) switch (d) {
+      case 8: return fx_forward<float, 8>(a, im, dm, st);
+      case 16: return fx_forward<float, 16>(a, im, dm, st);
+      case 24: return fx_forward<float, 24>(a, im, dm, st);
+      case 32: return fx_forward<float, 32>(a, im, dm, st);
+      case 64: return fx_forward<float, 64>(a, im, dm, st);
+      default: break;
+    }
+  return set_error(NGT_ERR_UNSUPPORTED, "dense: head_dim %d", d);
 }
 
-int f32_dense_bwd(int d, const float* q, const float* k, const float* v, const float* go,
-                  const float* out, const float* lse, float* dsum, int n_q, int n_k, int H,
-                  float scale, const DropoutMask* dm, float* gq, float* gk, float* gv, MfSplit sq,
-                  float* part_dq, char* images, hipStream_t st) {
-  Images im{images, H, d};
+int fx_dense_bwd(int dtype, int d, const void* q, const void* k, const void* v, const void* go,
+                 const void* out, const float* out32, const float* lse, float* dsum, int n_q,
+                 int n_k, int H, float scale, const DropoutMask* dm, void* gq, void* gk, void* gv,
+                 MfSplit sq, float* part_dq, char* images, hipStream_t st) {
+  Images im{images, H, d, dtype == NGT_F32 ? 3 : 1};
   BwdArgs a{};
+  drop_terms(dm, &a.thr16, &a.drop_scale);
   a.q = im.add(q, n_q, scale, true);
-  float gs;
-  drop_terms(dm, &a.thr16, &gs);
-  a.g = im.add(go, n_q, gs, true);
+  a.g = im.add(go, n_q, a.drop_scale, true);
   a.k = im.add(k, n_k, 1.f, true);
   a.v = im.add(v, n_k, 1.f, false);
   a.H = H;
   if (dm) a.dm = *dm;
-  a.out = out, a.lse = lse, a.dsum = dsum, a.scale = scale;
+  a.out = out, a.out32 = out32, a.lse = lse, a.dsum = dsum, a.scale = scale;
   a.grad_q = gq, a.grad_k = gk, a.grad_v = gv;
   a.split_keys = sq.split_keys;
   a.n_split = sq.n_split;
   a.part_dq = n_q > 0 && sq.n_split > 1 ? part_dq : nullptr;
-  switch (d) {
-    case 8: return fx_backward<8>(a, im, dm, st);
-    case 16: return fx_backward<16>(a, im, dm, st);
-    case 24: return fx_backward<24>(a, im, dm, st);
-    case 32: return fx_backward<32>(a, im, dm, st);
-    case 64: return fx_backward<64>(a, im, dm, st);
-    default: return set_error(NGT_ERR_UNSUPPORTED, "fp32 dense: head_dim %d", d);
-  }
+  if (dtype == NGT_BF16 && d == 64) return fx_backward<bf16_t, 64>(a, im, dm, st);
+  if (dtype == NGT_F32) switch (d) {
+      case 8: return fx_backward<float, 8>(a, im, dm, st);
+      case 16: return fx_backward<float, 16>(a, im, dm, st);
+      case 24: return fx_backward<float, 24>(a, im, dm, st);
+      case 32: return fx_backward<float, 32>(a, im, dm, st);
+      case 64: return fx_backward<float, 64>(a, im, dm, st);
+      default: break;
+    }
+  return set_error(NGT_ERR_UNSUPPORTED, "dense: head_dim %d", d);
 }
 
 }  // namespace ngt
