@@ -563,7 +563,9 @@ int ngt_ppr_step_direct(const int64_t* rowptr, const int64_t* col, const float* 
  *   with out = NULL, read result, then again with cap = result[0].
  * Workspace from ngt_subgraph_workspace_bytes(n_nodes, n_edges, n_set, ...)
  * with n_edges = edges of edge_index (COO form) or entries of col (CSR form);
- * the map it holds is rebuilt by every call.  The CSR form spreads each row
+ * the map it holds is rebuilt by every call, except that the _emit forms use
+ * the map and counts which the last call with the same arguments left in the
+ * workspace: count, read result, then emit with cap = result[0].  The CSR form spreads each row
  * over waves of 2,048 entries, so hub rows do not serialise.
  */
 int ngt_subgraph_workspace_bytes(int64_t n_nodes, int64_t n_edges, int32_t n_set, size_t* bytes);
@@ -573,6 +575,13 @@ int ngt_subgraph_coo(const int64_t* edge_index, int64_t n_edges, int64_t n_nodes
 int ngt_subgraph_csr(const int64_t* rowptr, const int64_t* col, int64_t n_col, int64_t n_nodes,
                      const int64_t* node_set, int32_t n_set, int64_t* out, int64_t cap,
                      int64_t* result, void* workspace, size_t workspace_bytes, void* stream);
+int ngt_subgraph_coo_emit(const int64_t* edge_index, int64_t n_edges, int64_t n_nodes,
+                          const int64_t* subset, int32_t n_subset, int64_t* out, int64_t cap,
+                          int64_t* result, void* workspace, size_t workspace_bytes, void* stream);
+int ngt_subgraph_csr_emit(const int64_t* rowptr, const int64_t* col, int64_t n_col,
+                          int64_t n_nodes, const int64_t* node_set, int32_t n_set, int64_t* out,
+                          int64_t cap, int64_t* result, void* workspace, size_t workspace_bytes,
+                          void* stream);
 
 /*
  * Per-kernel timing (no counterpart in the reference: instrumentation for the

@@ -152,6 +152,8 @@ SIGNATURES = {
                             C.c_float, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
     "ngt_subgraph_workspace_bytes": [_i64, _i64, _i32, _vp],
     "ngt_subgraph_coo": [_vp, _i64, _i64, _vp, _i32, _vp, _i64, _vp, _vp, _sz, _vp],
+    "ngt_subgraph_coo_emit": [_vp, _i64, _i64, _vp, _i32, _vp, _i64, _vp, _vp, _sz, _vp],
+    "ngt_subgraph_csr_emit": [_vp, _vp, _i64, _i64, _vp, _i32, _vp, _i64, _vp, _vp, _sz, _vp],
     "ngt_subgraph_csr": [_vp, _vp, _i64, _i64, _vp, _i32, _vp, _i64, _vp, _vp, _sz, _vp],
     "ngt_timing_enable": [_i32],
     "ngt_timing_summary": [C.c_char_p, _sz],

@@ -142,7 +142,6 @@ class WindowAdjacency:
         self.mem = torch.empty(total, dtype=torch.int32, device=dev)
         for (name, shape), o in zip(layout, offs):
             setattr(self, name, self.mem[o:o + math.prod(shape)].view(shape))
-        self.info_dev.zero_()
         s = _lib.WindowCSR()
         s.n_q, s.n_k, s.n_edges, s.chunk_q, s.chunk_k = n_q, n_k, E, chunk, chunk
         s.small_q, s.small_k = small_q, small

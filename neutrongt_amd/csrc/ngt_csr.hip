@@ -15,8 +15,17 @@
 // (NeutronGT/models/graphormer_dist_node_level.py:75-97).  Here the ordering is
 // made canonical: query-major rows are sorted by (dst, src, edge id) and
 // key-major rows by (src, dst, edge id), so the CSR is a pure function of the
-// edge list (bit-exact, independent of launch shapes).  The sort is rocPRIM's
-// LSD radix sort, which is stable, so duplicate edges keep edge-id order.
+// edge list (bit-exact, independent of launch shapes).  Three stable sorts by
+// one endpoint each make both orders: by src, then by dst, which leaves the
+// edges in (dst, src, edge id) order, then those by src again, which gives
+// (src, dst, edge id) and, with query-major positions as the values, the map
+// between the two.  Keys are 32 bits with bits_for(n) significant ones (15 at
+// 16,384 rows: two digit passes), where sorting the combined 64-bit keys of
+// each order took five passes of 12 bytes.  The sorts are rocPRIM's radix sort;
+// its default switches to a merge sort below 1 M entries, 23 launches for the
+// 0.67 M edges of a 16,384-node window against 5 or 6 (one window's build
+// there is bound by launches, not bytes), so SortConfig keeps radix passes
+// down to 16 K entries.
 #include "ngt_common.h"
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -48,63 +57,79 @@ inline unsigned bits_for(uint64_t v) {
 
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-__global__ void k_make_keys(const int64_t* __restrict__ src, const int64_t* __restrict__ dst,
-                            int64_t E, int32_t n_q, int32_t n_k, uint64_t* __restrict__ key_q,
-                            uint64_t* __restrict__ key_k, int32_t* __restrict__ eid,
+using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                              rocprim::default_config, 16 * 1024>;
+
+// 32-bit endpoints; edges outside the window become {n_k, n_q}, which sorts
+// behind every row in both orders.
+__global__ void k_endpoints(const int64_t* __restrict__ src, const int64_t* __restrict__ dst,
+                            int64_t E, int32_t n_q, int32_t n_k, uint32_t* __restrict__ src32,
+                            uint32_t* __restrict__ dst32, int32_t* __restrict__ eid,
                             int32_t* __restrict__ info) {
-  const uint64_t sentinel = uint64_t(n_q) * uint64_t(n_k);
   for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < E;
        e += int64_t(gridDim.x) * blockDim.x) {
     const int64_t s = src[e];
     const int64_t d = dst[e];
     const bool ok = s >= 0 && s < n_k && d >= 0 && d < n_q;
-    if (ok) {
-      key_q[e] = uint64_t(d) * uint64_t(n_k) + uint64_t(s);
-      key_k[e] = uint64_t(s) * uint64_t(n_q) + uint64_t(d);
-    } else {
-      key_q[e] = sentinel;
-      key_k[e] = sentinel;
-      atomicAdd(info + NGT_INFO_BAD_EDGES, 1);
-    }
+    src32[e] = ok ? uint32_t(s) : uint32_t(n_k);
+    dst32[e] = ok ? uint32_t(d) : uint32_t(n_q);
+    if (!ok) atomicAdd(info + NGT_INFO_BAD_EDGES, 1);
     eid[e] = static_cast<int32_t>(e);
   }
 }
 
-// rowptr[r] = first sorted position whose row >= r; col = key % n_cols.
-// Sentinel keys (dropped edges) map to row n_rows and therefore sit past
-// rowptr[n_rows].
-__global__ void k_rowptr(const uint64_t* __restrict__ keys, int64_t E, uint64_t n_cols,
-                         int32_t n_rows, int32_t* __restrict__ rowptr,
-                         int32_t* __restrict__ col) {
+__global__ void k_gather_u32(const uint32_t* __restrict__ x, const int32_t* __restrict__ at,
+                             int64_t E, uint32_t* __restrict__ out) {
+  for (int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; p < E;
+       p += int64_t(gridDim.x) * blockDim.x)
+    out[p] = x[at[p]];
+}
+
+// rowptr[r] = first position p of the sorted rows with rows[p] >= r; edges
+// outside the window (row n_rows) sit past rowptr[n_rows].
+__device__ __forceinline__ void fill_rowptr(const uint32_t* __restrict__ rows, int64_t E,
+                                            int64_t p, int32_t n_rows,
+                                            int32_t* __restrict__ rowptr) {
+  const int64_t r_cur = p < E ? int64_t(rows[p]) : int64_t(n_rows);
+  const int64_t r_prev = p > 0 ? int64_t(rows[p - 1]) : -1;
+  for (int64_t r = r_prev + 1; r <= r_cur; ++r) rowptr[r] = static_cast<int32_t>(p);
+}
+
+// Query-major rows: row pointers and columns; the columns are also the third
+// sort's keys (n_k for an edge outside the window) and the positions its values.
+__global__ void k_rows_q(const uint32_t* __restrict__ dst_sorted, const int32_t* __restrict__ perm,
+                         const uint32_t* __restrict__ src32, int64_t E, int32_t n_q, int32_t n_k,
+                         int32_t* __restrict__ rowptr, int32_t* __restrict__ col,
+                         uint32_t* __restrict__ key, int32_t* __restrict__ pos) {
   for (int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; p <= E;
        p += int64_t(gridDim.x) * blockDim.x) {
-    int64_t r_cur = n_rows;
     if (p < E) {
-      const uint64_t r = keys[p] / n_cols;
-      r_cur = r < uint64_t(n_rows) ? int64_t(r) : int64_t(n_rows);
-      col[p] = r_cur < n_rows ? static_cast<int32_t>(keys[p] % n_cols) : 0;
+      const uint32_t s = src32[perm[p]];
+      col[p] = s < uint32_t(n_k) ? static_cast<int32_t>(s) : 0;
+      key[p] = s;
+      pos[p] = static_cast<int32_t>(p);
     }
-    int64_t r_prev = -1;
-    if (p > 0) {
-      const uint64_t r = keys[p - 1] / n_cols;
-      r_prev = r < uint64_t(n_rows) ? int64_t(r) : int64_t(n_rows);
-    }
-    for (int64_t r = r_prev + 1; r <= r_cur; ++r) rowptr[r] = static_cast<int32_t>(p);
+    fill_rowptr(dst_sorted, E, p, n_q, rowptr);
   }
 }
 
-__global__ void k_scatter_pos(const int32_t* __restrict__ perm, int64_t E,
-                              int32_t* __restrict__ pos_of_eid) {
-  for (int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; p < E;
-       p += int64_t(gridDim.x) * blockDim.x)
-    pos_of_eid[perm[p]] = static_cast<int32_t>(p);
-}
-
-__global__ void k_compose(const int32_t* __restrict__ perm, const int32_t* __restrict__ tpos_of_eid,
-                          int64_t E, int32_t* __restrict__ q2t) {
-  for (int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; p < E;
-       p += int64_t(gridDim.x) * blockDim.x)
-    q2t[p] = tpos_of_eid[perm[p]];
+// Key-major rows: row pointers, columns, edge ids, and q2t.
+__global__ void k_rows_k(const uint32_t* __restrict__ src_sorted, const int32_t* __restrict__ qpos,
+                         const int32_t* __restrict__ perm, const uint32_t* __restrict__ dst_sorted,
+                         int64_t E, int32_t n_q, int32_t n_k, int32_t* __restrict__ t_rowptr,
+                         int32_t* __restrict__ t_col, int32_t* __restrict__ t_perm,
+                         int32_t* __restrict__ q2t) {
+  for (int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; t <= E;
+       t += int64_t(gridDim.x) * blockDim.x) {
+    if (t < E) {
+      const int32_t p = qpos[t];
+      const uint32_t d = dst_sorted[p];
+      t_col[t] = d < uint32_t(n_q) ? static_cast<int32_t>(d) : 0;
+      t_perm[t] = perm[p];
+      q2t[p] = static_cast<int32_t>(t);
+    }
+    fill_rowptr(src_sorted, E, t, n_k, t_rowptr);
+  }
 }
 
 __device__ __forceinline__ Count3 row_counts(int32_t deg, int32_t chunk) {
@@ -225,13 +250,13 @@ __global__ void k_emit_order(const int32_t* __restrict__ srow, int32_t n,
     order[n - 1 - p] = srow[p];
 }
 
-__global__ void k_ends(const uint64_t* __restrict__ key_q, const uint64_t* __restrict__ key_k,
-                       const int32_t* __restrict__ rowptr, int32_t n_q, int32_t n_k,
-                       int32_t* __restrict__ info) {
+__global__ void k_ends(const uint32_t* __restrict__ dst_sorted,
+                       const uint32_t* __restrict__ src_sorted, const int32_t* __restrict__ rowptr,
+                       int32_t n_q, int32_t* __restrict__ info) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int32_t nv = rowptr[n_q];  // valid edges (dropped ones sort last)
-    info[NGT_INFO_DST_END] = nv > 0 ? int32_t(key_q[nv - 1] / uint64_t(n_k)) + 1 : 0;
-    info[NGT_INFO_SRC_END] = nv > 0 ? int32_t(key_k[nv - 1] / uint64_t(n_q)) + 1 : 0;
+    info[NGT_INFO_DST_END] = nv > 0 ? int32_t(dst_sorted[nv - 1]) + 1 : 0;
+    info[NGT_INFO_SRC_END] = nv > 0 ? int32_t(src_sorted[nv - 1]) + 1 : 0;
   }
 }
 
@@ -247,8 +272,8 @@ inline int grid_for(int64_t n) {
 }
 
 struct CsrLayout {
-  size_t key_a, key_b, key_c, eid, tpos, cnt, cnt_scan, deg_a, deg_b, row_a, row_b, deg_c, row_c,
-      temp, total;
+  size_t src32, dst32, key_a, key_b, key_c, val_a, val_b, cnt, cnt_scan, deg_a, deg_b, row_a,
+      row_b, deg_c, row_c, temp, total;
   size_t temp_bytes;
 };
 
@@ -256,9 +281,9 @@ int csr_layout(int64_t E, int32_t n_q, int32_t n_k, CsrLayout* L) {
   const int64_t n_rows = n_q > n_k ? n_q : n_k;
   size_t sort_bytes = 0, scan_bytes = 0;
   const size_t n = static_cast<size_t>(E > 0 ? E : 1);
-  NGT_HIP_CHECK(rocprim::radix_sort_pairs(nullptr, sort_bytes, (uint64_t*)nullptr,
-                                          (uint64_t*)nullptr, (int32_t*)nullptr,
-                                          (int32_t*)nullptr, n, 0u, 64u, hipStream_t(0)));
+  NGT_HIP_CHECK(rocprim::radix_sort_pairs<SortConfig>(
+      nullptr, sort_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, (int32_t*)nullptr,
+      (int32_t*)nullptr, n, 0u, 32u, hipStream_t(0)));
   NGT_HIP_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, (Count3*)nullptr, (Count3*)nullptr,
                                         Count3{0, 0, 0}, size_t(n_rows > 0 ? n_rows : 1),
                                         Count3Plus(), hipStream_t(0)));
@@ -268,11 +293,13 @@ int csr_layout(int64_t E, int32_t n_q, int32_t n_k, CsrLayout* L) {
     off += align256(bytes);
     return at;
   };
-  L->key_a = take(n * 8);
-  L->key_b = take(n * 8);
-  L->key_c = take(n * 8);
-  L->eid = take(n * 4);
-  L->tpos = take(n * 4);
+  L->src32 = take(n * 4);
+  L->dst32 = take(n * 4);
+  L->key_a = take(n * 4);
+  L->key_b = take(n * 4);
+  L->key_c = take(n * 4);
+  L->val_a = take(n * 4);
+  L->val_b = take(n * 4);
   L->cnt = take(size_t(n_rows + 1) * sizeof(Count3));
   L->cnt_scan = take(size_t(n_rows + 1) * sizeof(Count3));
   L->deg_a = take(size_t(n_rows + 1) * 4);
@@ -413,43 +440,43 @@ extern "C" int ngt_csr_build(const int64_t* edge_index, ngt_window_csr* csr, voi
 
   hipStream_t st = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
-  uint64_t* key_a = reinterpret_cast<uint64_t*>(ws + L.key_a);
-  uint64_t* key_b = reinterpret_cast<uint64_t*>(ws + L.key_b);
-  uint64_t* key_c = reinterpret_cast<uint64_t*>(ws + L.key_c);
-  int32_t* eid = reinterpret_cast<int32_t*>(ws + L.eid);
-  int32_t* tpos = reinterpret_cast<int32_t*>(ws + L.tpos);
+  uint32_t* src32 = reinterpret_cast<uint32_t*>(ws + L.src32);
+  uint32_t* dst32 = reinterpret_cast<uint32_t*>(ws + L.dst32);
+  uint32_t* key_a = reinterpret_cast<uint32_t*>(ws + L.key_a);
+  uint32_t* key_b = reinterpret_cast<uint32_t*>(ws + L.key_b);
+  uint32_t* key_c = reinterpret_cast<uint32_t*>(ws + L.key_c);
+  int32_t* val_a = reinterpret_cast<int32_t*>(ws + L.val_a);
+  int32_t* val_b = reinterpret_cast<int32_t*>(ws + L.val_b);
 
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, csr->info, NGT_INFO_LEN);
   NGT_HIP_CHECK(hipGetLastError());
-  const uint64_t sentinel = uint64_t(n_q) * uint64_t(n_k);
-  const unsigned end_bit = bits_for(sentinel);
-  if (E > 0) {
-    // key_a <- query-major keys, key_c <- key-major keys.
-    hipLaunchKernelGGL(k_make_keys, dim3(grid_for(E)), dim3(kBlock), 0, st, edge_index,
-                       edge_index + E, E, n_q, n_k, key_a, key_c, eid, csr->info);
-    NGT_HIP_CHECK(hipGetLastError());
+  auto sort = [&](uint32_t* key_in, uint32_t* key_out, int32_t* val_in, int32_t* val_out,
+                  int32_t n) -> int {  // keys 0 .. n
     size_t tb = L.temp_bytes;
-    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, tb, key_a, key_b, eid, csr->perm,
-                                            size_t(E), 0u, end_bit, st));
-    tb = L.temp_bytes;
-    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, tb, key_c, key_a, eid, csr->t_perm,
-                                            size_t(E), 0u, end_bit, st));
-    // Sorted: key_b = query-major keys, key_a = key-major keys.
+    NGT_HIP_CHECK(rocprim::radix_sort_pairs<SortConfig>(ws + L.temp, tb, key_in, key_out, val_in,
+                                                        val_out, size_t(E), 0u,
+                                                        bits_for(uint64_t(n)), st));
+    return NGT_OK;
+  };
+  if (E > 0) {
+    hipLaunchKernelGGL(k_endpoints, dim3(grid_for(E)), dim3(kBlock), 0, st, edge_index,
+                       edge_index + E, E, n_q, n_k, src32, dst32, val_a, csr->info);
+    NGT_HIP_CHECK(hipGetLastError());
+    NGT_CHECK_OK(sort(src32, key_a, val_a, val_b, n_k));  // val_b: edge ids by src
+    hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(E)), dim3(kBlock), 0, st, dst32, val_b, E,
+                       key_a);
+    NGT_HIP_CHECK(hipGetLastError());
+    NGT_CHECK_OK(sort(key_a, key_b, val_b, csr->perm, n_q));  // key_b: dst, query-major
   }
-  hipLaunchKernelGGL(k_rowptr, dim3(grid_for(E + 1)), dim3(kBlock), 0, st, key_b, E,
-                     uint64_t(n_k > 0 ? n_k : 1), n_q, csr->rowptr, csr->col);
+  hipLaunchKernelGGL(k_rows_q, dim3(grid_for(E + 1)), dim3(kBlock), 0, st, key_b, csr->perm, src32,
+                     E, n_q, n_k, csr->rowptr, csr->col, key_a, val_a);
   NGT_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_rowptr, dim3(grid_for(E + 1)), dim3(kBlock), 0, st, key_a, E,
-                     uint64_t(n_q > 0 ? n_q : 1), n_k, csr->t_rowptr, csr->t_col);
+  if (E > 0) NGT_CHECK_OK(sort(key_a, key_c, val_a, val_b, n_k));  // key_c: src, key-major
+  hipLaunchKernelGGL(k_rows_k, dim3(grid_for(E + 1)), dim3(kBlock), 0, st, key_c, val_b, csr->perm,
+                     key_b, E, n_q, n_k, csr->t_rowptr, csr->t_col, csr->t_perm, csr->q2t);
   NGT_HIP_CHECK(hipGetLastError());
   if (E > 0) {
-    hipLaunchKernelGGL(k_scatter_pos, dim3(grid_for(E)), dim3(kBlock), 0, st, csr->t_perm, E,
-                       tpos);
-    NGT_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_compose, dim3(grid_for(E)), dim3(kBlock), 0, st, csr->perm, tpos, E,
-                       csr->q2t);
-    NGT_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_ends, dim3(1), dim3(64), 0, st, key_b, key_a, csr->rowptr, n_q, n_k,
+    hipLaunchKernelGGL(k_ends, dim3(1), dim3(64), 0, st, key_b, key_c, csr->rowptr, n_q,
                        csr->info);
     NGT_HIP_CHECK(hipGetLastError());
   }

@@ -212,6 +212,29 @@ __device__ __forceinline__ bool find_segment(int64_t w, const int64_t* seg_end, 
   return true;
 }
 
+// Set positions (-1: outside the set) of the entries p, p + 64, ... of a
+// segment, kAhead of them with their loads in flight together: a segment of
+// 2,048 entries is a wave's serial chain of column and position loads (16,384
+// of 200,000 nodes, 2.6 M entries: count and emit 36 us each one round of 64 at
+// a time).  Returns whether some column was outside the graph.
+constexpr int kAhead = 8;
+__device__ __forceinline__ bool load_positions(const int64_t* __restrict__ col, int64_t n_nodes,
+                                               const int32_t* __restrict__ pos, int64_t p,
+                                               int64_t end, int32_t (&pn)[kAhead]) {
+  int64_t nb[kAhead];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) nb[u] = p + 64 * u < end ? col[p + 64 * u] : 0;
+  bool bad = false;
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    const bool in = p + 64 * u < end;
+    const bool ok = nb[u] >= 0 && nb[u] < n_nodes;
+    bad |= in && !ok;
+    pn[u] = in && ok ? pos[nb[u]] : -1;
+  }
+  return bad;
+}
+
 __global__ __launch_bounds__(kBlock) void k_csr_count(const int64_t* rowptr, const int64_t* col,
                                                       int64_t n_nodes, const int64_t* set,
                                                       int32_t n_set, const int64_t* nseg,
@@ -232,17 +255,11 @@ __global__ __launch_bounds__(kBlock) void k_csr_count(const int64_t* rowptr, con
   }
   int64_t c = 0;
   bool bad = false;
-  for (int64_t p0 = sg.b; p0 < sg.e; p0 += 64) {
-    const int64_t p = p0 + lane;
-    bool keep = false;
-    if (p < sg.e) {
-      const int64_t nb = col[p];
-      if (nb < 0 || nb >= n_nodes)
-        bad = true;
-      else
-        keep = pos[nb] >= 0;
-    }
-    c += __popcll(__ballot(keep));
+  for (int64_t p0 = sg.b; p0 < sg.e; p0 += kAhead * 64) {
+    int32_t pn[kAhead];
+    bad |= load_positions(col, n_nodes, pos, p0 + lane, sg.e, pn);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) c += __popcll(__ballot(pn[u] >= 0));
   }
   if (bad) atomicOr(&result[1], kBadEdge);
   if (lane == 0) cnt[w] = c;
@@ -261,23 +278,22 @@ __global__ __launch_bounds__(kBlock) void k_csr_emit(const int64_t* rowptr, cons
   Segment sg;
   if (!find_segment(w, seg_end, nseg, n_set, rowptr, set, sg)) return;
   int64_t at = end[w] - cnt[w];
-  for (int64_t p0 = sg.b; p0 < sg.e; p0 += 64) {
-    const int64_t p = p0 + lane;
-    int32_t pn = -1;
-    if (p < sg.e) {
-      const int64_t nb = col[p];
-      if (nb >= 0 && nb < n_nodes) pn = pos[nb];
-    }
-    const bool keep = pn >= 0;
-    const unsigned long long m = __ballot(keep);
-    if (keep) {
-      const int64_t k = at + lane_rank(m);
-      if (k < cap) {
-        out[k] = sg.row;
-        out[cap + k] = pn;
+  for (int64_t p0 = sg.b; p0 < sg.e; p0 += kAhead * 64) {
+    int32_t pn[kAhead];
+    load_positions(col, n_nodes, pos, p0 + lane, sg.e, pn);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const bool keep = pn[u] >= 0;
+      const unsigned long long m = __ballot(keep);
+      if (keep) {
+        const int64_t k = at + lane_rank(m);
+        if (k < cap) {
+          out[k] = sg.row;
+          out[cap + k] = pn[u];
+        }
       }
+      at += __popcll(m);
     }
-    at += __popcll(m);
   }
 }
 
@@ -293,11 +309,12 @@ inline int grid_for(int64_t n) {
   return int(g);
 }
 
-int sub_prepare(int64_t n_nodes, int64_t n_items, const int64_t* set, int32_t n_set, void* ws,
+int sub_prepare(bool init, int64_t n_nodes, int64_t n_items, const int64_t* set, int32_t n_set, void* ws,
                 size_t ws_bytes, hipStream_t s, int64_t* result, SubLayout* L, const char* who) {
   NGT_CHECK_OK(sub_layout(n_nodes, n_items, n_set, L));
   if (!ws || ws_bytes < L->total)
     return set_error(NGT_ERR_ARG, "%s: workspace too small (%zu < %zu)", who, ws_bytes, L->total);
+  if (!init) return NGT_OK;
   char* base = static_cast<char*>(ws);
   int32_t* pos = reinterpret_cast<int32_t*>(base + L->pos);
   auto* res = reinterpret_cast<unsigned long long*>(result);
@@ -340,9 +357,11 @@ extern "C" int ngt_subgraph_workspace_bytes(int64_t n_nodes, int64_t n_edges, in
   return NGT_OK;
 }
 
-extern "C" int ngt_subgraph_coo(const int64_t* edge_index, int64_t n_edges, int64_t n_nodes,
-                                const int64_t* subset, int32_t n_subset, int64_t* out, int64_t cap,
-                                int64_t* result, void* ws, size_t ws_bytes, void* stream) {
+// count: the map, the counts and their scan; without it the workspace still
+// holds those of an earlier call with the same arguments.
+static int subgraph_coo(bool count, const int64_t* edge_index, int64_t n_edges, int64_t n_nodes,
+                        const int64_t* subset, int32_t n_subset, int64_t* out, int64_t cap,
+                        int64_t* result, void* ws, size_t ws_bytes, void* stream) {
   if (n_edges < 0 || n_nodes < 0 || n_subset < 0 || cap < 0 || !result ||
       (n_edges > 0 && !edge_index) || (n_subset > 0 && !subset))
     return set_error(NGT_ERR_ARG, "ngt_subgraph_coo: bad arguments");
@@ -351,8 +370,8 @@ extern "C" int ngt_subgraph_coo(const int64_t* edge_index, int64_t n_edges, int6
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t tiles = (n_edges + kTile - 1) / kTile;
   SubLayout L;
-  NGT_CHECK_OK(sub_prepare(n_nodes, tiles > n_subset ? tiles : n_subset, subset, n_subset, ws,
-                           ws_bytes, s, result, &L, "ngt_subgraph_coo"));
+  NGT_CHECK_OK(sub_prepare(count, n_nodes, tiles > n_subset ? tiles : n_subset, subset, n_subset,
+                           ws, ws_bytes, s, result, &L, "ngt_subgraph_coo"));
   if (tiles == 0) return NGT_OK;
   char* base = static_cast<char*>(ws);
   const int32_t* pos = reinterpret_cast<const int32_t*>(base + L.pos);
@@ -360,9 +379,11 @@ extern "C" int ngt_subgraph_coo(const int64_t* edge_index, int64_t n_edges, int6
   const int64_t* end = reinterpret_cast<const int64_t*>(base + L.end);
   auto* res = reinterpret_cast<unsigned long long*>(result);
   KernelTimer timer_("subgraph_coo", s);
-  hipLaunchKernelGGL(k_coo_count, dim3(tiles), dim3(kBlock), 0, s, edge_index, n_edges, n_nodes,
-                     pos, cnt, res);
-  NGT_CHECK_OK(sub_scan(L, base, tiles, result, s));
+  if (count) {
+    hipLaunchKernelGGL(k_coo_count, dim3(tiles), dim3(kBlock), 0, s, edge_index, n_edges, n_nodes,
+                       pos, cnt, res);
+    NGT_CHECK_OK(sub_scan(L, base, tiles, result, s));
+  }
   if (out && cap > 0)
     hipLaunchKernelGGL(k_coo_emit, dim3(tiles), dim3(kBlock), 0, s, edge_index, n_edges, n_nodes,
                        pos, cnt, end, out, cap);
@@ -370,10 +391,23 @@ extern "C" int ngt_subgraph_coo(const int64_t* edge_index, int64_t n_edges, int6
   return NGT_OK;
 }
 
-extern "C" int ngt_subgraph_csr(const int64_t* rowptr, const int64_t* col, int64_t n_col,
-                                int64_t n_nodes, const int64_t* node_set, int32_t n_set,
-                                int64_t* out, int64_t cap, int64_t* result, void* ws,
-                                size_t ws_bytes, void* stream) {
+extern "C" int ngt_subgraph_coo(const int64_t* edge_index, int64_t n_edges, int64_t n_nodes,
+                                const int64_t* subset, int32_t n_subset, int64_t* out, int64_t cap,
+                                int64_t* result, void* ws, size_t ws_bytes, void* stream) {
+  return subgraph_coo(true, edge_index, n_edges, n_nodes, subset, n_subset, out, cap, result, ws,
+                      ws_bytes, stream);
+}
+extern "C" int ngt_subgraph_coo_emit(const int64_t* edge_index, int64_t n_edges, int64_t n_nodes,
+                                     const int64_t* subset, int32_t n_subset, int64_t* out,
+                                     int64_t cap, int64_t* result, void* ws, size_t ws_bytes,
+                                     void* stream) {
+  return subgraph_coo(false, edge_index, n_edges, n_nodes, subset, n_subset, out, cap, result, ws,
+                      ws_bytes, stream);
+}
+
+static int subgraph_csr(bool count, const int64_t* rowptr, const int64_t* col, int64_t n_col,
+                        int64_t n_nodes, const int64_t* node_set, int32_t n_set, int64_t* out,
+                        int64_t cap, int64_t* result, void* ws, size_t ws_bytes, void* stream) {
   if (n_nodes < 0 || n_col < 0 || n_set < 0 || cap < 0 || !result || (n_nodes > 0 && !rowptr) ||
       (n_col > 0 && !col) || (n_set > 0 && !node_set))
     return set_error(NGT_ERR_ARG, "ngt_subgraph_csr: bad arguments");
@@ -382,7 +416,7 @@ extern "C" int ngt_subgraph_csr(const int64_t* rowptr, const int64_t* col, int64
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t n_waves = int64_t(n_set) + (n_col + kSeg - 1) / kSeg;
   SubLayout L;
-  NGT_CHECK_OK(sub_prepare(n_nodes, n_waves, node_set, n_set, ws, ws_bytes, s, result, &L,
+  NGT_CHECK_OK(sub_prepare(count, n_nodes, n_waves, node_set, n_set, ws, ws_bytes, s, result, &L,
                            "ngt_subgraph_csr"));
   if (n_set == 0) return NGT_OK;
   char* base = static_cast<char*>(ws);
@@ -393,18 +427,35 @@ extern "C" int ngt_subgraph_csr(const int64_t* rowptr, const int64_t* col, int64
   int64_t* seg_end = reinterpret_cast<int64_t*>(base + L.seg_end);
   auto* res = reinterpret_cast<unsigned long long*>(result);
   KernelTimer timer_("subgraph_csr", s);
-  hipLaunchKernelGGL(k_csr_segs, dim3((n_set + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rowptr,
-                     n_col, n_nodes, node_set, n_set, nseg, res);
-  size_t temp_bytes = L.temp_bytes;
-  NGT_HIP_CHECK(rocprim::inclusive_scan(base + L.temp, temp_bytes, nseg, seg_end, size_t(n_set),
-                                        rocprim::plus<int64_t>(), s));
   const int64_t grid = (n_waves + kWaves - 1) / kWaves;
-  hipLaunchKernelGGL(k_csr_count, dim3(grid), dim3(kBlock), 0, s, rowptr, col, n_nodes, node_set,
-                     n_set, nseg, seg_end, n_waves, pos, cnt, res);
-  NGT_CHECK_OK(sub_scan(L, base, n_waves, result, s));
+  if (count) {
+    hipLaunchKernelGGL(k_csr_segs, dim3((n_set + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rowptr,
+                       n_col, n_nodes, node_set, n_set, nseg, res);
+    size_t temp_bytes = L.temp_bytes;
+    NGT_HIP_CHECK(rocprim::inclusive_scan(base + L.temp, temp_bytes, nseg, seg_end, size_t(n_set),
+                                          rocprim::plus<int64_t>(), s));
+    hipLaunchKernelGGL(k_csr_count, dim3(grid), dim3(kBlock), 0, s, rowptr, col, n_nodes, node_set,
+                       n_set, nseg, seg_end, n_waves, pos, cnt, res);
+    NGT_CHECK_OK(sub_scan(L, base, n_waves, result, s));
+  }
   if (out && cap > 0)
     hipLaunchKernelGGL(k_csr_emit, dim3(grid), dim3(kBlock), 0, s, rowptr, col, n_nodes, node_set,
                        n_set, nseg, seg_end, n_waves, pos, cnt, end, out, cap);
   NGT_HIP_CHECK(hipGetLastError());
   return NGT_OK;
+}
+
+extern "C" int ngt_subgraph_csr(const int64_t* rowptr, const int64_t* col, int64_t n_col,
+                                int64_t n_nodes, const int64_t* node_set, int32_t n_set,
+                                int64_t* out, int64_t cap, int64_t* result, void* ws,
+                                size_t ws_bytes, void* stream) {
+  return subgraph_csr(true, rowptr, col, n_col, n_nodes, node_set, n_set, out, cap, result, ws,
+                      ws_bytes, stream);
+}
+extern "C" int ngt_subgraph_csr_emit(const int64_t* rowptr, const int64_t* col, int64_t n_col,
+                                     int64_t n_nodes, const int64_t* node_set, int32_t n_set,
+                                     int64_t* out, int64_t cap, int64_t* result, void* ws,
+                                     size_t ws_bytes, void* stream) {
+  return subgraph_csr(false, rowptr, col, n_col, n_nodes, node_set, n_set, out, cap, result, ws,
+                      ws_bytes, stream);
 }

@@ -186,16 +186,18 @@ _SUBGRAPH_ERRORS = {1: "node id out of range in the node set", 2: "duplicate nod
 
 def _subgraph_job(call, n_nodes: int, n_edges: int, n_set: int, device, stream, host):
     """Count pass, the count copied into ``host`` (pinned) asynchronously, a
-    yield, then the emit pass into an exact [2, n] tensor: a job of
-    _streams.run_in_flight."""
+    yield, then the emit pass into an exact [2, n] tensor, from the map and
+    counts that the count pass left in the workspace: a job of
+    _streams.run_in_flight.  ``call`` = (count, emit) entry points."""
+    count, emit = call
     lib = _lib.load()
     nb = C.c_size_t()
     _lib.check(lib.ngt_subgraph_workspace_bytes(n_nodes, n_edges, n_set, C.byref(nb)))
     with torch.cuda.stream(stream):
         ws = torch.empty(max(nb.value, 1), dtype=torch.uint8, device=device)
-        result = torch.zeros(2, dtype=torch.int64, device=device)
+        result = torch.empty(2, dtype=torch.int64, device=device)  # the count pass clears it
     sp = stream.cuda_stream
-    _lib.check(call(None, 0, result.data_ptr(), ws.data_ptr(), nb.value, sp))
+    _lib.check(count(None, 0, result.data_ptr(), ws.data_ptr(), nb.value, sp))
     with torch.cuda.stream(stream):
         host[:2].copy_(result, non_blocking=True)
     landed = torch.cuda.Event()
@@ -209,7 +211,7 @@ def _subgraph_job(call, n_nodes: int, n_edges: int, n_set: int, device, stream, 
     with torch.cuda.stream(stream):
         out = torch.empty(2, n, dtype=torch.int64, device=device)
     if n:
-        _lib.check(call(out.data_ptr(), n, result.data_ptr(), ws.data_ptr(), nb.value, sp))
+        _lib.check(emit(out.data_ptr(), n, result.data_ptr(), ws.data_ptr(), nb.value, sp))
     return out
 
 
@@ -222,9 +224,10 @@ def _coo_call(subset: torch.Tensor, edge_index: torch.Tensor, num_nodes: int):
     subset = subset.to(torch.int64).contiguous()
     ei = edge_index.to(torch.int64).contiguous()
     E, n_set = int(ei.shape[1]), int(subset.numel())
-    call = lambda out, cap, res, ws, wb, st: lib.ngt_subgraph_coo(  # noqa: E731
+    call = lambda fn: lambda out, cap, res, ws, wb, st: fn(  # noqa: E731
         ei.data_ptr(), E, int(num_nodes), subset.data_ptr(), n_set, out, cap, res, ws, wb, st)
-    return functools.partial(_subgraph_job, call, int(num_nodes), E, n_set, subset.device)
+    return functools.partial(_subgraph_job,
+                             (call(lib.ngt_subgraph_coo), call(lib.ngt_subgraph_coo_emit)), int(num_nodes), E, n_set, subset.device)
 
 
 def _csr_call(node_set: torch.Tensor, rowptr: torch.Tensor, col: torch.Tensor):
@@ -237,10 +240,11 @@ def _csr_call(node_set: torch.Tensor, rowptr: torch.Tensor, col: torch.Tensor):
     n_nodes, n_set = int(rowptr.numel()) - 1, int(node_set.numel())
     if n_nodes < 0:
         raise ValueError("subgraph_from_csr: rowptr must have n_nodes + 1 entries")
-    call = lambda out, cap, res, ws, wb, st: lib.ngt_subgraph_csr(  # noqa: E731
+    call = lambda fn: lambda out, cap, res, ws, wb, st: fn(  # noqa: E731
         rowptr.data_ptr(), col.data_ptr(), int(col.numel()), n_nodes, node_set.data_ptr(), n_set,
         out, cap, res, ws, wb, st)
-    return functools.partial(_subgraph_job, call, n_nodes, int(col.numel()), n_set,
+    return functools.partial(_subgraph_job,
+                             (call(lib.ngt_subgraph_csr), call(lib.ngt_subgraph_csr_emit)), n_nodes, int(col.numel()), n_set,
                              node_set.device)
 
 
