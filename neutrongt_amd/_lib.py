@@ -199,10 +199,10 @@ EXT_PATH = Path(__file__).resolve().parent / "ngt_autograd.so"
 
 
 def autograd_ext():
-    """The C++ autograd node of the sparse attention (ngt_autograd.so, built
-    beside the library), bound to the loaded library's entry points; None when
-    it is not built -- the Python autograd.Function then drives the same
-    library calls."""
+    """The C++ autograd nodes of the sparse attention and the encoder's layers
+    (ngt_autograd.so, built beside the library), bound to the loaded library's
+    entry points; None when it is not built -- the Python autograd.Functions
+    then drive the same library calls."""
     global _ext
     if _ext is not None:
         return _ext or None
@@ -227,10 +227,20 @@ def autograd_ext():
                     raise RuntimeError(f"{EXT_PATH.name} was built against another "
                                        "ngt_window_csr; rebuild it")
                 addr = lambda fn: C.cast(fn, C.c_void_p).value
-                mod.init(addr(lib.ngt_sparse_fwd_ext), addr(lib.ngt_sparse_bwd_strided),
-                         addr(lib.ngt_last_error))
+                mod.init({name: addr(getattr(lib, name)) for name in SIGNATURES})
                 _ext = mod
     return _ext or None
+
+
+def node_ext():
+    """autograd_ext() where a C++ node can stand in for a Python
+    autograd.Function, else None: under torch.func transforms, torch.compile
+    and jit tracing the call stays with the Python class, which those handle
+    (or refuse) by their own rules."""
+    if (torch._C._are_functorch_transforms_active() or torch.compiler.is_compiling()
+            or torch.jit.is_tracing()):
+        return None
+    return autograd_ext()
 
 
 def stream_ptr(device) -> int:

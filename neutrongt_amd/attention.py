@@ -214,12 +214,13 @@ def window_attention(q, k, v, adj, scale, lo=CLAMP_LO, hi=CLAMP_HI, eps=EPS, k_e
     without the GIL on the autograd engine's device thread -- else by
     SparseAttentionFunction.  q/k/v (and k_ext/v_ext) as that function takes
     them: contiguous, 16-byte aligned, on the GPU.  ``interleave_grads``: see
-    SparseAttentionFunction."""
+    SparseAttentionFunction.  The C++ node also takes q/k/v as [1, N, H, d]
+    (all three alike); out is then [1, N_q, H * d]."""
     ext = _lib.autograd_ext()
     if ext is None:
         return SparseAttentionFunction.apply(q, k, v, adj, scale, lo, hi, eps, k_ext, v_ext,
                                              interleave_grads)
-    H, d = q.shape[1], q.shape[2]
+    H, d = q.shape[-2], q.shape[-1]
     fwd_bytes, bwd_bytes = adj.workspace_bytes(H, d)
     return ext.sparse_attention(q, k, v, k_ext, v_ext, adj.csr_bytes, adj.mem, adj.dst_end,
                                 float(scale), float(lo), float(hi), float(eps), fwd_bytes,
@@ -241,36 +242,46 @@ def sparse_attention(q, k, v, edge_index, num_heads=None, scale=None, cache: Adj
     score and receives a gradient when it requires one.  ``interleave_grads``
     (N_q == N_k, no bias): dQ, dK, dV as views of one [N, 3, H, d] buffer.
     """
+    return _sparse(q, k, v, edge_index, num_heads, scale, cache, lo, hi, eps, kv_ext, attn_bias,
+                   interleave_grads, False)
+
+
+def _sparse(q, k, v, edge_index, num_heads, scale, cache, lo, hi, eps, kv_ext, attn_bias,
+            interleave_grads, flat):
+    """sparse_attention; with ``flat`` the output may come as [1, N_q, H * d]
+    (q, k, v of [1, .., H, d] each and the C++ node: no view between them)."""
     H, d = q.shape[-2], q.shape[-1]
     if num_heads is not None and num_heads != H:
         raise ValueError(f"q has {H} heads, expected {num_heads}")
-    q = _prep(q.reshape(-1, H, d), "q")
-    k = _prep(k.reshape(-1, H, d), "k")
-    v = _prep(v.reshape(-1, H, d), "v")
+    if not (flat and attn_bias is None and _lib.node_ext() is not None
+            and all(t.dim() == 4 and t.shape[0] == 1 and t.shape[2:] == q.shape[2:]
+                    for t in (q, k, v)) and q.shape[1] > 0):
+        q, k, v = q.reshape(-1, H, d), k.reshape(-1, H, d), v.reshape(-1, H, d)
+    q, k, v = _prep(q, "q"), _prep(k, "k"), _prep(v, "v")
     if not (q.dtype == k.dtype == v.dtype):
         raise TypeError("q, k, v must share a dtype")
     _dtype_code(q)
-    if k.shape != v.shape or k.shape[1:] != q.shape[1:]:
+    if k.shape != v.shape or k.shape[-2:] != q.shape[-2:]:
         raise ValueError(f"shape mismatch q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
     k_ext = v_ext = None
-    n_k = k.shape[0]
+    n_q, n_k = q.shape[-3], k.shape[-3]
     if kv_ext is not None:
         k_ext = _prep(kv_ext[0].detach().reshape(-1, H, d), "k_ext")
         v_ext = _prep(kv_ext[1].detach().reshape(-1, H, d), "v_ext")
         if k_ext.shape != v_ext.shape or k_ext.dtype != q.dtype or v_ext.dtype != q.dtype:
             raise ValueError(f"kv_ext must be two [R, {H}, {d}] tensors of dtype {q.dtype}")
         n_k += k_ext.shape[0]
-    if q.shape[0] > n_k:
-        raise ValueError(f"N_q={q.shape[0]} exceeds N_k={n_k}")
+    if n_q > n_k:
+        raise ValueError(f"N_q={n_q} exceeds N_k={n_k}")
     if scale is None:
         scale = math.sqrt(d)
     cache = cache or default_cache
-    adj = cache.get(edge_index, q.shape[0], n_k, chunk_for_heads(H, int(edge_index.shape[-1])),
+    adj = cache.get(edge_index, n_q, n_k, chunk_for_heads(H, int(edge_index.shape[-1])),
                     small_for_heads(H), pack_q_adaptive(H))
     if attn_bias is not None:
         if (attn_bias.dim() != 4 or attn_bias.shape[0] != 1 or attn_bias.shape[1] != H
-                or attn_bias.shape[2] < n_k or attn_bias.shape[3] < q.shape[0]):
-            raise ValueError(f"attn_bias must be [1, {H}, >= {n_k}, >= {q.shape[0]}] "
+                or attn_bias.shape[2] < n_k or attn_bias.shape[3] < n_q):
+            raise ValueError(f"attn_bias must be [1, {H}, >= {n_k}, >= {n_q}] "
                              f"(indexed [0, h, src, dst]), got {tuple(attn_bias.shape)}")
         if not attn_bias.is_cuda:
             raise ValueError("attn_bias must be a GPU tensor")
@@ -677,8 +688,14 @@ class CoreAttention(nn.Module):
             k = torch.cat([k, kv_ext[0].detach().to(k.dtype).reshape(1, -1, *k.shape[2:])], dim=1)
             v = torch.cat([v, kv_ext[1].detach().to(v.dtype).reshape(1, -1, *v.shape[2:])], dim=1)
         if attn_type == "sparse":
-            x, score = self.sparse_attention_bias(q, k, v, edge_index, attn_bias, kv_ext=kv_ext,
-                                                  interleave_grads=interleave_grads)
+            if type(self).sparse_attention_bias is CoreAttention.sparse_attention_bias:
+                x, score = _sparse(q, k, v, edge_index, self.num_heads, self.scale,
+                                   self.adjacency_cache, CLAMP_LO, CLAMP_HI, EPS, kv_ext,
+                                   attn_bias, interleave_grads, True)
+            else:
+                x, score = self.sparse_attention_bias(q, k, v, edge_index, attn_bias,
+                                                      kv_ext=kv_ext,
+                                                      interleave_grads=interleave_grads)
         elif attn_type == "flash":
             # The reference casts q/k/v to fp16 and the result back to fp32
             # (graphormer_dist_node_level.py:111-122).  Here the inputs are
@@ -693,7 +710,8 @@ class CoreAttention(nn.Module):
                 x = x.transpose(1, 2).contiguous()
         else:
             x, score = self.full_attention(k, q, v, attn_bias, mask=mask, pruning_mask=pruning_mask)
-        x = x.view(batch_size, s_len, -1)
+        if x.dim() != 3 or x.shape[:2] != (batch_size, s_len):
+            x = x.view(batch_size, s_len, -1)
         return x, score
 
 

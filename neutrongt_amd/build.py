@@ -100,8 +100,8 @@ def build_library(verbose: bool = False, jobs: int | None = None, out: Path | No
 
 
 def build_autograd_ext(verbose: bool = False) -> Path:
-    """Compiles csrc/ngt_autograd.cpp (host C++: the sparse attention's
-    autograd node, see that file) as a torch extension with g++ and puts
+    """Compiles csrc/ngt_autograd.cpp (host C++: the autograd nodes
+    of the sparse attention and the encoder's layers, see that file) as a torch extension with g++ and puts
     ngt_autograd.so beside the library; returns its path."""
     import torch
     from torch.utils import cpp_extension

@@ -232,7 +232,7 @@ class AdjacencyCache:
 
     def get(self, edge_index: torch.Tensor, n_q: int, n_k: int, chunk: int,
             small: int = 0, pack_q: bool = False) -> WindowAdjacency:
-        shape_key = (tuple(edge_index.shape), str(edge_index.device), edge_index.dtype, n_q, n_k,
+        shape_key = (tuple(edge_index.shape), edge_index.device, edge_index.dtype, n_q, n_k,
                      chunk, small, pack_q)
         same_shape = []
         for eid in reversed(self._d):  # most recent first

@@ -1,6 +1,7 @@
-// C++ autograd node of the sparse window attention.
+// C++ autograd nodes of the sparse window attention and of the encoder around
+// it (linear layers, projection group, LayerNorms).
 //
-// The same operation and contract as SparseAttentionFunction in attention.py
+// Sparse attention: the same operation and contract as SparseAttentionFunction in attention.py
 // (the reference op is CoreAttention.sparse_attention_bias,
 // NeutronGT/models/graphormer_dist_node_level.py:67-98): (q, k, v) ->
 // (out, node_scores), node scores without gradient, optional detached extra
@@ -14,9 +15,26 @@
 // The window is passed as two tensors: `csr` (CPU bytes of one
 // ngt_window_csr) and `csr_mem` (the device allocation its pointers point
 // into).  Both are kept by the node until the backward has run.
+//
+// q, k, v may also come as [1, n, H, d], the layout the encoders hold: the
+// output is then [1, n_q, H * d] and the gradients have the inputs' shape, so
+// that no view node stands between the projections, the core and the output
+// projection.
+//
+// Linear, Projection3, LayerNorm and AddLayerNorm are _WgradLinearFn,
+// _ProjectionGroupFn (of three layers), _LayerNormFn and _AddLayerNormFn of
+// linear.py and layernorm.py: the same casts, library GEMMs and kernels in the
+// same order, bit for bit.  Those Python nodes and the view nodes cost 10-60 us
+// of host time each: forward and backward of the 3-layer GPH_Slim model (254
+// launches, 1.4 ms of kernels) took 4.0 ms and take 2.9, a GPH_Large block
+// over 10,007 queries 1.37 -> 0.97 ms, and the core alone over a small window
+// 113 -> 91 us (74 -> 60 us on a faster host).
 #include <torch/extension.h>
 
 #include <c10/hip/HIPStream.h>
+
+#include <map>
+#include <string>
 
 #include "ngt_attn.h"
 
@@ -29,6 +47,14 @@ using torch::autograd::tensor_list;
 decltype(&ngt_sparse_fwd_ext) g_fwd = nullptr;
 decltype(&ngt_sparse_bwd_strided) g_bwd = nullptr;
 decltype(&ngt_last_error) g_err = nullptr;
+decltype(&ngt_colsum_workspace_bytes) g_colsum_ws = nullptr;
+decltype(&ngt_colsum_bf16) g_colsum = nullptr;
+decltype(&ngt_chunk_sum_f32) g_chunk_sum = nullptr;
+decltype(&ngt_layernorm_fwd) g_ln_fwd = nullptr;
+decltype(&ngt_layernorm_bwd_workspace_bytes) g_ln_bwd_ws = nullptr;
+decltype(&ngt_layernorm_bwd) g_ln_bwd = nullptr;
+decltype(&ngt_add_layernorm_fwd) g_add_ln_fwd = nullptr;
+decltype(&ngt_add_layernorm_bwd) g_add_ln_bwd = nullptr;
 
 void check(int rc) {
   if (rc != NGT_OK) {
@@ -68,8 +94,9 @@ void check_rows(const char* name, const Tensor& t, const Tensor& q) {
   TORCH_CHECK(t.device() == q.device(), name, " is on ", t.device(), ", q on ", q.device());
   TORCH_CHECK(t.scalar_type() == q.scalar_type(), name, " has dtype ", t.scalar_type(),
               ", q has ", q.scalar_type());
-  TORCH_CHECK(t.dim() == 3 && t.size(1) == q.size(1) && t.size(2) == q.size(2), name,
-              " must be [n, ", q.size(1), ", ", q.size(2), "], got ", t.sizes());
+  TORCH_CHECK((t.dim() == 3 || (t.dim() == 4 && t.size(0) == 1)) && t.size(-2) == q.size(-2) &&
+                  t.size(-1) == q.size(-1),
+              name, " must be [n, ", q.size(-2), ", ", q.size(-1), "], got ", t.sizes());
   TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
   TORCH_CHECK(reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, name,
               " must be 16-byte aligned");
@@ -102,15 +129,16 @@ struct SparseAttention : public torch::autograd::Function<SparseAttention> {
       check_rows("v_ext", v_ext, q);
       TORCH_CHECK(k_ext.sizes() == v_ext.sizes(), "k_ext and v_ext differ in shape");
     }
-    const int64_t n_q = q.size(0), H = q.size(1), d = q.size(2);
-    Tensor out = at::empty_like(q);
+    TORCH_CHECK(q.dim() == k.dim(), "q and k differ in dimensions");
+    const int64_t n_q = q.size(-3), n_k = k.size(-3), H = q.size(-2), d = q.size(-1);
+    Tensor out = q.dim() == 4 ? at::empty({1, n_q, H * d}, q.options()) : at::empty_like(q);
     const auto f32 = q.options().dtype(at::kFloat);
     Tensor rinv = at::empty({n_q, H}, f32);
     Tensor ns = at::empty({dst_end}, f32);
     Tensor ws = workspace(fwd_bytes, q);
     check(g_fwd(dtype_code(q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                 ext ? k_ext.data_ptr() : nullptr, ext ? v_ext.data_ptr() : nullptr,
-                static_cast<int32_t>(k.size(0)), csr_of(csr), static_cast<int32_t>(H),
+                static_cast<int32_t>(n_k), csr_of(csr), static_cast<int32_t>(H),
                 static_cast<int32_t>(d), static_cast<float>(scale), static_cast<float>(lo),
                 static_cast<float>(hi), static_cast<float>(eps), out.data_ptr(),
                 rinv.data_ptr<float>(), dst_end ? ns.data_ptr<float>() : nullptr,
@@ -125,7 +153,7 @@ struct SparseAttention : public torch::autograd::Function<SparseAttention> {
     ctx->saved_data["lo"] = lo;
     ctx->saved_data["hi"] = hi;
     ctx->saved_data["bwd_bytes"] = bwd_bytes;
-    ctx->saved_data["interleave"] = interleave_grads && n_q == k.size(0);
+    ctx->saved_data["interleave"] = interleave_grads && n_q == n_k;
     ctx->mark_non_differentiable({ns});
     // the node scores have no gradient: no zero tensor is made for them
     ctx->set_materialize_grads(false);
@@ -142,15 +170,18 @@ struct SparseAttention : public torch::autograd::Function<SparseAttention> {
     const Tensor csr = ctx->saved_data["csr"].toTensor();
     const int64_t bwd_bytes = ctx->saved_data["bwd_bytes"].toInt();
     const Tensor g = rows16(grads[0].to(q.scalar_type()));
+    const int64_t n_q = q.size(-3), n_k = k.size(-3), H = q.size(-2), d = q.size(-1);
     Tensor gq, gk, gv;
     int64_t ldg = 0;
     if (ctx->saved_data["interleave"].toBool()) {
       // one [N, 3, H, d] buffer: row i holds dQ, dK, dV of row i side by side
-      const Tensor buf = at::empty({q.size(0), 3, q.size(1), q.size(2)}, q.options());
-      gq = buf.select(1, 0);
-      gk = buf.select(1, 1);
-      gv = buf.select(1, 2);
-      ldg = 3 * q.size(1) * q.size(2);
+      const Tensor buf = at::empty({n_q, 3, H, d}, q.options());
+      ldg = 3 * H * d;
+      const auto rows = q.dim() == 4 ? std::vector<int64_t>{n_q * ldg, ldg, d, 1}
+                                     : std::vector<int64_t>{ldg, d, 1};
+      gq = buf.as_strided(q.sizes(), rows, 0);
+      gk = buf.as_strided(q.sizes(), rows, H * d);
+      gv = buf.as_strided(q.sizes(), rows, 2 * H * d);
     } else {
       gq = at::empty_like(q);
       gk = at::empty_like(k);
@@ -160,9 +191,9 @@ struct SparseAttention : public torch::autograd::Function<SparseAttention> {
     const bool ext = k_ext.defined();
     check(g_bwd(dtype_code(q), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                 ext ? k_ext.data_ptr() : nullptr, ext ? v_ext.data_ptr() : nullptr,
-                static_cast<int32_t>(k.size(0)), out.data_ptr(), g.data_ptr(),
-                rinv.data_ptr<float>(), csr_of(csr), static_cast<int32_t>(q.size(1)),
-                static_cast<int32_t>(q.size(2)),
+                static_cast<int32_t>(n_k), out.data_ptr(), g.data_ptr(),
+                rinv.data_ptr<float>(), csr_of(csr), static_cast<int32_t>(H),
+                static_cast<int32_t>(d),
                 static_cast<float>(ctx->saved_data["scale"].toDouble()),
                 static_cast<float>(ctx->saved_data["lo"].toDouble()),
                 static_cast<float>(ctx->saved_data["hi"].toDouble()), gq.data_ptr(),
@@ -189,16 +220,354 @@ std::tuple<Tensor, Tensor> sparse_attention(Tensor q, Tensor k, Tensor v,
   return {r[0], r[1]};
 }
 
-void init(int64_t fwd, int64_t bwd, int64_t err) {
-  g_fwd = reinterpret_cast<decltype(&ngt_sparse_fwd_ext)>(fwd);
-  g_bwd = reinterpret_cast<decltype(&ngt_sparse_bwd_strided)>(bwd);
-  g_err = reinterpret_cast<decltype(&ngt_last_error)>(err);
+// ------------------------------------------------------- the encoder's layers
+// torch's casts of the operands stay off inside these nodes: their GEMMs take
+// the operands as they are
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
+};
+
+constexpr int64_t kChunk = 2048;  // as _CHUNK and _MAX_SPLITS of linear.py
+constexpr int64_t kMaxSplits = 16;
+
+// fp32 column sums of a contiguous bf16 [K, n] matrix
+Tensor colsum(const Tensor& dy) {
+  const int64_t K = dy.size(0);
+  const auto n = static_cast<int32_t>(dy.size(1));
+  Tensor out = at::empty({n}, dy.options().dtype(at::kFloat));
+  size_t bytes = 0;
+  check(g_colsum_ws(K, n, &bytes));
+  Tensor ws = workspace(static_cast<int64_t>(bytes), dy);
+  check(g_colsum(dy.data_ptr(), K, n, out.data_ptr<float>(), ws.data_ptr(), bytes, stream_of(dy)));
+  return out;
+}
+
+// dY^T X in fp32, split over rows (weight_grad of linear.py)
+Tensor weight_grad(const Tensor& x, const Tensor& dy) {
+  const int64_t K = x.size(0), n_in = x.size(1), n_out = dy.size(1);
+  const int64_t most = n_out * n_in < 1500000 ? kMaxSplits : kMaxSplits / 2;
+  const int64_t splits = std::max<int64_t>(1, std::min(most, K / kChunk));
+  const int64_t c = K / splits, main = splits * c;
+  if (splits == 1) return at::mm(dy.t(), x, at::kFloat);
+  Tensor parts = at::bmm(dy.narrow(0, 0, main).view({splits, c, n_out}).transpose(1, 2),
+                         x.narrow(0, 0, main).view({splits, c, n_in}), at::kFloat)
+                     .contiguous();
+  Tensor dw = at::empty({n_out, n_in}, parts.options());
+  check(g_chunk_sum(parts.data_ptr<float>(), static_cast<int32_t>(splits), n_out * n_in,
+                    dw.data_ptr<float>(), stream_of(x)));
+  if (main < K) dw.add_(at::mm(dy.narrow(0, main, K - main).t(), x.narrow(0, main, K - main),
+                               at::kFloat));
+  return dw;
+}
+
+Tensor bf16(const Tensor& t) { return t.to(at::kBFloat16); }
+
+std::optional<Tensor> bf16(const std::optional<Tensor>& t) {
+  return t.has_value() ? std::optional<Tensor>(bf16(*t)) : std::nullopt;
+}
+
+// y = x W^T + b in bf16; fp32 dW and db
+struct Linear : public torch::autograd::Function<Linear> {
+  static Tensor forward(AutogradContext* ctx, Tensor x, Tensor weight,
+                        std::optional<Tensor> bias) {
+    NoAutocast off;
+    const Tensor x16 = bf16(x), w16 = bf16(weight);
+    Tensor y = at::linear(x16, w16, bf16(bias));
+    ctx->save_for_backward({x16, w16});
+    ctx->saved_data["bias"] = bias.has_value();
+    return y;
+  }
+
+  static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+    NoAutocast off;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x16 = saved[0], &w16 = saved[1];
+    const int64_t n_out = w16.size(0), n_in = w16.size(1);
+    tensor_list res(3);
+    const Tensor g2 = bf16(grads[0]).reshape({-1, n_out}).contiguous();
+    if (ctx->needs_input_grad(0)) res[0] = at::mm(g2, w16).view(x16.sizes());
+    if (ctx->needs_input_grad(1)) res[1] = weight_grad(x16.reshape({-1, n_in}).contiguous(), g2);
+    if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) res[2] = colsum(g2);
+    return res;
+  }
+};
+
+Tensor linear(Tensor x, Tensor weight, std::optional<Tensor> bias) {
+  return Linear::apply(x, weight, bias);
+}
+
+// the [M, 3 * n_out] matrix whose column blocks are the gradients g, when they
+// are views of one buffer laid out that way; else undefined
+Tensor joint_rows(const tensor_list& g, int64_t n_out) {
+  const Tensor& g0 = g[0];
+  if (!g0.defined() || g0.scalar_type() != at::kBFloat16) return Tensor();
+  const int64_t width = n_out * static_cast<int64_t>(g.size());
+  const int64_t m = g0.numel() / n_out;
+  for (size_t i = 0; i < g.size(); ++i) {
+    const Tensor& t = g[i];
+    if (!t.defined() || t.scalar_type() != at::kBFloat16 || t.sizes() != g0.sizes() ||
+        !t.storage().is_alias_of(g0.storage()) ||
+        t.storage_offset() != g0.storage_offset() + static_cast<int64_t>(i) * n_out)
+      return Tensor();
+    // rows of n_out adjacent elements, width apart: from the last dimension
+    // up, strides run over a row and then over the rows
+    int64_t inner = 1, outer = 1;
+    for (int64_t a = t.dim() - 1; a >= 0; --a) {
+      const int64_t len = t.size(a);
+      if (len == 1) continue;
+      if (inner < n_out) {
+        if (t.stride(a) != inner) return Tensor();
+        inner *= len;
+        if (inner > n_out) return Tensor();
+      } else {
+        if (t.stride(a) != outer * width) return Tensor();
+        outer *= len;
+      }
+    }
+    if (inner != n_out || outer != m) return Tensor();
+  }
+  const int64_t end = (g0.storage_offset() + m * width) * static_cast<int64_t>(g0.element_size());
+  if (m == 0 || end > static_cast<int64_t>(g0.storage().nbytes())) return Tensor();
+  return g0.as_strided({m, width}, {width, 1});
+}
+
+// Three projections of one input (Q, K, V) as one node.  heads > 0: the
+// outputs as [..., heads, n_out / heads].
+struct Projection3 : public torch::autograd::Function<Projection3> {
+  static tensor_list forward(AutogradContext* ctx, Tensor x, Tensor w0, std::optional<Tensor> b0,
+                             Tensor w1, std::optional<Tensor> b1, Tensor w2,
+                             std::optional<Tensor> b2, int64_t heads) {
+    NoAutocast off;
+    const Tensor x16 = bf16(x);
+    const Tensor w[3] = {bf16(w0), bf16(w1), bf16(w2)};
+    const std::optional<Tensor> b[3] = {b0, b1, b2};
+    tensor_list ys;
+    int64_t has_bias = 0;
+    for (int i = 0; i < 3; ++i) {
+      Tensor y = at::linear(x16, w[i], bf16(b[i]));
+      if (heads > 0) {
+        auto shape = y.sizes().vec();
+        shape.back() /= heads;
+        shape.insert(shape.end() - 1, heads);
+        y = y.view(shape);
+      }
+      ys.push_back(y);
+      has_bias |= int64_t(b[i].has_value()) << i;
+    }
+    ctx->save_for_backward({x16, w[0], w[1], w[2]});
+    ctx->saved_data["bias"] = has_bias;
+    ctx->set_materialize_grads(false);  // an unused output: no GEMMs, no weight gradient
+    return ys;
+  }
+
+  static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+    NoAutocast off;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor& x16 = saved[0];
+    const tensor_list w(saved.begin() + 1, saved.end());
+    const int64_t has_bias = ctx->saved_data["bias"].toInt();
+    const int64_t n_in = x16.size(-1), n_out = w[0].size(0);
+    // the node's edges are numbered over the tensors that were given
+    bool want_w[3], want_b[3];
+    size_t edge = 1;
+    for (int i = 0; i < 3; ++i) {
+      want_w[i] = ctx->needs_input_grad(edge++);
+      want_b[i] = (has_bias >> i & 1) && ctx->needs_input_grad(edge++);
+    }
+    tensor_list res(8);
+    Tensor joint;
+    if (w[1].size(0) == n_out && w[2].size(0) == n_out && want_w[0] && want_w[1] && want_w[2] &&
+        ((want_b[0] && want_b[1] && want_b[2]) || has_bias == 0))
+      joint = joint_rows(grads, n_out);
+    if (joint.defined()) {
+      if (ctx->needs_input_grad(0)) res[0] = at::mm(joint, at::cat(w, 0)).view(x16.sizes());
+      const Tensor dw = weight_grad(x16.reshape({-1, n_in}).contiguous(), joint);
+      const Tensor db = has_bias ? colsum(joint) : Tensor();
+      for (int i = 0; i < 3; ++i) {
+        res[1 + 2 * i] = dw.narrow(0, i * n_out, n_out);
+        if (has_bias) res[2 + 2 * i] = db.narrow(0, i * n_out, n_out);
+      }
+      return res;
+    }
+    Tensor x2, gx;
+    for (int i = 0; i < 3; ++i) {
+      if (!grads[i].defined()) continue;
+      const Tensor g2 = bf16(grads[i]).reshape({-1, w[i].size(0)}).contiguous();
+      if (ctx->needs_input_grad(0)) {
+        if (gx.defined())
+          gx.addmm_(g2, w[i]);
+        else
+          gx = at::mm(g2, w[i]);
+      }
+      if (want_w[i]) {
+        if (!x2.defined()) x2 = x16.reshape({-1, n_in}).contiguous();
+        res[1 + 2 * i] = weight_grad(x2, g2);
+      }
+      if (want_b[i]) res[2 + 2 * i] = colsum(g2);
+    }
+    if (gx.defined()) res[0] = gx.view(x16.sizes());
+    return res;
+  }
+};
+
+tensor_list project3(Tensor x, Tensor w0, std::optional<Tensor> b0, Tensor w1,
+                     std::optional<Tensor> b1, Tensor w2, std::optional<Tensor> b2,
+                     int64_t heads) {
+  return Projection3::apply(x, w0, b0, w1, b1, w2, b2, heads);
+}
+
+// [n, n_cols] contiguous rows whose base meets the LayerNorm kernels'
+// alignment: 16 bytes for fp32, 8 for bf16
+Tensor ln_rows(const Tensor& t, int64_t n_cols) {
+  const Tensor r = t.reshape({-1, n_cols});
+  const uintptr_t align = r.scalar_type() == at::kFloat ? 16 : 8;
+  if (!r.is_contiguous() || reinterpret_cast<uintptr_t>(r.data_ptr()) % align)
+    return r.clone(at::MemoryFormat::Contiguous);
+  return r;
+}
+
+Tensor ln_grad(const Tensor& g) {
+  return g.scalar_type() == at::kFloat || g.scalar_type() == at::kBFloat16 ? g : g.to(at::kFloat);
+}
+
+Tensor f32(const Tensor& t) { return t.to(at::kFloat).contiguous(); }
+
+struct LayerNorm : public torch::autograd::Function<LayerNorm> {
+  static Tensor forward(AutogradContext* ctx, Tensor x, Tensor weight, Tensor bias, double eps,
+                        bool out_bf16) {
+    NoAutocast off;
+    const int64_t n_cols = weight.numel();
+    const Tensor x2 = ln_rows(x, n_cols), w = f32(weight), b = f32(bias);
+    const int64_t n = x2.size(0);
+    const auto opt = x.options().dtype(at::kFloat);
+    Tensor y = at::empty(x.sizes(), out_bf16 ? x.options().dtype(at::kBFloat16) : opt,
+                         at::MemoryFormat::Contiguous);
+    Tensor mean = at::empty({n}, opt), rstd = at::empty({n}, opt);
+    check(g_ln_fwd(dtype_code(x2), x2.data_ptr(), n, static_cast<int32_t>(n_cols),
+                   w.data_ptr<float>(), b.data_ptr<float>(), static_cast<float>(eps),
+                   dtype_code(y), y.data_ptr(), mean.data_ptr<float>(), rstd.data_ptr<float>(),
+                   stream_of(x)));
+    ctx->save_for_backward({x2, w, mean, rstd});
+    ctx->saved_data["shape"] = x.sizes().vec();
+    return y;
+  }
+
+  static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+    NoAutocast off;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x2 = saved[0], &w = saved[1], &mean = saved[2], &rstd = saved[3];
+    const int64_t n = x2.size(0), n_cols = x2.size(1);
+    const Tensor g2 = ln_rows(ln_grad(grads[0]), n_cols);
+    Tensor dx = at::empty_like(x2);
+    Tensor dw = at::empty({n_cols}, w.options()), db = at::empty({n_cols}, w.options());
+    size_t bytes = 0;
+    check(g_ln_bwd_ws(n, static_cast<int32_t>(n_cols), &bytes));
+    Tensor ws = workspace(static_cast<int64_t>(bytes), x2);
+    check(g_ln_bwd(dtype_code(x2), x2.data_ptr(), dtype_code(g2), g2.data_ptr(), n,
+                   static_cast<int32_t>(n_cols), w.data_ptr<float>(), mean.data_ptr<float>(),
+                   rstd.data_ptr<float>(), dx.data_ptr(), dw.data_ptr<float>(),
+                   db.data_ptr<float>(), ws.data_ptr(), bytes, stream_of(x2)));
+    return {dx.view(ctx->saved_data["shape"].toIntVector()), dw, db, Tensor(), Tensor()};
+  }
+};
+
+Tensor layernorm(Tensor x, Tensor weight, Tensor bias, double eps, bool out_bf16) {
+  return LayerNorm::apply(x, weight, bias, eps, out_bf16);
+}
+
+// (s, LayerNorm(s)) with s = x + dropout(y)
+struct AddLayerNorm : public torch::autograd::Function<AddLayerNorm> {
+  static tensor_list forward(AutogradContext* ctx, Tensor x, Tensor y, Tensor weight, Tensor bias,
+                             double eps, double p, std::optional<Tensor> seed_opt, bool out_bf16) {
+    NoAutocast off;
+    const int64_t n_cols = weight.numel();
+    const Tensor x2 = ln_rows(x, n_cols), y2 = ln_rows(y, n_cols), w = f32(weight), b = f32(bias);
+    TORCH_CHECK(y2.scalar_type() == x2.scalar_type() && y2.sizes() == x2.sizes(),
+                "x and y differ in dtype or shape");
+    const Tensor seed = seed_opt.value_or(Tensor());
+    const int64_t n = x2.size(0);
+    const auto opt = x.options().dtype(at::kFloat);
+    Tensor s = at::empty(x.sizes(), x.options(), at::MemoryFormat::Contiguous);
+    Tensor out = at::empty(x.sizes(), out_bf16 ? x.options().dtype(at::kBFloat16) : opt,
+                           at::MemoryFormat::Contiguous);
+    Tensor mean = at::empty({n}, opt), rstd = at::empty({n}, opt);
+    check(g_add_ln_fwd(dtype_code(x2), x2.data_ptr(), y2.data_ptr(), n,
+                       static_cast<int32_t>(n_cols), static_cast<float>(p), 0, seed_ptr(seed),
+                       w.data_ptr<float>(), b.data_ptr<float>(), static_cast<float>(eps),
+                       s.data_ptr(), dtype_code(out), out.data_ptr(), mean.data_ptr<float>(),
+                       rstd.data_ptr<float>(), stream_of(x)));
+    ctx->save_for_backward({s, w, mean, rstd, seed});
+    ctx->saved_data["p"] = p;
+    ctx->set_materialize_grads(false);  // an unused sum: no zero tensor for its gradient
+    return {s, out};
+  }
+
+  static tensor_list backward(AutogradContext* ctx, tensor_list grads) {
+    NoAutocast off;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &s = saved[0], &w = saved[1], &mean = saved[2], &rstd = saved[3];
+    const int64_t n = mean.numel(), n_cols = w.numel();
+    tensor_list res(8);
+    if (!grads[0].defined() && !grads[1].defined()) return res;
+    const Tensor g_out =
+        grads[1].defined() ? ln_rows(ln_grad(grads[1]), n_cols) : at::zeros({n, n_cols}, w.options());
+    const Tensor g_s =
+        grads[0].defined() ? ln_rows(grads[0].to(s.scalar_type()), n_cols) : Tensor();
+    Tensor dx = at::empty_like(s), dy = at::empty_like(s);
+    Tensor dw = at::empty({n_cols}, w.options()), db = at::empty({n_cols}, w.options());
+    size_t bytes = 0;
+    check(g_ln_bwd_ws(n, static_cast<int32_t>(n_cols), &bytes));
+    Tensor ws = workspace(static_cast<int64_t>(bytes), s);
+    check(g_add_ln_bwd(dtype_code(s), s.data_ptr(), dtype_code(g_out), g_out.data_ptr(),
+                       g_s.defined() ? g_s.data_ptr() : nullptr, n, static_cast<int32_t>(n_cols),
+                       static_cast<float>(ctx->saved_data["p"].toDouble()), 0, seed_ptr(saved[4]),
+                       w.data_ptr<float>(), mean.data_ptr<float>(), rstd.data_ptr<float>(),
+                       dx.data_ptr(), dy.data_ptr(), dw.data_ptr<float>(), db.data_ptr<float>(),
+                       ws.data_ptr(), bytes, stream_of(s)));
+    res[0] = dx;
+    res[1] = dy;
+    res[2] = dw;
+    res[3] = db;
+    return res;
+  }
+
+ private:
+  static const uint64_t* seed_ptr(const Tensor& seed) {
+    return seed.defined() ? static_cast<const uint64_t*>(seed.data_ptr()) : nullptr;
+  }
+};
+
+std::tuple<Tensor, Tensor> add_layernorm(Tensor x, Tensor y, Tensor weight, Tensor bias, double eps,
+                                         double p, std::optional<Tensor> seed, bool out_bf16) {
+  auto r = AddLayerNorm::apply(x, y, weight, bias, eps, p, seed, out_bf16);
+  return {r[0], r[1]};
+}
+
+template <typename F>
+void entry(F*& fn, const std::map<std::string, int64_t>& addr, const char* name) {
+  const auto it = addr.find(name);
+  TORCH_CHECK(it != addr.end() && it->second, "ngt_autograd.init: no address of ", name);
+  fn = reinterpret_cast<F*>(it->second);
+}
+
+void init(const std::map<std::string, int64_t>& addr) {
+  entry(g_fwd, addr, "ngt_sparse_fwd_ext");
+  entry(g_bwd, addr, "ngt_sparse_bwd_strided");
+  entry(g_err, addr, "ngt_last_error");
+  entry(g_colsum_ws, addr, "ngt_colsum_workspace_bytes");
+  entry(g_colsum, addr, "ngt_colsum_bf16");
+  entry(g_chunk_sum, addr, "ngt_chunk_sum_f32");
+  entry(g_ln_fwd, addr, "ngt_layernorm_fwd");
+  entry(g_ln_bwd_ws, addr, "ngt_layernorm_bwd_workspace_bytes");
+  entry(g_ln_bwd, addr, "ngt_layernorm_bwd");
+  entry(g_add_ln_fwd, addr, "ngt_add_layernorm_fwd");
+  entry(g_add_ln_bwd, addr, "ngt_add_layernorm_bwd");
 }
 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("init", &init, "entry points of libngt_attn.so: fwd, bwd, last_error (addresses)");
+  m.def("init", &init, "{name: address} of libngt_attn.so's entry points");
   m.def("csr_struct_bytes", []() { return static_cast<int64_t>(sizeof(ngt_window_csr)); });
   m.def("abi_version", []() { return static_cast<int64_t>(NGT_ABI_VERSION); },
         "NGT_ABI_VERSION of the header this extension was compiled against");
@@ -206,4 +575,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "(q, k, v, k_ext, v_ext, csr, csr_mem, dst_end, scale, lo, hi, eps, fwd_bytes, "
         "bwd_bytes, interleave_grads) -> (out, node_scores); interleave_grads: dQ, dK, dV as "
         "views of one [N, 3, H, d] buffer (when q and k have the same rows)");
+  m.def("linear", &linear, "(x, weight, bias) -> y: linear.py's _WgradLinearFn");
+  m.def("project3", &project3,
+        "(x, w0, b0, w1, b1, w2, b2, heads) -> [y0, y1, y2]: linear.py's _ProjectionGroupFn; "
+        "heads > 0: outputs [..., heads, n_out / heads]");
+  m.def("layernorm", &layernorm, "(x, weight, bias, eps, out_bf16) -> y: layernorm.py's _LayerNormFn");
+  m.def("add_layernorm", &add_layernorm,
+        "(x, y, weight, bias, eps, p, seed tensor or None, out_bf16) -> (s, out): layernorm.py's "
+        "_AddLayerNormFn");
 }

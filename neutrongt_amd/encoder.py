@@ -91,7 +91,6 @@ class _Attention(nn.Module):
         self.local_attn = CoreAttention(hidden_size, attention_dropout_rate, num_heads)
 
     def attend(self, x, edge_index, attn_type, kv_cache):
-        b, n, _ = x.shape
         H, d = self.num_heads, self.att_size
         lins = (self.linear_q, self.linear_k, self.linear_v)
         # one projection node, and the sparse core hands back dQ, dK, dV as
@@ -99,8 +98,7 @@ class _Attention(nn.Module):
         interleave = (groupable(x, *lins) and attn_type == "sparse"
                       and isinstance(self.local_attn, CoreAttention))
         extra = {"interleave_grads": True} if interleave else {}
-        q, k, v = project(x, *lins)
-        q, k, v = q.view(b, n, H, d), k.view(b, n, H, d), v.view(b, n, H, d)
+        q, k, v = project(x, *lins, heads=H)  # [b, n, H, d] each
         if kv_cache is None:
             y, score = self.local_attn(q, k, v, None, edge_index, attn_type, **extra)
             return y, score, [k, v]

@@ -97,6 +97,9 @@ class FusedLayerNorm(nn.LayerNorm):
                 and torch.is_autocast_enabled("cuda")
                 and torch.get_autocast_dtype("cuda") == torch.bfloat16
                 and n_cols % 4 == 0 and 4 <= n_cols <= 2048):
+            ext = _lib.node_ext()
+            if ext is not None:
+                return ext.layernorm(x, self.weight, self.bias, self.eps, self.out_bf16)
             return _LayerNormFn.apply(x, self.weight, self.bias, self.eps, self.out_bf16)
         return super().forward(x)
 
@@ -176,6 +179,9 @@ def add_dropout_layernorm(x: torch.Tensor, y: torch.Tensor, ln: nn.LayerNorm,
     if (_fused_ok(x, ln) and y.dtype == x.dtype and y.shape == x.shape and p < 1.0
             and torch.is_grad_enabled()):
         seed_t = draw_seed(x.device) if p > 0 else None
+        ext = _lib.node_ext()
+        if ext is not None:
+            return ext.add_layernorm(x, y, ln.weight, ln.bias, ln.eps, p, seed_t, ln.out_bf16)
         return _AddLayerNormFn.apply(x, y, ln.weight, ln.bias, ln.eps, p, 0, ln.out_bf16, seed_t)
     s = x + F.dropout(y, p, dropout.training) if p > 0 else x + y
     return s, ln(s)

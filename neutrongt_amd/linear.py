@@ -228,17 +228,26 @@ def groupable(x: torch.Tensor, *lins: nn.Linear) -> bool:
     return len(lins) > 1 and all(isinstance(l, WgradLinear) and _fast_path(l, x) for l in lins)
 
 
-def project(x: torch.Tensor, *lins: nn.Linear):
-    """(lin(x) for lin in lins), with the backward's dX summed inside the
+def project(x: torch.Tensor, *lins: nn.Linear, heads: int = 0):
+    """(lin(x) for lin in lins), viewed as [..., heads, n_out / heads] when
+    ``heads`` is given, with the backward's dX summed inside the
     GEMMs (and, for gradients that arrive as column blocks of one matrix, dW
     and db as one GEMM and one column sum) when all of them take the bf16
-    autocast path; otherwise each module's own forward."""
+    autocast path; otherwise each module's own forward.  Three layers (Q, K,
+    V) run as one C++ node where ngt_autograd.so is built."""
     if groupable(x, *lins):
+        ext = _lib.node_ext() if len(lins) == 3 else None
+        if ext is not None:
+            a, b, c = lins
+            return tuple(ext.project3(x, a.weight, a.bias, b.weight, b.bias, c.weight, c.bias,
+                                      heads))
         params = []
         for l in lins:
             params += [l.weight, l.bias]
-        return _ProjectionGroupFn.apply(x, *params)
-    return tuple(l(x) for l in lins)
+        ys = _ProjectionGroupFn.apply(x, *params)
+    else:
+        ys = tuple(l(x) for l in lins)
+    return tuple(y.view(*y.shape[:-1], heads, -1) for y in ys) if heads else ys
 
 
 class WgradLinear(nn.Linear):
@@ -247,5 +256,8 @@ class WgradLinear(nn.Linear):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if _fast_path(self, x):
+            ext = _lib.node_ext()
+            if ext is not None:
+                return ext.linear(x, self.weight, self.bias)
             return _WgradLinearFn.apply(x, self.weight, self.bias)
         return super().forward(x)
