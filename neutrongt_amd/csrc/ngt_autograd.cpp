@@ -297,38 +297,16 @@ Tensor linear(Tensor x, Tensor weight, std::optional<Tensor> bias) {
 }
 
 // the [M, 3 * n_out] matrix whose column blocks are the gradients g, when they
-// are views of one buffer laid out that way; else undefined
+// are views of one buffer laid out that way (linear.py's _joint_rows, the one
+// place that knows the layout); else undefined
 Tensor joint_rows(const tensor_list& g, int64_t n_out) {
-  const Tensor& g0 = g[0];
-  if (!g0.defined() || g0.scalar_type() != at::kBFloat16) return Tensor();
-  const int64_t width = n_out * static_cast<int64_t>(g.size());
-  const int64_t m = g0.numel() / n_out;
-  for (size_t i = 0; i < g.size(); ++i) {
-    const Tensor& t = g[i];
-    if (!t.defined() || t.scalar_type() != at::kBFloat16 || t.sizes() != g0.sizes() ||
-        !t.storage().is_alias_of(g0.storage()) ||
-        t.storage_offset() != g0.storage_offset() + static_cast<int64_t>(i) * n_out)
-      return Tensor();
-    // rows of n_out adjacent elements, width apart: from the last dimension
-    // up, strides run over a row and then over the rows
-    int64_t inner = 1, outer = 1;
-    for (int64_t a = t.dim() - 1; a >= 0; --a) {
-      const int64_t len = t.size(a);
-      if (len == 1) continue;
-      if (inner < n_out) {
-        if (t.stride(a) != inner) return Tensor();
-        inner *= len;
-        if (inner > n_out) return Tensor();
-      } else {
-        if (t.stride(a) != outer * width) return Tensor();
-        outer *= len;
-      }
-    }
-    if (inner != n_out || outer != m) return Tensor();
-  }
-  const int64_t end = (g0.storage_offset() + m * width) * static_cast<int64_t>(g0.element_size());
-  if (m == 0 || end > static_cast<int64_t>(g0.storage().nbytes())) return Tensor();
-  return g0.as_strided({m, width}, {width, 1});
+  pybind11::gil_scoped_acquire gil;
+  pybind11::tuple views(g.size());
+  for (size_t i = 0; i < g.size(); ++i)
+    views[i] = g[i].defined() ? pybind11::cast(g[i]) : pybind11::none();
+  const pybind11::object r =
+      pybind11::module_::import("neutrongt_amd.linear").attr("_joint_rows")(views, n_out);
+  return r.is_none() ? Tensor() : r.cast<Tensor>();
 }
 
 // Three projections of one input (Q, K, V) as one node.  heads > 0: the
