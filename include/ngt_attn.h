@@ -663,6 +663,18 @@ int ngt_colsum_bf16(const void* dy, int64_t n_rows, int32_t n_cols, float* out, 
  */
 int ngt_chunk_sum_f32(const float* in, int32_t n_chunks, int64_t n, float* out, void* stream);
 
+/*
+ * Weight and bias gradient of a bf16 linear layer: dw[o][i] = sum_k dy[k][o]
+ * x[k][i] and db[o] = sum_k dy[k][o], both fp32, from x [n_rows, n_in] and dy
+ * [n_rows, n_out] (bf16, row-major, any widths and 2-byte alignment).  db may
+ * be null.  The sums are in a fixed order.  workspace: 16-byte
+ * aligned, ngt_wgrad_workspace_bytes.  The autograd of nn.Linear's weight and
+ * bias, NeutronGT/models/graphormer_dist_node_level.py:130-206.
+ */
+int ngt_wgrad_workspace_bytes(int64_t n_rows, int32_t n_out, int32_t n_in, size_t* bytes);
+int ngt_wgrad_bf16(const void* x, const void* dy, int64_t n_rows, int32_t n_out, int32_t n_in,
+                   float* dw, float* db, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

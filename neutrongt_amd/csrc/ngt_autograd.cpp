@@ -50,6 +50,8 @@ decltype(&ngt_last_error) g_err = nullptr;
 decltype(&ngt_colsum_workspace_bytes) g_colsum_ws = nullptr;
 decltype(&ngt_colsum_bf16) g_colsum = nullptr;
 decltype(&ngt_chunk_sum_f32) g_chunk_sum = nullptr;
+decltype(&ngt_wgrad_workspace_bytes) g_wgrad_ws = nullptr;
+decltype(&ngt_wgrad_bf16) g_wgrad = nullptr;
 decltype(&ngt_layernorm_fwd) g_ln_fwd = nullptr;
 decltype(&ngt_layernorm_bwd_workspace_bytes) g_ln_bwd_ws = nullptr;
 decltype(&ngt_layernorm_bwd) g_ln_bwd = nullptr;
@@ -227,8 +229,9 @@ struct NoAutocast {
   c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
 };
 
-constexpr int64_t kChunk = 2048;  // as _CHUNK and _MAX_SPLITS of linear.py
+constexpr int64_t kChunk = 2048;  // as the limits of linear.py
 constexpr int64_t kMaxSplits = 16;
+constexpr int64_t kFusedProducts = 18000000000, kFusedRows = 3000, kFusedOutputs = 1000000;
 
 // fp32 column sums of a contiguous bf16 [K, n] matrix
 Tensor colsum(const Tensor& dy) {
@@ -242,8 +245,9 @@ Tensor colsum(const Tensor& dy) {
   return out;
 }
 
-// dY^T X in fp32, split over rows (weight_grad of linear.py)
-Tensor weight_grad(const Tensor& x, const Tensor& dy) {
+// dY^T X in fp32 by library GEMMs split over rows (_library_weight_grad of
+// linear.py)
+Tensor library_weight_grad(const Tensor& x, const Tensor& dy) {
   const int64_t K = x.size(0), n_in = x.size(1), n_out = dy.size(1);
   const int64_t most = n_out * n_in < 1500000 ? kMaxSplits : kMaxSplits / 2;
   const int64_t splits = std::max<int64_t>(1, std::min(most, K / kChunk));
@@ -258,6 +262,27 @@ Tensor weight_grad(const Tensor& x, const Tensor& dy) {
   if (main < K) dw.add_(at::mm(dy.narrow(0, main, K - main).t(), x.narrow(0, main, K - main),
                                at::kFloat));
   return dw;
+}
+
+// dw = dY^T X and, where wanted, db = column sums of dY, in fp32 from
+// contiguous bf16 rows (_grads of linear.py; its _fused explains the rule)
+void linear_grads(const Tensor& x, const Tensor& dy, Tensor* dw, Tensor* db) {
+  const int64_t K = x.size(0), n_in = x.size(1), n_out = dy.size(1);
+  if (!dw || at::GradMode::is_enabled() || n_in == 0 || n_out == 0 ||
+      K * n_in * n_out > kFusedProducts || (K < kFusedRows && n_in * n_out >= kFusedOutputs)) {
+    if (dw) *dw = library_weight_grad(x, dy);
+    if (db) *db = colsum(dy);
+    return;
+  }
+  const auto opt = x.options().dtype(at::kFloat);
+  *dw = at::empty({n_out, n_in}, opt);
+  if (db) *db = at::empty({n_out}, opt);
+  size_t bytes = 0;
+  check(g_wgrad_ws(K, static_cast<int32_t>(n_out), static_cast<int32_t>(n_in), &bytes));
+  Tensor ws = workspace(static_cast<int64_t>(bytes), x);
+  check(g_wgrad(x.data_ptr(), dy.data_ptr(), K, static_cast<int32_t>(n_out),
+                static_cast<int32_t>(n_in), dw->data_ptr<float>(),
+                db ? db->data_ptr<float>() : nullptr, ws.data_ptr(), bytes, stream_of(x)));
 }
 
 Tensor bf16(const Tensor& t) { return t.to(at::kBFloat16); }
@@ -286,8 +311,9 @@ struct Linear : public torch::autograd::Function<Linear> {
     tensor_list res(3);
     const Tensor g2 = bf16(grads[0]).reshape({-1, n_out}).contiguous();
     if (ctx->needs_input_grad(0)) res[0] = at::mm(g2, w16).view(x16.sizes());
-    if (ctx->needs_input_grad(1)) res[1] = weight_grad(x16.reshape({-1, n_in}).contiguous(), g2);
-    if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) res[2] = colsum(g2);
+    const bool want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
+    linear_grads(x16.reshape({-1, n_in}).contiguous(), g2,
+                 ctx->needs_input_grad(1) ? &res[1] : nullptr, want_b ? &res[2] : nullptr);
     return res;
   }
 };
@@ -359,8 +385,8 @@ struct Projection3 : public torch::autograd::Function<Projection3> {
       joint = joint_rows(grads, n_out);
     if (joint.defined()) {
       if (ctx->needs_input_grad(0)) res[0] = at::mm(joint, at::cat(w, 0)).view(x16.sizes());
-      const Tensor dw = weight_grad(x16.reshape({-1, n_in}).contiguous(), joint);
-      const Tensor db = has_bias ? colsum(joint) : Tensor();
+      Tensor dw, db;
+      linear_grads(x16.reshape({-1, n_in}).contiguous(), joint, &dw, has_bias ? &db : nullptr);
       for (int i = 0; i < 3; ++i) {
         res[1 + 2 * i] = dw.narrow(0, i * n_out, n_out);
         if (has_bias) res[2 + 2 * i] = db.narrow(0, i * n_out, n_out);
@@ -377,11 +403,9 @@ struct Projection3 : public torch::autograd::Function<Projection3> {
         else
           gx = at::mm(g2, w[i]);
       }
-      if (want_w[i]) {
-        if (!x2.defined()) x2 = x16.reshape({-1, n_in}).contiguous();
-        res[1 + 2 * i] = weight_grad(x2, g2);
-      }
-      if (want_b[i]) res[2 + 2 * i] = colsum(g2);
+      if (!x2.defined()) x2 = x16.reshape({-1, n_in}).contiguous();
+      linear_grads(x2, g2, want_w[i] ? &res[1 + 2 * i] : nullptr,
+                   want_b[i] ? &res[2 + 2 * i] : nullptr);
     }
     if (gx.defined()) res[0] = gx.view(x16.sizes());
     return res;
@@ -535,6 +559,8 @@ void init(const std::map<std::string, int64_t>& addr) {
   entry(g_colsum_ws, addr, "ngt_colsum_workspace_bytes");
   entry(g_colsum, addr, "ngt_colsum_bf16");
   entry(g_chunk_sum, addr, "ngt_chunk_sum_f32");
+  entry(g_wgrad_ws, addr, "ngt_wgrad_workspace_bytes");
+  entry(g_wgrad, addr, "ngt_wgrad_bf16");
   entry(g_ln_fwd, addr, "ngt_layernorm_fwd");
   entry(g_ln_bwd_ws, addr, "ngt_layernorm_bwd_workspace_bytes");
   entry(g_ln_bwd, addr, "ngt_layernorm_bwd");

@@ -1,5 +1,4 @@
-"""nn.Linear with a split-K weight gradient and a HIP bias gradient under
-bf16 autocast.
+"""nn.Linear with HIP weight and bias gradients under bf16 autocast.
 
 The encoder's projections (NeutronGT/models/graphormer_dist_node_level.py:
 130-206, the GT twin's :230-302) multiply [32,768 x 768] activations by
@@ -9,10 +8,10 @@ and a 32,768-long reduction, and autocast's single GEMM for it ran at 190 us
 nn.Linear's parameters, names and forward (the same bf16 GEMM autocast runs)
 and in the backward computes
   dX = dY W                          (torch GEMM, bf16, as autocast does),
-  dW = sum_c dY_c^T X_c              (one batched library GEMM over 16 row
-                                      chunks with fp32 output, then a sum in
-                                      chunk order, ngt_chunk_sum_f32),
-  db = column sums of dY             (ngt_colsum_bf16, fp32, fixed order).
+  dW = dY^T X and db = column sums of dY, in fp32 and a fixed order, from one
+                                     pass over the rows (ngt_wgrad_bf16) or,
+                                     for the largest, library GEMMs over row
+                                     chunks and ngt_colsum_bf16 (_fused).
 dW and db are fp32 (autocast's own backward rounds dW to bf16 first).
 Outside bf16 autocast or without gradients it is a plain nn.Linear.  Any
 widths: the node encoder (100 -> 768) and a 47-class readout take the same
@@ -31,8 +30,10 @@ import torch.nn.functional as F
 
 from . import _lib
 
-_CHUNK = 2048      # rows per split of the weight-gradient reduction
+_CHUNK = 2048      # rows per split of the library's weight-gradient reduction
 _MAX_SPLITS = 16   # 16 x 2048 rows measured fastest for 32,768 x 768 x 768
+_FUSED_PRODUCTS = 18_000_000_000  # the limits of _fused
+_FUSED_ROWS, _FUSED_OUTPUTS = 3000, 1_000_000
 
 
 def colsum_bf16(dy: torch.Tensor) -> torch.Tensor:
@@ -65,8 +66,26 @@ def chunk_sum(parts: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def weight_grad(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
-    """dY^T X in fp32 for bf16 x [K, n_in], dy [K, n_out], split over rows.
+def linear_grads(x: torch.Tensor, dy: torch.Tensor, bias: bool):
+    """(dY^T X, column sums of dY or None) in fp32 for bf16 GPU matrices
+    x [K, n_in], dy [K, n_out], from one pass over their rows."""
+    lib = _lib.load()
+    x, dy = x.contiguous(), dy.contiguous()
+    (K, n_in), n_out = x.shape, dy.shape[1]
+    dw = torch.empty(n_out, n_in, dtype=torch.float32, device=x.device)
+    db = torch.empty(n_out, dtype=torch.float32, device=x.device) if bias else None
+    nb = C.c_size_t()
+    _lib.check(lib.ngt_wgrad_workspace_bytes(K, n_out, n_in, C.byref(nb)))
+    ws = torch.empty(max(nb.value, 1), dtype=torch.uint8, device=x.device)
+    _lib.check(lib.ngt_wgrad_bf16(x.data_ptr(), dy.data_ptr(), K, n_out, n_in, dw.data_ptr(),
+                                  db.data_ptr() if bias else None, ws.data_ptr(), nb.value,
+                                  _lib.stream_ptr(x.device)))
+    return dw, db
+
+
+def _library_weight_grad(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
+    """dY^T X in fp32 by library GEMMs for x [K, n_in], dy [K, n_out], split over
+    rows.
     Outputs of 1.5 M elements or more (the stacked Q/K/V gradient, 2,304 x
     768) take at most 8 splits: their GEMM has tiles enough at 8, and the
     chunk sum reads half as much (146 against 154 us with the sum)."""
@@ -86,6 +105,37 @@ def weight_grad(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
     return dw
 
 
+def _fused(x: torch.Tensor, dy: torch.Tensor) -> bool:
+    """Whether linear_grads takes these rows (a gradient that will itself be
+    differentiated is torch's).  The library's large GEMM tiles are the faster
+    from about 1.8e10 products on (32,768 x 768 x 768 with the bias 65.8 us
+    against 66 to 72, 32,768 x 2,304 x 768 168 against 181; but 10,007 x 2,304 x
+    768 92 against 73), and for a million outputs over few rows, where the
+    partials weigh most (1,000 x 2,304 x 768 25.8 against 32, 3,000 rows 40.7
+    against 37.6)."""
+    rows, outputs = x.shape[0], x.shape[1] * dy.shape[1]
+    return (not torch.is_grad_enabled() and outputs > 0 and rows * outputs <= _FUSED_PRODUCTS
+            and (rows >= _FUSED_ROWS or outputs < _FUSED_OUTPUTS))
+
+
+def _grads(x2: torch.Tensor, g2: torch.Tensor, want_w: bool, want_b: bool):
+    """(dW or None, db or None) of contiguous bf16 rows inside a backward."""
+    if want_w and _fused(x2, g2):
+        return linear_grads(x2, g2, want_b)
+    return _library_weight_grad(x2, g2) if want_w else None, colsum_bf16(g2) if want_b else None
+
+
+def weight_grad(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
+    """dY^T X in fp32 for x [K, n_in], dy [K, n_out] on the GPU."""
+    if (x.dtype == dy.dtype == torch.bfloat16 and x.is_cuda and x.device == dy.device
+            and x.dim() == dy.dim() == 2 and x.shape[0] == dy.shape[0]
+            and not (torch.is_grad_enabled() and (x.requires_grad or dy.requires_grad))):
+        with torch.no_grad():
+            if _fused(x, dy):
+                return linear_grads(x, dy, False)[0]
+    return _library_weight_grad(x, dy)
+
+
 class _WgradLinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
@@ -103,14 +153,12 @@ class _WgradLinearFn(torch.autograd.Function):
         x16, w16 = ctx.saved_tensors
         n_out, n_in = w16.shape
         g2 = gy.to(torch.bfloat16).reshape(-1, n_out).contiguous()
-        gx = dw = db = None
+        gx = None
         if ctx.needs_input_grad[0]:
             with torch.autocast("cuda", enabled=False):
                 gx = (g2 @ w16).view(*x16.shape)
-        if ctx.needs_input_grad[1]:
-            dw = weight_grad(x16.reshape(-1, n_in).contiguous(), g2)
-        if ctx.has_bias and ctx.needs_input_grad[2]:
-            db = colsum_bf16(g2)
+        dw, db = _grads(x16.reshape(-1, n_in).contiguous(), g2, ctx.needs_input_grad[1],
+                        ctx.has_bias and ctx.needs_input_grad[2])
         return gx, dw, db
 
 
@@ -183,8 +231,7 @@ class _ProjectionGroupFn(torch.autograd.Function):
             if ctx.needs_input_grad[0]:
                 with torch.autocast("cuda", enabled=False):
                     gx = (joint @ torch.cat(ws, 0)).view(*x16.shape)
-            dw = weight_grad(x16.reshape(-1, n_in).contiguous(), joint)
-            db = colsum_bf16(joint) if ctx.has_bias[0] else None
+            dw, db = _grads(x16.reshape(-1, n_in).contiguous(), joint, True, ctx.has_bias[0])
             grads = []
             for i in range(len(ws)):
                 grads += [dw[i * n_out:(i + 1) * n_out],
@@ -204,14 +251,10 @@ class _ProjectionGroupFn(torch.autograd.Function):
                         gx = g2 @ w16
                     else:
                         gx.addmm_(g2, w16)
-            dw = db = None
-            if ctx.needs_input_grad[1 + 2 * i]:
-                if x2 is None:
-                    x2 = x16.reshape(-1, n_in).contiguous()
-                dw = weight_grad(x2, g2)
-            if ctx.has_bias[i] and ctx.needs_input_grad[2 + 2 * i]:
-                db = colsum_bf16(g2)
-            grads += [dw, db]
+            if x2 is None:
+                x2 = x16.reshape(-1, n_in).contiguous()
+            grads += _grads(x2, g2, ctx.needs_input_grad[1 + 2 * i],
+                            ctx.has_bias[i] and ctx.needs_input_grad[2 + 2 * i])
         if gx is not None:
             gx = gx.view(*x16.shape)
         return (gx, *grads)
@@ -232,7 +275,7 @@ def project(x: torch.Tensor, *lins: nn.Linear, heads: int = 0):
     """(lin(x) for lin in lins), viewed as [..., heads, n_out / heads] when
     ``heads`` is given, with the backward's dX summed inside the
     GEMMs (and, for gradients that arrive as column blocks of one matrix, dW
-    and db as one GEMM and one column sum) when all of them take the bf16
+    and db from one pass over its rows) when all of them take the bf16
     autocast path; otherwise each module's own forward.  Three layers (Q, K,
     V) run as one C++ node where ngt_autograd.so is built."""
     if groupable(x, *lins):
@@ -251,8 +294,8 @@ def project(x: torch.Tensor, *lins: nn.Linear, heads: int = 0):
 
 
 class WgradLinear(nn.Linear):
-    """nn.Linear (same parameters and state-dict names) with the split-K
-    weight gradient and the HIP bias gradient under bf16 autocast."""
+    """nn.Linear (same parameters and state-dict names) with the HIP weight
+    and bias gradients under bf16 autocast."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if _fast_path(self, x):
