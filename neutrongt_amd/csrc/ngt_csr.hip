@@ -24,7 +24,7 @@
 // each order took five passes of 12 bytes.  The sorts are rocPRIM's radix sort;
 // its default switches to a merge sort below 1 M entries, 23 launches for the
 // 0.67 M edges of a 16,384-node window against 5 or 6 (one window's build
-// there is bound by launches, not bytes), so SortConfig keeps radix passes
+// there is bound by launches, not bytes), so sort_edges keeps radix passes
 // down to 16 K entries.
 #include "ngt_common.h"
 
@@ -57,8 +57,59 @@ inline unsigned bits_for(uint64_t v) {
 
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+// Tiles of 16,384 keys (the library's choice) leave most of the chip idle below
+// a million edges; tiles of 4,096 fill it but look back over four times as many
+// predecessors.  One sort by a 15-bit endpoint with either: 30,000 keys 59 / 30
+// us, 230,000 63 / 37, 671,744 67 / 50, 1,800,000 77 / 80, 3,600,000 89 / 124.
+constexpr int64_t kSmallTiles = 1200000;
+using LargeTiles = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
                                               rocprim::default_config, 16 * 1024>;
+using SmallTiles = rocprim::radix_sort_config<
+    rocprim::default_config, rocprim::default_config,
+    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<256, 8>,
+                                        rocprim::kernel_config<1024, 4>, 8,
+                                        rocprim::block_radix_rank_algorithm::match>,
+    16 * 1024>;
+
+template <class Config>
+hipError_t sort_with(void* temp, size_t& bytes, uint32_t* key_in, uint32_t* key_out,
+                     int32_t* val_in, int32_t* val_out, int64_t n, unsigned bits, hipStream_t st) {
+  return rocprim::radix_sort_pairs<Config>(temp, bytes, key_in, key_out, val_in, val_out,
+                                           size_t(n), 0u, bits, st);
+}
+
+// Radix passes clear their counters with memsets, which replays of a captured
+// graph do not repeat reliably: under capture the library's default stays (a
+// merge sort, kernels only, below a million keys).
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  return st && hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
+int sort_edges(void* temp, size_t bytes, uint32_t* key_in, uint32_t* key_out, int32_t* val_in,
+               int32_t* val_out, int64_t n, unsigned bits, hipStream_t st) {
+  if (capturing(st))
+    NGT_HIP_CHECK(sort_with<rocprim::default_config>(temp, bytes, key_in, key_out, val_in, val_out,
+                                                     n, bits, st));
+  else if (n <= kSmallTiles)
+    NGT_HIP_CHECK(sort_with<SmallTiles>(temp, bytes, key_in, key_out, val_in, val_out, n, bits, st));
+  else
+    NGT_HIP_CHECK(sort_with<LargeTiles>(temp, bytes, key_in, key_out, val_in, val_out, n, bits, st));
+  return NGT_OK;
+}
+
+int sort_edges_bytes(int64_t n, size_t* bytes) {
+  size_t a = 0, b = 0;
+  uint32_t* k = nullptr;
+  int32_t* v = nullptr;
+  NGT_HIP_CHECK(sort_with<rocprim::default_config>(nullptr, a, k, k, v, v, n, 32u, nullptr));
+  if (n <= kSmallTiles)
+    NGT_HIP_CHECK(sort_with<SmallTiles>(nullptr, b, k, k, v, v, n, 32u, nullptr));
+  else
+    NGT_HIP_CHECK(sort_with<LargeTiles>(nullptr, b, k, k, v, v, n, 32u, nullptr));
+  *bytes = a > b ? a : b;
+  return NGT_OK;
+}
 
 // 32-bit endpoints; edges outside the window become {n_k, n_q}, which sorts
 // behind every row in both orders.
@@ -281,9 +332,7 @@ int csr_layout(int64_t E, int32_t n_q, int32_t n_k, CsrLayout* L) {
   const int64_t n_rows = n_q > n_k ? n_q : n_k;
   size_t sort_bytes = 0, scan_bytes = 0;
   const size_t n = static_cast<size_t>(E > 0 ? E : 1);
-  NGT_HIP_CHECK(rocprim::radix_sort_pairs<SortConfig>(
-      nullptr, sort_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, (int32_t*)nullptr,
-      (int32_t*)nullptr, n, 0u, 32u, hipStream_t(0)));
+  NGT_CHECK_OK(sort_edges_bytes(static_cast<int64_t>(n), &sort_bytes));
   NGT_HIP_CHECK(rocprim::exclusive_scan(nullptr, scan_bytes, (Count3*)nullptr, (Count3*)nullptr,
                                         Count3{0, 0, 0}, size_t(n_rows > 0 ? n_rows : 1),
                                         Count3Plus(), hipStream_t(0)));
@@ -452,11 +501,8 @@ extern "C" int ngt_csr_build(const int64_t* edge_index, ngt_window_csr* csr, voi
   NGT_HIP_CHECK(hipGetLastError());
   auto sort = [&](uint32_t* key_in, uint32_t* key_out, int32_t* val_in, int32_t* val_out,
                   int32_t n) -> int {  // keys 0 .. n
-    size_t tb = L.temp_bytes;
-    NGT_HIP_CHECK(rocprim::radix_sort_pairs<SortConfig>(ws + L.temp, tb, key_in, key_out, val_in,
-                                                        val_out, size_t(E), 0u,
-                                                        bits_for(uint64_t(n)), st));
-    return NGT_OK;
+    return sort_edges(ws + L.temp, L.temp_bytes, key_in, key_out, val_in, val_out, E,
+                      bits_for(uint64_t(n)), st);
   };
   if (E > 0) {
     hipLaunchKernelGGL(k_endpoints, dim3(grid_for(E)), dim3(kBlock), 0, st, edge_index,
