@@ -188,38 +188,62 @@ __device__ __forceinline__ Count3 row_counts(int32_t deg, int32_t chunk) {
   return Count3{0, 1, 0};
 }
 
+// One order's rows and the lists made for them.  Both orders go through the
+// same launches, the query rows first: row r of a side is entry base + r.
+struct Side {
+  const int32_t* rowptr;
+  int32_t n_rows, chunk, small;
+  int64_t base;
+  int4 *items, *splits;
+  int32_t *packed, *order;  // order: every row, longest first (null: not here)
+  int32_t info_base, packed_slot, small_slot, max_deg_slot;
+};
+struct Sides {
+  Side s[2];
+};
+constexpr uint32_t kKeySide = 0x80000000u;  // of a degree: sorts behind the query rows
+
+__device__ __forceinline__ Count3 operator-(const Count3& a, const Count3& b) {
+  return Count3{int32_t(uint32_t(a.split_items) - uint32_t(b.split_items)),
+                int32_t(uint32_t(a.plain_items) - uint32_t(b.plain_items)),
+                int32_t(uint32_t(a.split_rows) - uint32_t(b.split_rows))};
+}
+
 // Per row: chunk counts for the scan, and (degree, row) pairs for the sort.
-__global__ void k_count(const int32_t* __restrict__ rowptr, int32_t n_rows, int32_t chunk,
-                        Count3* __restrict__ cnt, uint32_t* __restrict__ deg_key,
-                        int32_t* __restrict__ row_val, int32_t* __restrict__ info,
-                        int max_deg_slot) {
+// grid.y = side, as in the two kernels below.
+__global__ void k_count(const Sides sides, Count3* __restrict__ cnt,
+                        uint32_t* __restrict__ deg_key, int32_t* __restrict__ row_val,
+                        int32_t* __restrict__ info) {
+  const Side s = sides.s[blockIdx.y];
+  const uint32_t flag = blockIdx.y ? kKeySide : 0u;
   int32_t local_max = 0;
-  for (int32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n_rows; r += gridDim.x * blockDim.x) {
-    const int32_t deg = rowptr[r + 1] - rowptr[r];
-    cnt[r] = row_counts(deg, chunk);
-    deg_key[r] = static_cast<uint32_t>(deg);
-    row_val[r] = r;
+  for (int64_t r = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; r < s.n_rows;
+       r += int64_t(gridDim.x) * blockDim.x) {
+    const int32_t deg = s.rowptr[r + 1] - s.rowptr[r];
+    cnt[s.base + r] = row_counts(deg, s.chunk);
+    deg_key[s.base + r] = static_cast<uint32_t>(deg) | flag;
+    row_val[s.base + r] = static_cast<int32_t>(r);
     local_max = max(local_max, deg);
   }
-  if (local_max > 0) atomicMax(info + max_deg_slot, local_max);
+  if (local_max > 0) atomicMax(info + s.max_deg_slot, local_max);
 }
 
 // Chunks of the rows longer than `chunk` (row order) and the split table.
-__global__ void k_emit_split(const int32_t* __restrict__ rowptr, int32_t n_rows, int32_t chunk,
-                             const Count3* __restrict__ scan, int4* __restrict__ items,
-                             int4* __restrict__ splits) {
-  for (int32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n_rows; r += gridDim.x * blockDim.x) {
-    const int32_t beg = rowptr[r];
-    const int32_t end = rowptr[r + 1];
-    if (end - beg <= chunk) continue;
-    const Count3 pre = scan[r];
-    const int32_t n = (end - beg + chunk - 1) / chunk;
+__global__ void k_emit_split(const Sides sides, const Count3* __restrict__ scan) {
+  const Side s = sides.s[blockIdx.y];
+  for (int64_t r = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; r < s.n_rows;
+       r += int64_t(gridDim.x) * blockDim.x) {
+    const int32_t beg = s.rowptr[r];
+    const int32_t end = s.rowptr[r + 1];
+    if (end - beg <= s.chunk) continue;
+    const Count3 pre = scan[s.base + r] - scan[s.base];
+    const int32_t n = (end - beg + s.chunk - 1) / s.chunk;
     for (int32_t c = 0; c < n; ++c) {
-      const int32_t b = beg + c * chunk;
+      const int32_t b = beg + c * s.chunk;
       const int32_t slot = pre.split_items + c;
-      items[slot] = make_int4(r, b, min(end, b + chunk), slot);
+      s.items[slot] = make_int4(static_cast<int32_t>(r), b, min(end, b + s.chunk), slot);
     }
-    splits[pre.split_rows] = make_int4(r, pre.split_items, n, 0);
+    s.splits[pre.split_rows] = make_int4(static_cast<int32_t>(r), pre.split_items, n, 0);
   }
 }
 
@@ -241,11 +265,12 @@ constexpr int32_t kPackSteps[4] = {8, 16, 24, 32};
 constexpr int64_t kPackSharePct = 78;
 
 __device__ __forceinline__ int32_t packing_threshold(const uint32_t* __restrict__ sdeg,
-                                                     int32_t n_rows, int32_t chunk) {
+                                                     int32_t n_rows, int32_t chunk,
+                                                     uint32_t flag) {
   int32_t t = 0;
   for (int i = 0; i < 4; ++i) {
     t = min(kPackSteps[i], chunk - 1);
-    const int32_t packed = upper_bound_u32(sdeg, n_rows, static_cast<uint32_t>(t));
+    const int32_t packed = upper_bound_u32(sdeg, n_rows, static_cast<uint32_t>(t) | flag);
     if (int64_t(packed) * 100 >= int64_t(n_rows) * kPackSharePct) break;
   }
   return t;
@@ -254,44 +279,43 @@ __device__ __forceinline__ int32_t packing_threshold(const uint32_t* __restrict_
 // From the rows sorted by ascending degree: the packed small rows and the
 // single-item medium rows, both longest first.  info gets the totals and the
 // packing threshold used.
-__global__ void k_emit_sorted(const int32_t* __restrict__ rowptr, int32_t n_rows, int32_t chunk,
-                              int32_t small_in, const uint32_t* __restrict__ sdeg,
-                              const int32_t* __restrict__ srow, const Count3* __restrict__ scan,
-                              int4* __restrict__ items, int32_t* __restrict__ packed,
-                              int32_t* __restrict__ order, int32_t* __restrict__ info,
-                              int info_base, int packed_slot, int small_slot) {
-  const int32_t small = small_in < 0 ? packing_threshold(sdeg, n_rows, chunk) : small_in;
-  const int32_t n_small = upper_bound_u32(sdeg, n_rows, static_cast<uint32_t>(small));
-  const int32_t n_le_chunk = upper_bound_u32(sdeg, n_rows, static_cast<uint32_t>(chunk));
+__global__ void k_emit_sorted(const Sides sides, const uint32_t* __restrict__ sorted_deg,
+                              const int32_t* __restrict__ sorted_row,
+                              const Count3* __restrict__ scan, int32_t* __restrict__ info) {
+  const Side s = sides.s[blockIdx.y];
+  const uint32_t flag = blockIdx.y ? kKeySide : 0u;
+  const uint32_t* sdeg = sorted_deg + s.base;
+  const int32_t* srow = sorted_row + s.base;
+  const int32_t small =
+      s.small < 0 ? packing_threshold(sdeg, s.n_rows, s.chunk, flag) : s.small;
+  const int32_t n_small = upper_bound_u32(sdeg, s.n_rows, static_cast<uint32_t>(small) | flag);
+  const int32_t n_le_chunk =
+      upper_bound_u32(sdeg, s.n_rows, static_cast<uint32_t>(s.chunk) | flag);
   const int32_t n_medium = n_le_chunk - n_small;
   Count3 tot{0, 0, 0};
-  if (n_rows > 0) {
-    const Count3 last = scan[n_rows - 1];
-    const Count3 own = row_counts(rowptr[n_rows] - rowptr[n_rows - 1], chunk);
+  if (s.n_rows > 0) {
+    const Count3 last = scan[s.base + s.n_rows - 1] - scan[s.base];
+    const Count3 own = row_counts(s.rowptr[s.n_rows] - s.rowptr[s.n_rows - 1], s.chunk);
     tot = Count3{last.split_items + own.split_items, last.plain_items + own.plain_items,
                  last.split_rows + own.split_rows};
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    info[info_base + 0] = tot.split_items + n_medium;  // work items
-    info[info_base + 1] = tot.split_items;             // partial slots
-    info[info_base + 2] = tot.split_rows;              // split rows
-    info[packed_slot] = n_small;                       // packed rows
-    info[small_slot] = small;                          // their threshold
+    info[s.info_base + 0] = tot.split_items + n_medium;  // work items
+    info[s.info_base + 1] = tot.split_items;             // partial slots
+    info[s.info_base + 2] = tot.split_rows;              // split rows
+    info[s.packed_slot] = n_small;                       // packed rows
+    info[s.small_slot] = small;                          // their threshold
   }
-  for (int32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n_le_chunk;
-       p += gridDim.x * blockDim.x) {
+  for (int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; p < s.n_rows;
+       p += int64_t(gridDim.x) * blockDim.x) {
     const int32_t r = srow[p];
-    if (p < n_small) {
-      packed[n_small - 1 - p] = r;
-    } else {
-      items[tot.split_items + (n_le_chunk - 1 - p)] = make_int4(r, rowptr[r], rowptr[r + 1], -1);
-    }
+    if (p < n_small)
+      s.packed[n_small - 1 - p] = r;
+    else if (p < n_le_chunk)
+      s.items[tot.split_items + (n_le_chunk - 1 - p)] =
+          make_int4(r, s.rowptr[r], s.rowptr[r + 1], -1);
+    if (s.order) s.order[s.n_rows - 1 - p] = r;
   }
-  // every row, longest first (when the order covers all rows)
-  if (order)
-    for (int32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n_rows;
-         p += gridDim.x * blockDim.x)
-      order[n_rows - 1 - p] = srow[p];
 }
 
 // order[n - 1 - p] = srow[p]: rows sorted by ascending degree, reversed.
@@ -329,7 +353,7 @@ struct CsrLayout {
 };
 
 int csr_layout(int64_t E, int32_t n_q, int32_t n_k, CsrLayout* L) {
-  const int64_t n_rows = n_q > n_k ? n_q : n_k;
+  const int64_t n_rows = int64_t(n_q) + n_k;  // both orders' rows
   size_t sort_bytes = 0, scan_bytes = 0;
   const size_t n = static_cast<size_t>(E > 0 ? E : 1);
   NGT_CHECK_OK(sort_edges_bytes(static_cast<int64_t>(n), &sort_bytes));
@@ -369,53 +393,42 @@ int csr_layout(int64_t E, int32_t n_q, int32_t n_k, CsrLayout* L) {
   return NGT_OK;
 }
 
-// order (optional): the first n_order rows (all rows when n_order == n_rows),
-// longest first.
-int build_worklist(const int32_t* rowptr, int32_t n_rows, int32_t chunk, int32_t small,
-                   int4* items, int4* splits, int32_t* packed, int32_t* order, int32_t n_order,
-                   int32_t* info, int info_base,
-                   int packed_slot, int small_slot, int max_deg_slot, char* ws,
-                   const CsrLayout& L, hipStream_t st) {
+// Both orders' work lists (q.base = 0, k.base = the query rows).  order_lead
+// (optional): the first n_lead key rows, longest first.
+int build_worklists(const Sides& sides, int32_t* order_lead, int32_t n_lead, int32_t* info,
+                    char* ws, const CsrLayout& L, hipStream_t st) {
   Count3* cnt = reinterpret_cast<Count3*>(ws + L.cnt);
   Count3* scan = reinterpret_cast<Count3*>(ws + L.cnt_scan);
   uint32_t* deg_a = reinterpret_cast<uint32_t*>(ws + L.deg_a);
   uint32_t* deg_b = reinterpret_cast<uint32_t*>(ws + L.deg_b);
   int32_t* row_a = reinterpret_cast<int32_t*>(ws + L.row_a);
   int32_t* row_b = reinterpret_cast<int32_t*>(ws + L.row_b);
-  if (n_rows == 0) {
-    hipLaunchKernelGGL(k_emit_sorted, dim3(1), dim3(kBlock), 0, st, rowptr, n_rows, chunk, small,
-                       deg_b, row_b, scan, items, packed, order, info, info_base, packed_slot,
-                       small_slot);
+  const Side &q = sides.s[0], &k = sides.s[1];
+  const int64_t rows = int64_t(q.n_rows) + k.n_rows;
+  const dim3 grid(grid_for(q.n_rows > k.n_rows ? q.n_rows : k.n_rows), 2);
+  if (rows > 0) {
+    hipLaunchKernelGGL(k_count, grid, dim3(kBlock), 0, st, sides, cnt, deg_a, row_a, info);
     NGT_HIP_CHECK(hipGetLastError());
-    return NGT_OK;
+    size_t temp_bytes = L.temp_bytes;
+    NGT_HIP_CHECK(rocprim::exclusive_scan(ws + L.temp, temp_bytes, cnt, scan, Count3{0, 0, 0},
+                                          size_t(rows), Count3Plus(), st));
+    hipLaunchKernelGGL(k_emit_split, grid, dim3(kBlock), 0, st, sides, scan);
+    NGT_HIP_CHECK(hipGetLastError());
+    temp_bytes = L.temp_bytes;
+    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, deg_a, deg_b, row_a, row_b,
+                                            size_t(rows), 0u, 32u, st));
   }
-  hipLaunchKernelGGL(k_count, dim3(grid_for(n_rows)), dim3(kBlock), 0, st, rowptr, n_rows, chunk,
-                     cnt, deg_a, row_a, info, max_deg_slot);
+  hipLaunchKernelGGL(k_emit_sorted, grid, dim3(kBlock), 0, st, sides, deg_b, row_b, scan, info);
   NGT_HIP_CHECK(hipGetLastError());
-  size_t temp_bytes = L.temp_bytes;
-  NGT_HIP_CHECK(rocprim::exclusive_scan(ws + L.temp, temp_bytes, cnt, scan, Count3{0, 0, 0},
-                                        size_t(n_rows), Count3Plus(), st));
-  hipLaunchKernelGGL(k_emit_split, dim3(grid_for(n_rows)), dim3(kBlock), 0, st, rowptr, n_rows,
-                     chunk, scan, items, splits);
-  NGT_HIP_CHECK(hipGetLastError());
-  temp_bytes = L.temp_bytes;
-  NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, deg_a, deg_b, row_a, row_b,
-                                          size_t(n_rows), 0u, 32u, st));
-  const bool full_order = order && n_order >= n_rows;
-  hipLaunchKernelGGL(k_emit_sorted, dim3(grid_for(n_rows)), dim3(kBlock), 0, st, rowptr, n_rows,
-                     chunk, small, deg_b, row_b, scan, items, packed,
-                     full_order ? order : nullptr, info, info_base, packed_slot, small_slot);
-  NGT_HIP_CHECK(hipGetLastError());
-  if (order && !full_order && n_order > 0) {
-    // the leading rows alone: (degree, row) of rows [0, n_order) are the
-    // first n_order entries of deg_a / row_a (row order)
+  if (order_lead && n_lead > 0) {
+    // the leading rows alone: their (degree, row) are the first key entries
     uint32_t* deg_c = reinterpret_cast<uint32_t*>(ws + L.deg_c);
     int32_t* row_c = reinterpret_cast<int32_t*>(ws + L.row_c);
-    temp_bytes = L.temp_bytes;
-    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, deg_a, deg_c, row_a, row_c,
-                                            size_t(n_order), 0u, 32u, st));
-    hipLaunchKernelGGL(k_emit_order, dim3(grid_for(n_order)), dim3(kBlock), 0, st, row_c, n_order,
-                       order);
+    size_t temp_bytes = L.temp_bytes;
+    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, deg_a + k.base, deg_c,
+                                            row_a + k.base, row_c, size_t(n_lead), 0u, 32u, st));
+    hipLaunchKernelGGL(k_emit_order, dim3(grid_for(n_lead)), dim3(kBlock), 0, st, row_c, n_lead,
+                       order_lead);
     NGT_HIP_CHECK(hipGetLastError());
   }
   return NGT_OK;
@@ -526,16 +539,14 @@ extern "C" int ngt_csr_build(const int64_t* edge_index, ngt_window_csr* csr, voi
                        csr->info);
     NGT_HIP_CHECK(hipGetLastError());
   }
-  rc = build_worklist(csr->rowptr, n_q, csr->chunk_q, csr->small_q,
-                      reinterpret_cast<int4*>(csr->items_q), reinterpret_cast<int4*>(csr->splits_q),
-                      csr->packed_q, csr->order_q, n_q, csr->info, NGT_INFO_ITEMS_Q,
-                      NGT_INFO_PACKED_Q,
-                      NGT_INFO_SMALL_Q, NGT_INFO_MAX_DEG_Q, ws, L, st);
-  if (rc != NGT_OK) return rc;
-  rc = build_worklist(csr->t_rowptr, n_k, csr->chunk_k, csr->small_k,
-                      reinterpret_cast<int4*>(csr->items_k), reinterpret_cast<int4*>(csr->splits_k),
-                      csr->packed_k, csr->order_k, n_q < n_k ? n_q : n_k, csr->info,
-                      NGT_INFO_ITEMS_K, NGT_INFO_PACKED_K,
-                      NGT_INFO_SMALL_K, NGT_INFO_MAX_DEG_K, ws, L, st);
-  return rc;
+  const int32_t n_own = n_q < n_k ? n_q : n_k;  // the window's own key rows
+  const bool all_keys = n_own == n_k;
+  const Sides sides{{
+      {csr->rowptr, n_q, csr->chunk_q, csr->small_q, 0, reinterpret_cast<int4*>(csr->items_q),
+       reinterpret_cast<int4*>(csr->splits_q), csr->packed_q, csr->order_q, NGT_INFO_ITEMS_Q,
+       NGT_INFO_PACKED_Q, NGT_INFO_SMALL_Q, NGT_INFO_MAX_DEG_Q},
+      {csr->t_rowptr, n_k, csr->chunk_k, csr->small_k, n_q, reinterpret_cast<int4*>(csr->items_k),
+       reinterpret_cast<int4*>(csr->splits_k), csr->packed_k, all_keys ? csr->order_k : nullptr,
+       NGT_INFO_ITEMS_K, NGT_INFO_PACKED_K, NGT_INFO_SMALL_K, NGT_INFO_MAX_DEG_K}}};
+  return build_worklists(sides, all_keys ? nullptr : csr->order_k, n_own, csr->info, ws, L, st);
 }
