@@ -391,6 +391,12 @@ struct Fp32Ops {
 // bytes of a row image, its 16-byte unit chosen by (operand number, g): the
 // MFMAs of a tile pair A and B operands so that, over the four g, every piece
 // product down to 2^-16 is there once; the smallest come first.
+// The dK/dV pass has the two matrices the other way round, and its S has to
+// round as the forward's did: exp(S - lse) with another last bit of S is off by
+// as much as S is large (at d = 16, 8 heads, 406 nodes dV's error was 3.2e-6,
+// with the forward's S 1.2e-6).  So the leading products h h come last and in a
+// product by themselves with m m, and at d = 8, where one MFMA holds all four,
+// that pass swaps the operands' patterns too.
 // With one piece per operand (d = 64) they are the row's two halves.
 template <int DH, int NP>
 struct Pairs {
@@ -402,13 +408,13 @@ struct Pairs {
 };
 template <int DH>
 struct Pairs<DH, 3> {
-  static constexpr int NA = DH == 8 ? 2 : DH == 64 ? 6 : 3;   // A operands
-  static constexpr int NB = DH <= 16 ? 2 : DH == 64 ? 6 : 3;  // B operands
+  static constexpr int NA = DH <= 16 ? 2 : DH == 64 ? 6 : 3;  // A operands
+  static constexpr int NB = DH == 8 ? 2 : DH == 64 ? 6 : 3;   // B operands
   static constexpr int N = DH == 8 ? 2 : DH == 16 ? 3 : DH == 64 ? 12 : 6;
   // the N MFMAs, smallest products first
   static constexpr __host__ __device__ int a_of(int n) {
     if constexpr (DH == 8) return 1 - n;        // [h l m l] x [l h l m], [h h m m] x [h m h m]
-    else if constexpr (DH == 16) return 2 - n;  // [h l] x [l h], [m m] x [h m], [h h] x [h m]
+    else if constexpr (DH == 16) return n == 0;  // [h l] x [l h], [h m] x [m h], [h m] x [h m]
     else {
       constexpr int a[6] = {2, 0, 1, 1, 0, 0};
       return DH == 64 ? 2 * a[n / 2] + n % 2 : a[n];
@@ -416,7 +422,7 @@ struct Pairs<DH, 3> {
   }
   static constexpr __host__ __device__ int b_of(int n) {
     if constexpr (DH == 8) return 1 - n;
-    else if constexpr (DH == 16) return n == 0 ? 1 : 0;
+    else if constexpr (DH == 16) return n == 0 ? 1 : n == 1 ? 2 : 0;
     else {
       constexpr int b[6] = {0, 2, 1, 0, 1, 0};
       return DH == 64 ? 2 * b[n / 2] + n % 2 : b[n];
@@ -431,8 +437,8 @@ struct Pairs<DH, 3> {
       return 16 * (k == 0 ? first : second);
     } else if constexpr (DH == 16) {
       const int hi = g >> 1;  // the second two lane groups
-      const int piece = b ? (k == 0 ? hi : (hi ? 0 : 2))                      // hm / lh
-                          : (k == 0 ? 0 : k == 1 ? 1 : (hi ? 2 : 0));         // hh / mm / hl
+      const int piece = b ? (k == 0 ? hi : hi ? 0 : 3 - k)  // hm / lh / mh
+                          : (k == 0 ? hi : 2 * hi);         // hm / hl
       return 16 * (piece * CB + (g & 1));
     } else if constexpr (DH == 64) {
       return 16 * ((k / 2) * CB + 4 * (k % 2) + g);
@@ -442,9 +448,10 @@ struct Pairs<DH, 3> {
   }
 };
 
-template <typename T, int DH, int G>
+template <typename T, int DH, int G, bool SWAP = false>
 struct PieceOps {
   static constexpr int NP = pieces<T>();
+  static constexpr bool ROLE_A = SWAP && DH == 8;  // the pattern of a staged row
   static constexpr bool SCALED = NP == 3;
   static constexpr int SB = DH <= 16 || NP == 1 ? 64 : 32;
   static constexpr int MT = out_tiles(DH);
@@ -459,7 +466,7 @@ struct PieceOps {
 #pragma unroll
     for (int k = 0; k < P::NB; ++k) {
       uint4 w = make_uint4(0u, 0u, 0u, 0u);
-      if (row < n_pad) w = *reinterpret_cast<const uint4*>(p + P::unit(true, k, g));
+      if (row < n_pad) w = *reinterpret_cast<const uint4*>(p + P::unit(!ROLE_A, k, g));
       r.x[u][k] = __builtin_bit_cast(bf16x8, w);
     }
   }
@@ -507,7 +514,7 @@ struct PieceOps {
         bf16x8 a[P::NA];
 #pragma unroll
         for (int k = 0; k < P::NA; ++k)
-          a[k] = *reinterpret_cast<const bf16x8*>(p + P::unit(false, k, g));
+          a[k] = *reinterpret_cast<const bf16x8*>(p + P::unit(ROLE_A, k, g));
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           x[t][u] = zero4();
@@ -1126,7 +1133,7 @@ constexpr int bwd_kv_lds() {
 template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
-  using P = PieceOps<T, DH, G>;
+  using P = PieceOps<T, DH, G, true>;
   __shared__ __align__(16) char lds[max_of(bwd_kv_lds<F>(), bwd_kv_lds<P>())];
   __shared__ __align__(16) float ls[64];
   __shared__ __align__(16) float ds[64];
