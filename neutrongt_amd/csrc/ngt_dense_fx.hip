@@ -253,8 +253,9 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
 }
 
 // Whether any step of head h of these matrices takes the fp32 body (the same
-// answer in every thread of the block).
+// answer in every thread of the block).  Without images (few_scores) all do.
 __device__ __forceinline__ bool any_flag(const Mat& a, const Mat& b, const Mat& c, int h) {
+  if (!a.flag) return true;
   int bad = 0;
   const Mat* m[3] = {&a, &b, &c};
 #pragma unroll
@@ -1191,7 +1192,9 @@ struct Images {
   int H, d, np;
   PrepJobs jobs{};
   int n_jobs = 0, max_rows = 0;
+  bool none = false;  // no images: the fp32 bodies read the matrices themselves
   Mat add(const void* x, int n, float scale, bool want_t) {
+    if (none) return Mat{x, nullptr, nullptr, nullptr, n, scale};
     PrepJob& j = jobs.j[n_jobs++];
     j.x = x;
     j.row_img = ws;
@@ -1299,13 +1302,26 @@ MfSplit fx_dq_split(int n_q, int n_k, int H, int d) {
   return split_keys_for(n_q, n_k, H, d, 6144, 0, "NGT_DENSE_F32_DQ_SPLIT");
 }
 
+// Few scores: the fp32 bodies alone, on the matrices as they are.  Their MFMAs
+// take 8 times the cycles, but up to here the two preparation launches and the
+// pieces' splits cost more.  Forward and backward in us, pieces / fp32: 8 heads
+// of 8, 406 nodes 61 / 36, 2,048 nodes 170 / 144; 8 of 16, 2,048 nodes 204 / 193;
+// 32 of 24, 1,000 nodes 279 / 240, 2,048 nodes 942 / 1,103; 8 of 64, 406 nodes
+// 127 / 115, 1,000 nodes 214 / 236.  NGT_DENSE_F32_TILES asks for the pieces.
+bool few_scores(int dtype, int n_q, int n_k, int H, int d) {
+  return dtype == NGT_F32 && !getenv("NGT_DENSE_F32_TILES") &&
+         int64_t(n_q) * n_k <= (int64_t(1) << (d == 64 ? 22 : 25)) / std::max(H, 1);
+}
+
 // Bytes of the images and flags that the two directions keep in the workspace.
 size_t fx_fwd_image_bytes(int dtype, int n_q, int n_k, int H, int d) {
+  if (few_scores(dtype, n_q, n_k, H, d)) return 0;
   const int np = dtype == NGT_F32 ? 3 : 1;
   return row_image_bytes(n_q, H, d, np) + flag_bytes(n_q, H) + 2 * row_image_bytes(n_k, H, d, np) +
          t_image_bytes(n_k, H, d, np) + 2 * flag_bytes(n_k, H);
 }
 size_t fx_bwd_image_bytes(int dtype, int n_q, int n_k, int H, int d) {
+  if (few_scores(dtype, n_q, n_k, H, d)) return 0;
   const int np = dtype == NGT_F32 ? 3 : 1;
   return 2 * (row_image_bytes(n_q, H, d, np) + t_image_bytes(n_q, H, d, np) + flag_bytes(n_q, H)) +
          2 * (row_image_bytes(n_k, H, d, np) + flag_bytes(n_k, H)) + t_image_bytes(n_k, H, d, np);
@@ -1324,6 +1340,7 @@ int fx_dense_fwd(int dtype, int d, const void* q, const void* k, const void* v, 
                  float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
                  hipStream_t st) {
   Images im{images, H, d, dtype == NGT_F32 ? 3 : 1};
+  im.none = few_scores(dtype, n_q, n_k, H, d);
   FwdArgs a{};
   drop_terms(dm, &a.thr16, &a.drop_scale);
   a.q = im.add(q, n_q, scale, false);
@@ -1353,6 +1370,7 @@ int fx_dense_bwd(int dtype, int d, const void* q, const void* k, const void* v, 
                  int n_k, int H, float scale, const DropoutMask* dm, void* gq, void* gk, void* gv,
                  MfSplit sq, float* part_dq, char* images, hipStream_t st) {
   Images im{images, H, d, dtype == NGT_F32 ? 3 : 1};
+  im.none = few_scores(dtype, n_q, n_k, H, d);
   BwdArgs a{};
   drop_terms(dm, &a.thr16, &a.drop_scale);
   a.q = im.add(q, n_q, scale, true);
