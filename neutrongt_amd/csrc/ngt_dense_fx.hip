@@ -395,9 +395,8 @@ struct Fp32Ops {
 // The dK/dV pass has the two matrices the other way round, and its S has to
 // round as the forward's did: exp(S - lse) with another last bit of S is off by
 // as much as S is large (at d = 16, 8 heads, 406 nodes dV's error was 3.2e-6,
-// with the forward's S 1.2e-6).  So the leading products h h come last and in a
-// product by themselves with m m, and at d = 8, where one MFMA holds all four,
-// that pass swaps the operands' patterns too.
+// with the forward's S 1.2e-6).  So the leading products h h come last, with none
+// beside them that weighs 2^-8, and their group is the same from both sides.
 // With one piece per operand (d = 64) they are the row's two halves.
 template <int DH, int NP>
 struct Pairs {
@@ -414,7 +413,7 @@ struct Pairs<DH, 3> {
   static constexpr int N = DH == 8 ? 2 : DH == 16 ? 3 : DH == 64 ? 12 : 6;
   // the N MFMAs, smallest products first
   static constexpr __host__ __device__ int a_of(int n) {
-    if constexpr (DH == 8) return 1 - n;        // [h l m l] x [l h l m], [h h m m] x [h m h m]
+    if constexpr (DH == 8) return 1 - n;
     else if constexpr (DH == 16) return n == 0;  // [h l] x [l h], [h m] x [m h], [h m] x [h m]
     else {
       constexpr int a[6] = {2, 0, 1, 1, 0, 0};
@@ -433,9 +432,9 @@ struct Pairs<DH, 3> {
   static __device__ __forceinline__ int unit(bool b, int k, int g) {
     constexpr int CB = col_blocks(DH);
     if constexpr (DH == 8) {
-      const int first = b ? (g & 1) : (g >> 1);                              // hmhm / hhmm
-      const int second = b ? (g == 1 ? 0 : g == 3 ? 1 : 2) : (g == 0 ? 0 : g == 2 ? 1 : 2);
-      return 16 * (k == 0 ? first : second);
+      // [h m m l] x [h m l m] last, [h l h m] x [l h m h] first
+      const uint32_t units = k == 0 ? (b ? 0x1210u : 0x2110u) : (b ? 0x0102u : 0x1020u);
+      return 16 * int(units >> (4 * g) & 15u);
     } else if constexpr (DH == 16) {
       const int hi = g >> 1;  // the second two lane groups
       const int piece = b ? (k == 0 ? hi : hi ? 0 : 3 - k)  // hm / lh / mh
@@ -449,10 +448,9 @@ struct Pairs<DH, 3> {
   }
 };
 
-template <typename T, int DH, int G, bool SWAP = false>
+template <typename T, int DH, int G>
 struct PieceOps {
   static constexpr int NP = pieces<T>();
-  static constexpr bool ROLE_A = SWAP && DH == 8;  // the pattern of a staged row
   static constexpr bool SCALED = NP == 3;
   static constexpr int SB = DH <= 16 || NP == 1 ? 64 : 32;
   static constexpr int MT = out_tiles(DH);
@@ -467,7 +465,7 @@ struct PieceOps {
 #pragma unroll
     for (int k = 0; k < P::NB; ++k) {
       uint4 w = make_uint4(0u, 0u, 0u, 0u);
-      if (row < n_pad) w = *reinterpret_cast<const uint4*>(p + P::unit(!ROLE_A, k, g));
+      if (row < n_pad) w = *reinterpret_cast<const uint4*>(p + P::unit(true, k, g));
       r.x[u][k] = __builtin_bit_cast(bf16x8, w);
     }
   }
@@ -515,7 +513,7 @@ struct PieceOps {
         bf16x8 a[P::NA];
 #pragma unroll
         for (int k = 0; k < P::NA; ++k)
-          a[k] = *reinterpret_cast<const bf16x8*>(p + P::unit(ROLE_A, k, g));
+          a[k] = *reinterpret_cast<const bf16x8*>(p + P::unit(false, k, g));
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           x[t][u] = zero4();
@@ -1134,7 +1132,7 @@ constexpr int bwd_kv_lds() {
 template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
-  using P = PieceOps<T, DH, G, true>;
+  using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(bwd_kv_lds<F>(), bwd_kv_lds<P>())];
   __shared__ __align__(16) float ls[64];
   __shared__ __align__(16) float ds[64];
