@@ -4,7 +4,8 @@
 // Part of the backward of the encoder's nn.Linear layers (MultiHeadAttention
 // projections and FFN, NeutronGT/models/graphormer_dist_node_level.py:130-206)
 // under bf16 autocast, where dy is [32,768 x 768]; the weight gradient itself
-// is a library GEMM (neutrongt_amd/linear.py).  A column reduction of a tall
+// is a library GEMM here; smaller layers take both from ngt_wgrad.hip
+// (neutrongt_amd/linear.py, _fused, has the rule).  A column reduction of a tall
 // matrix: blocks own 256 columns (a thread 8 adjacent columns, one 16-byte
 // load per row when the width allows) of a chunk of rows, and a second pass adds the chunks'
 // partials in chunk order.  HBM-bound: K * n * 2 bytes read once.
