@@ -79,8 +79,11 @@ hipError_t sort_with(void* temp, size_t& bytes, uint32_t* key_in, uint32_t* key_
 }
 
 // Radix passes clear their counters with memsets, which replays of a captured
-// graph do not repeat reliably: under capture the library's default stays (a
-// merge sort, kernels only, below a million keys).
+// graph do not repeat reliably: under capture every sort is a merge sort, kernels
+// only.  (The library's default takes radix passes above a million entries, and
+// the row sort below holds both sides' rows.)
+using KernelsOnly = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                               rocprim::default_config, (size_t(1) << 32)>;
 bool capturing(hipStream_t st) {
   hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
   return st && hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
@@ -89,8 +92,8 @@ bool capturing(hipStream_t st) {
 int sort_edges(void* temp, size_t bytes, uint32_t* key_in, uint32_t* key_out, int32_t* val_in,
                int32_t* val_out, int64_t n, unsigned bits, hipStream_t st) {
   if (capturing(st))
-    NGT_HIP_CHECK(sort_with<rocprim::default_config>(temp, bytes, key_in, key_out, val_in, val_out,
-                                                     n, bits, st));
+    NGT_HIP_CHECK(sort_with<KernelsOnly>(temp, bytes, key_in, key_out, val_in, val_out, n, bits,
+                                         st));
   else if (n <= kSmallTiles)
     NGT_HIP_CHECK(sort_with<SmallTiles>(temp, bytes, key_in, key_out, val_in, val_out, n, bits, st));
   else
@@ -102,11 +105,32 @@ int sort_edges_bytes(int64_t n, size_t* bytes) {
   size_t a = 0, b = 0;
   uint32_t* k = nullptr;
   int32_t* v = nullptr;
-  NGT_HIP_CHECK(sort_with<rocprim::default_config>(nullptr, a, k, k, v, v, n, 32u, nullptr));
+  NGT_HIP_CHECK(sort_with<KernelsOnly>(nullptr, a, k, k, v, v, n, 32u, nullptr));
   if (n <= kSmallTiles)
     NGT_HIP_CHECK(sort_with<SmallTiles>(nullptr, b, k, k, v, v, n, 32u, nullptr));
   else
     NGT_HIP_CHECK(sort_with<LargeTiles>(nullptr, b, k, k, v, v, n, 32u, nullptr));
+  *bytes = a > b ? a : b;
+  return NGT_OK;
+}
+
+// Rows by degree: the library's default, but for capture.
+int sort_rows(void* temp, size_t bytes, uint32_t* key_in, uint32_t* key_out, int32_t* val_in,
+              int32_t* val_out, int64_t n, hipStream_t st) {
+  if (capturing(st))
+    NGT_HIP_CHECK(sort_with<KernelsOnly>(temp, bytes, key_in, key_out, val_in, val_out, n, 32u, st));
+  else
+    NGT_HIP_CHECK(sort_with<rocprim::default_config>(temp, bytes, key_in, key_out, val_in, val_out,
+                                                     n, 32u, st));
+  return NGT_OK;
+}
+
+int sort_rows_bytes(int64_t n, size_t* bytes) {
+  size_t a = 0, b = 0;
+  uint32_t* k = nullptr;
+  int32_t* v = nullptr;
+  NGT_HIP_CHECK(sort_with<KernelsOnly>(nullptr, a, k, k, v, v, n, 32u, nullptr));
+  NGT_HIP_CHECK(sort_with<rocprim::default_config>(nullptr, b, k, k, v, v, n, 32u, nullptr));
   *bytes = a > b ? a : b;
   return NGT_OK;
 }
@@ -382,10 +406,7 @@ int csr_layout(int64_t E, int32_t n_q, int32_t n_k, CsrLayout* L) {
   L->deg_c = take(size_t(n_rows + 1) * 4);
   L->row_c = take(size_t(n_rows + 1) * 4);
   size_t deg_sort_bytes = 0;
-  NGT_HIP_CHECK(rocprim::radix_sort_pairs(nullptr, deg_sort_bytes, (uint32_t*)nullptr,
-                                          (uint32_t*)nullptr, (int32_t*)nullptr,
-                                          (int32_t*)nullptr, size_t(n_rows > 0 ? n_rows : 1),
-                                          0u, 32u, hipStream_t(0)));
+  NGT_CHECK_OK(sort_rows_bytes(n_rows > 0 ? n_rows : 1, &deg_sort_bytes));
   L->temp_bytes = sort_bytes > scan_bytes ? sort_bytes : scan_bytes;
   if (deg_sort_bytes > L->temp_bytes) L->temp_bytes = deg_sort_bytes;
   L->temp = take(L->temp_bytes);
@@ -414,9 +435,7 @@ int build_worklists(const Sides& sides, int32_t* order_lead, int32_t n_lead, int
                                           size_t(rows), Count3Plus(), st));
     hipLaunchKernelGGL(k_emit_split, grid, dim3(kBlock), 0, st, sides, scan);
     NGT_HIP_CHECK(hipGetLastError());
-    temp_bytes = L.temp_bytes;
-    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, deg_a, deg_b, row_a, row_b,
-                                            size_t(rows), 0u, 32u, st));
+    NGT_CHECK_OK(sort_rows(ws + L.temp, L.temp_bytes, deg_a, deg_b, row_a, row_b, rows, st));
   }
   hipLaunchKernelGGL(k_emit_sorted, grid, dim3(kBlock), 0, st, sides, deg_b, row_b, scan, info);
   NGT_HIP_CHECK(hipGetLastError());
@@ -424,9 +443,8 @@ int build_worklists(const Sides& sides, int32_t* order_lead, int32_t n_lead, int
     // the leading rows alone: their (degree, row) are the first key entries
     uint32_t* deg_c = reinterpret_cast<uint32_t*>(ws + L.deg_c);
     int32_t* row_c = reinterpret_cast<int32_t*>(ws + L.row_c);
-    size_t temp_bytes = L.temp_bytes;
-    NGT_HIP_CHECK(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, deg_a + k.base, deg_c,
-                                            row_a + k.base, row_c, size_t(n_lead), 0u, 32u, st));
+    NGT_CHECK_OK(sort_rows(ws + L.temp, L.temp_bytes, deg_a + k.base, deg_c, row_a + k.base, row_c,
+                           n_lead, st));
     hipLaunchKernelGGL(k_emit_order, dim3(grid_for(n_lead)), dim3(kBlock), 0, st, row_c, n_lead,
                        order_lead);
     NGT_HIP_CHECK(hipGetLastError());

@@ -1,6 +1,6 @@
 """GPU tests of the window CSR build where its sorts change: the merge sort below
-16,384 edges, small radix tiles up to 1,200,000, large ones above, and the
-library's default under graph capture."""
+16,384 edges, small radix tiles up to 1,200,000, large ones above, and merge
+sorts under graph capture."""
 import ctypes as C
 
 import numpy as np
@@ -40,10 +40,12 @@ def test_csr_at_the_sorts_edges(n_q, n_k, E):
     _check(WindowAdjacency(torch.from_numpy(ei).cuda(), n_q, n_k, 128, 16), ei, n_q, n_k, 128, 16)
 
 
-def test_csr_build_replayed_from_a_graph():
-    """Each replay rebuilds the arrays from the edges that the buffer holds then."""
-    n_q, n_k, E, chunk, small = 2000, 2300, 50000, 128, 16
-    print("case csr captured", flush=True)
+@pytest.mark.parametrize("n_q,n_k,E", [(2000, 2300, 50000), (600000, 600001, 50000)])
+def test_csr_build_replayed_from_a_graph(n_q, n_k, E):
+    """Each replay rebuilds the arrays from the edges that the buffer holds then;
+    the second case's row sort, both sides together, is longer than 1,048,576."""
+    chunk, small = 128, 16
+    print(f"case csr captured n_q={n_q} n_k={n_k} E={E}", flush=True)
     buf = torch.from_numpy(_edges(n_q, n_k, E, 0)).cuda()
     adj = WindowAdjacency(buf.clone(), n_q, n_k, chunk, small)
     lib, nb = _lib.load(), C.c_size_t()
