@@ -265,12 +265,17 @@ Tensor library_weight_grad(const Tensor& x, const Tensor& dy) {
 }
 
 // dw = dY^T X and, where wanted, db = column sums of dY, in fp32 from
-// contiguous bf16 rows (_grads of linear.py; its _fused explains the rule)
+// contiguous bf16 rows (_grads of linear.py; its _fused explains the rule).  x
+// may be undefined where dw is not wanted.
 void linear_grads(const Tensor& x, const Tensor& dy, Tensor* dw, Tensor* db) {
+  if (!dw) {
+    if (db) *db = colsum(dy);
+    return;
+  }
   const int64_t K = x.size(0), n_in = x.size(1), n_out = dy.size(1);
-  if (!dw || at::GradMode::is_enabled() || n_in == 0 || n_out == 0 ||
+  if (at::GradMode::is_enabled() || n_in == 0 || n_out == 0 ||
       K * n_in * n_out > kFusedProducts || (K < kFusedRows && n_in * n_out >= kFusedOutputs)) {
-    if (dw) *dw = library_weight_grad(x, dy);
+    *dw = library_weight_grad(x, dy);
     if (db) *db = colsum(dy);
     return;
   }
@@ -312,8 +317,9 @@ struct Linear : public torch::autograd::Function<Linear> {
     const Tensor g2 = bf16(grads[0]).reshape({-1, n_out}).contiguous();
     if (ctx->needs_input_grad(0)) res[0] = at::mm(g2, w16).view(x16.sizes());
     const bool want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
-    linear_grads(x16.reshape({-1, n_in}).contiguous(), g2,
-                 ctx->needs_input_grad(1) ? &res[1] : nullptr, want_b ? &res[2] : nullptr);
+    const bool want_w = ctx->needs_input_grad(1);
+    linear_grads(want_w ? x16.reshape({-1, n_in}).contiguous() : Tensor(), g2,
+                 want_w ? &res[1] : nullptr, want_b ? &res[2] : nullptr);
     return res;
   }
 };
@@ -403,7 +409,7 @@ struct Projection3 : public torch::autograd::Function<Projection3> {
         else
           gx = at::mm(g2, w[i]);
       }
-      if (!x2.defined()) x2 = x16.reshape({-1, n_in}).contiguous();
+      if (want_w[i] && !x2.defined()) x2 = x16.reshape({-1, n_in}).contiguous();
       linear_grads(x2, g2, want_w[i] ? &res[1 + 2 * i] : nullptr,
                    want_b[i] ? &res[2 + 2 * i] : nullptr);
     }

@@ -119,7 +119,8 @@ def _fused(x: torch.Tensor, dy: torch.Tensor) -> bool:
 
 
 def _grads(x2: torch.Tensor, g2: torch.Tensor, want_w: bool, want_b: bool):
-    """(dW or None, db or None) of contiguous bf16 rows inside a backward."""
+    """(dW or None, db or None) of contiguous bf16 rows inside a backward (x2
+    only where dW is wanted)."""
     if want_w and _fused(x2, g2):
         return linear_grads(x2, g2, want_b)
     return _library_weight_grad(x2, g2) if want_w else None, colsum_bf16(g2) if want_b else None
@@ -157,8 +158,9 @@ class _WgradLinearFn(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             with torch.autocast("cuda", enabled=False):
                 gx = (g2 @ w16).view(*x16.shape)
-        dw, db = _grads(x16.reshape(-1, n_in).contiguous(), g2, ctx.needs_input_grad[1],
-                        ctx.has_bias and ctx.needs_input_grad[2])
+        want_w = ctx.needs_input_grad[1]
+        x2 = x16.reshape(-1, n_in).contiguous() if want_w else None
+        dw, db = _grads(x2, g2, want_w, ctx.has_bias and ctx.needs_input_grad[2])
         return gx, dw, db
 
 
@@ -251,9 +253,10 @@ class _ProjectionGroupFn(torch.autograd.Function):
                         gx = g2 @ w16
                     else:
                         gx.addmm_(g2, w16)
-            if x2 is None:
+            want_w = ctx.needs_input_grad[1 + 2 * i]
+            if want_w and x2 is None:
                 x2 = x16.reshape(-1, n_in).contiguous()
-            grads += _grads(x2, g2, ctx.needs_input_grad[1 + 2 * i],
+            grads += _grads(x2, g2, want_w,
                             ctx.has_bias[i] and ctx.needs_input_grad[2 + 2 * i])
         if gx is not None:
             gx = gx.view(*x16.shape)
