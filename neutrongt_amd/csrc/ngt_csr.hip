@@ -15,13 +15,16 @@
 // (NeutronGT/models/graphormer_dist_node_level.py:75-97).  Here the ordering is
 // made canonical: query-major rows are sorted by (dst, src, edge id) and
 // key-major rows by (src, dst, edge id), so the CSR is a pure function of the
-// edge list (bit-exact, independent of launch shapes).  Three stable sorts by
-// one endpoint each make both orders: by src, then by dst, which leaves the
-// edges in (dst, src, edge id) order, then those by src again, which gives
-// (src, dst, edge id) and, with query-major positions as the values, the map
-// between the two.  Keys are 32 bits with bits_for(n) significant ones (15 at
-// 16,384 rows: two digit passes), where sorting the combined 64-bit keys of
-// each order took five passes of 12 bytes.  The sorts are rocPRIM's radix sort;
+// edge list (bit-exact, independent of launch shapes).  Stable sorts make both
+// orders: by (dst, src), which leaves the edges in (dst, src, edge id) order,
+// then those by src, which gives (src, dst, edge id) and, with query-major
+// positions as the values, the map between the two.  Keys are 32 bits; the first
+// sort is one of combined keys where both endpoints fit 32 bits (up to 65,535
+// rows a side) and else two, by src and by dst: the digit passes are as many,
+// but one sort spares a histogram, its scan, the gather of dst between the two
+// and the one of src after them (16,384 of 200,000 nodes: the window's whole
+// preparation 434 -> 420 us).  Combined 64-bit keys of each order took five
+// passes of 12 bytes.  The sorts are rocPRIM's radix sort;
 // its default switches to a merge sort below 1 M entries, 23 launches for the
 // 0.67 M edges of a 16,384-node window against 5 or 6 (one window's build
 // there is bound by launches, not bytes), so sort_edges keeps radix passes
@@ -135,19 +138,22 @@ int sort_rows_bytes(int64_t n, size_t* bytes) {
   return NGT_OK;
 }
 
-// 32-bit endpoints; edges outside the window become {n_k, n_q}, which sorts
-// behind every row in both orders.
+// 32-bit endpoints, or with dst32 null both in one key, dst << src_bits | src;
+// edges outside the window become {n_k, n_q}, which sorts behind every row in
+// both orders.
 __global__ void k_endpoints(const int64_t* __restrict__ src, const int64_t* __restrict__ dst,
-                            int64_t E, int32_t n_q, int32_t n_k, uint32_t* __restrict__ src32,
-                            uint32_t* __restrict__ dst32, int32_t* __restrict__ eid,
-                            int32_t* __restrict__ info) {
+                            int64_t E, int32_t n_q, int32_t n_k, unsigned src_bits,
+                            uint32_t* __restrict__ src32, uint32_t* __restrict__ dst32,
+                            int32_t* __restrict__ eid, int32_t* __restrict__ info) {
   for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < E;
        e += int64_t(gridDim.x) * blockDim.x) {
     const int64_t s = src[e];
     const int64_t d = dst[e];
     const bool ok = s >= 0 && s < n_k && d >= 0 && d < n_q;
-    src32[e] = ok ? uint32_t(s) : uint32_t(n_k);
-    dst32[e] = ok ? uint32_t(d) : uint32_t(n_q);
+    const uint32_t s32 = ok ? uint32_t(s) : uint32_t(n_k);
+    const uint32_t d32 = ok ? uint32_t(d) : uint32_t(n_q);
+    src32[e] = dst32 ? s32 : d32 << src_bits | s32;
+    if (dst32) dst32[e] = d32;
     if (!ok) atomicAdd(info + NGT_INFO_BAD_EDGES, 1);
     eid[e] = static_cast<int32_t>(e);
   }
@@ -160,50 +166,55 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ x, const int32_t* __re
     out[p] = x[at[p]];
 }
 
-// rowptr[r] = first position p of the sorted rows with rows[p] >= r; edges
-// outside the window (row n_rows) sit past rowptr[n_rows].
-__device__ __forceinline__ void fill_rowptr(const uint32_t* __restrict__ rows, int64_t E,
-                                            int64_t p, int32_t n_rows,
+// rowptr[r] = first position p of the sorted rows with rows[p] >= r (the rows
+// are the keys' bits from `shift` on); edges outside the window (row n_rows)
+// sit past rowptr[n_rows].
+__device__ __forceinline__ void fill_rowptr(const uint32_t* __restrict__ rows, unsigned shift,
+                                            int64_t E, int64_t p, int32_t n_rows,
                                             int32_t* __restrict__ rowptr) {
-  const int64_t r_cur = p < E ? int64_t(rows[p]) : int64_t(n_rows);
-  const int64_t r_prev = p > 0 ? int64_t(rows[p - 1]) : -1;
+  const int64_t r_cur = p < E ? int64_t(rows[p] >> shift) : int64_t(n_rows);
+  const int64_t r_prev = p > 0 ? int64_t(rows[p - 1] >> shift) : -1;
   for (int64_t r = r_prev + 1; r <= r_cur; ++r) rowptr[r] = static_cast<int32_t>(p);
 }
 
-// Query-major rows: row pointers and columns; the columns are also the third
+// Query-major rows: row pointers and columns; the columns are also the last
 // sort's keys (n_k for an edge outside the window) and the positions its values.
+// src_bits: the keys hold src in as many low bits (0: src32 does).
 __global__ void k_rows_q(const uint32_t* __restrict__ dst_sorted, const int32_t* __restrict__ perm,
-                         const uint32_t* __restrict__ src32, int64_t E, int32_t n_q, int32_t n_k,
+                         const uint32_t* __restrict__ src32, unsigned src_bits, int64_t E,
+                         int32_t n_q, int32_t n_k,
                          int32_t* __restrict__ rowptr, int32_t* __restrict__ col,
                          uint32_t* __restrict__ key, int32_t* __restrict__ pos) {
   for (int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; p <= E;
        p += int64_t(gridDim.x) * blockDim.x) {
     if (p < E) {
-      const uint32_t s = src32[perm[p]];
+      const uint32_t s =
+          src_bits ? dst_sorted[p] & ((1u << src_bits) - 1u) : src32[perm[p]];
       col[p] = s < uint32_t(n_k) ? static_cast<int32_t>(s) : 0;
       key[p] = s;
       pos[p] = static_cast<int32_t>(p);
     }
-    fill_rowptr(dst_sorted, E, p, n_q, rowptr);
+    fill_rowptr(dst_sorted, src_bits, E, p, n_q, rowptr);
   }
 }
 
 // Key-major rows: row pointers, columns, edge ids, and q2t.
 __global__ void k_rows_k(const uint32_t* __restrict__ src_sorted, const int32_t* __restrict__ qpos,
                          const int32_t* __restrict__ perm, const uint32_t* __restrict__ dst_sorted,
-                         int64_t E, int32_t n_q, int32_t n_k, int32_t* __restrict__ t_rowptr,
+                         unsigned src_bits, int64_t E, int32_t n_q, int32_t n_k,
+                         int32_t* __restrict__ t_rowptr,
                          int32_t* __restrict__ t_col, int32_t* __restrict__ t_perm,
                          int32_t* __restrict__ q2t) {
   for (int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; t <= E;
        t += int64_t(gridDim.x) * blockDim.x) {
     if (t < E) {
       const int32_t p = qpos[t];
-      const uint32_t d = dst_sorted[p];
+      const uint32_t d = dst_sorted[p] >> src_bits;
       t_col[t] = d < uint32_t(n_q) ? static_cast<int32_t>(d) : 0;
       t_perm[t] = perm[p];
       q2t[p] = static_cast<int32_t>(t);
     }
-    fill_rowptr(src_sorted, E, t, n_k, t_rowptr);
+    fill_rowptr(src_sorted, 0u, E, t, n_k, t_rowptr);
   }
 }
 
@@ -349,12 +360,12 @@ __global__ void k_emit_order(const int32_t* __restrict__ srow, int32_t n,
     order[n - 1 - p] = srow[p];
 }
 
-__global__ void k_ends(const uint32_t* __restrict__ dst_sorted,
+__global__ void k_ends(const uint32_t* __restrict__ dst_sorted, unsigned src_bits,
                        const uint32_t* __restrict__ src_sorted, const int32_t* __restrict__ rowptr,
                        int32_t n_q, int32_t* __restrict__ info) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int32_t nv = rowptr[n_q];  // valid edges (dropped ones sort last)
-    info[NGT_INFO_DST_END] = nv > 0 ? int32_t(dst_sorted[nv - 1]) + 1 : 0;
+    info[NGT_INFO_DST_END] = nv > 0 ? int32_t(dst_sorted[nv - 1] >> src_bits) + 1 : 0;
     info[NGT_INFO_SRC_END] = nv > 0 ? int32_t(src_sorted[nv - 1]) + 1 : 0;
   }
 }
@@ -531,30 +542,37 @@ extern "C" int ngt_csr_build(const int64_t* edge_index, ngt_window_csr* csr, voi
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, csr->info, NGT_INFO_LEN);
   NGT_HIP_CHECK(hipGetLastError());
   auto sort = [&](uint32_t* key_in, uint32_t* key_out, int32_t* val_in, int32_t* val_out,
-                  int32_t n) -> int {  // keys 0 .. n
-    return sort_edges(ws + L.temp, L.temp_bytes, key_in, key_out, val_in, val_out, E,
-                      bits_for(uint64_t(n)), st);
+                  unsigned bits) -> int {
+    return sort_edges(ws + L.temp, L.temp_bytes, key_in, key_out, val_in, val_out, E, bits, st);
   };
+  const unsigned bits_q = bits_for(uint64_t(n_q)), bits_k = bits_for(uint64_t(n_k));  // 0 .. n
+  const unsigned src_bits = bits_q + bits_k <= 32u ? bits_k : 0u;  // one combined key
   if (E > 0) {
     hipLaunchKernelGGL(k_endpoints, dim3(grid_for(E)), dim3(kBlock), 0, st, edge_index,
-                       edge_index + E, E, n_q, n_k, src32, dst32, val_a, csr->info);
+                       edge_index + E, E, n_q, n_k, src_bits, src32, src_bits ? nullptr : dst32,
+                       val_a, csr->info);
     NGT_HIP_CHECK(hipGetLastError());
-    NGT_CHECK_OK(sort(src32, key_a, val_a, val_b, n_k));  // val_b: edge ids by src
-    hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(E)), dim3(kBlock), 0, st, dst32, val_b, E,
-                       key_a);
-    NGT_HIP_CHECK(hipGetLastError());
-    NGT_CHECK_OK(sort(key_a, key_b, val_b, csr->perm, n_q));  // key_b: dst, query-major
+    // key_b: dst (above the src_bits of src), query-major
+    if (src_bits) {
+      NGT_CHECK_OK(sort(src32, key_b, val_a, csr->perm, bits_q + bits_k));
+    } else {
+      NGT_CHECK_OK(sort(src32, key_a, val_a, val_b, bits_k));  // val_b: edge ids by src
+      hipLaunchKernelGGL(k_gather_u32, dim3(grid_for(E)), dim3(kBlock), 0, st, dst32, val_b, E,
+                         key_a);
+      NGT_HIP_CHECK(hipGetLastError());
+      NGT_CHECK_OK(sort(key_a, key_b, val_b, csr->perm, bits_q));
+    }
   }
   hipLaunchKernelGGL(k_rows_q, dim3(grid_for(E + 1)), dim3(kBlock), 0, st, key_b, csr->perm, src32,
-                     E, n_q, n_k, csr->rowptr, csr->col, key_a, val_a);
+                     src_bits, E, n_q, n_k, csr->rowptr, csr->col, key_a, val_a);
   NGT_HIP_CHECK(hipGetLastError());
-  if (E > 0) NGT_CHECK_OK(sort(key_a, key_c, val_a, val_b, n_k));  // key_c: src, key-major
+  if (E > 0) NGT_CHECK_OK(sort(key_a, key_c, val_a, val_b, bits_k));  // key_c: src, key-major
   hipLaunchKernelGGL(k_rows_k, dim3(grid_for(E + 1)), dim3(kBlock), 0, st, key_c, val_b, csr->perm,
-                     key_b, E, n_q, n_k, csr->t_rowptr, csr->t_col, csr->t_perm, csr->q2t);
+                     key_b, src_bits, E, n_q, n_k, csr->t_rowptr, csr->t_col, csr->t_perm, csr->q2t);
   NGT_HIP_CHECK(hipGetLastError());
   if (E > 0) {
-    hipLaunchKernelGGL(k_ends, dim3(1), dim3(64), 0, st, key_b, key_c, csr->rowptr, n_q,
-                       csr->info);
+    hipLaunchKernelGGL(k_ends, dim3(1), dim3(64), 0, st, key_b, src_bits, key_c, csr->rowptr,
+                       n_q, csr->info);
     NGT_HIP_CHECK(hipGetLastError());
   }
   const int32_t n_own = n_q < n_k ? n_q : n_k;  // the window's own key rows

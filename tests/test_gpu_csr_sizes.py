@@ -1,6 +1,6 @@
 """GPU tests of the window CSR build where its sorts change: the merge sort below
-16,384 edges, small radix tiles up to 1,200,000, large ones above, and merge
-sorts under graph capture."""
+16,384 edges, small radix tiles up to 1,200,000, large ones above, merge sorts
+under graph capture, and one sort by (dst, src) where both fit 32 bits."""
 import ctypes as C
 
 import numpy as np
@@ -33,7 +33,8 @@ def _check(adj, ei, n_q, n_k, chunk, small):
 
 @pytest.mark.parametrize("n_q,n_k,E", [(3000, 3000, 16384), (3000, 3000, 16385), (257, 4000, 20481),
                                        (4000, 257, 262144), (32768, 32768, 1200000),
-                                       (32768, 40000, 1200001)])
+                                       (32768, 40000, 1200001), (65535, 65535, 70000),
+                                       (65535, 65536, 70000), (1, 90000, 30000)])
 def test_csr_at_the_sorts_edges(n_q, n_k, E):
     print(f"case csr n_q={n_q} n_k={n_k} E={E}", flush=True)
     ei = _edges(n_q, n_k, E, E)
