@@ -5,9 +5,11 @@
 // Products.  An fp32 value is the sum of three bf16 pieces h + m + l (each the
 // round-to-nearest of what is left, so the last remainder is zero or below
 // 2^-24 of the value).  A product of two such values is hh + (hm + mh) +
-// (mm + hl + lh) up to 2^-24, and v_mfma_f32_16x16x32_bf16 multiplies pieces
-// exactly, adds 8 products at a time exactly and rounds to fp32 once per 8
-// (checked on gfx950), so a contraction loses less than an fp32 FMA chain.
+// (mm + hl + lh) up to 2^-24.  v_mfma_f32_16x16x32_bf16 multiplies pieces
+// exactly, cuts the 8 products of a lane group to 24 bits of the largest, adds
+// them and the accumulator with 7 bits to spare and rounds to nearest, lane
+// group 0 first and 3 last (probed on gfx950), so a contraction whose largest
+// products come last loses less than an fp32 FMA chain.
 // At d = 8 a 32 x 32 tile of S takes 128 cycles of bf16 MFMAs where fp32 ones
 // take 256, and they leave the vector ALU to the exponentials: the fp32 MFMAs
 // do not overlap with vector instructions here (dK/dV at 16,000 nodes, 8
@@ -391,12 +393,15 @@ struct Fp32Ops {
 // S and dP contract the columns of two rows' pieces.  A lane's operand is 16
 // bytes of a row image, its 16-byte unit chosen by (operand number, g): the
 // MFMAs of a tile pair A and B operands so that, over the four g, every piece
-// product down to 2^-16 is there once; the smallest come first.
+// product down to 2^-16 is there once; the smallest come first, and the leading
+// products h h in the last lane groups of the last MFMA: all others meet in sums
+// 2^-8 of theirs, and S is rounded once at its own size (d = 8; with the h h in
+// the first group three more times: S off by up to 1.9 against 1.1 times 2^-24
+// sum |q k|, and at d = 16 2.2 against 1.2).
 // The dK/dV pass has the two matrices the other way round, and its S has to
 // round as the forward's did: exp(S - lse) with another last bit of S is off by
 // as much as S is large (at d = 16, 8 heads, 406 nodes dV's error was 3.2e-6,
-// with the forward's S 1.2e-6).  So the leading products h h come last, with none
-// beside them that weighs 2^-8, and their group is the same from both sides.
+// with the forward's S 1.2e-6).  The last group is the same from both sides.
 // With one piece per operand (d = 64) they are the row's two halves.
 template <int DH, int NP>
 struct Pairs {
@@ -414,7 +419,7 @@ struct Pairs<DH, 3> {
   // the N MFMAs, smallest products first
   static constexpr __host__ __device__ int a_of(int n) {
     if constexpr (DH == 8) return 1 - n;
-    else if constexpr (DH == 16) return n == 0;  // [h l] x [l h], [h m] x [m h], [h m] x [h m]
+    else if constexpr (DH == 16) return n == 0;  // [h l] x [l h], [m h] x [h m], [m h] x [m h]
     else {
       constexpr int a[6] = {2, 0, 1, 1, 0, 0};
       return DH == 64 ? 2 * a[n / 2] + n % 2 : a[n];
@@ -432,13 +437,13 @@ struct Pairs<DH, 3> {
   static __device__ __forceinline__ int unit(bool b, int k, int g) {
     constexpr int CB = col_blocks(DH);
     if constexpr (DH == 8) {
-      // [h m m l] x [h m l m] last, [h l h m] x [l h m h] first
-      const uint32_t units = k == 0 ? (b ? 0x1210u : 0x2110u) : (b ? 0x0102u : 0x1020u);
+      // [h l h m] x [l h m h] first, [l m m h] x [m l m h] last
+      const uint32_t units = k == 0 ? (b ? 0x0121u : 0x0112u) : (b ? 0x0102u : 0x1020u);
       return 16 * int(units >> (4 * g) & 15u);
     } else if constexpr (DH == 16) {
       const int hi = g >> 1;  // the second two lane groups
-      const int piece = b ? (k == 0 ? hi : hi ? 0 : 3 - k)  // hm / lh / mh
-                          : (k == 0 ? hi : 2 * hi);         // hm / hl
+      const int piece = b ? (k == 0 ? !hi : k == 1 ? 2 * !hi : hi)  // mh / lh / hm
+                          : (k == 0 ? !hi : 2 * hi);                // mh / hl
       return 16 * (piece * CB + (g & 1));
     } else if constexpr (DH == 64) {
       return 16 * ((k / 2) * CB + 4 * (k % 2) + g);
