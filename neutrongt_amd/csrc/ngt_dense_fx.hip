@@ -75,6 +75,7 @@ constexpr int kStep = 32;  // streamed rows per step of a wave (two tiles)
 constexpr int kPadRows = 64;  // the images' rows come in multiples of this
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+constexpr int kRun = 16;  // stages whose sums meet before they join a total (fwd_body)
 constexpr float kRebase = 5.5f;  // forward: P entries stay below e^5.5 (fp32 sums)
 constexpr float kHuge = 4.2535296e37f;  // 2^125: values past it take the fp32 MFMAs
 
@@ -654,6 +655,52 @@ struct FwdArgs {
 // moves only when some score exceeds it by more than kRebase, so after the
 // first step a wave rarely rescales; the column maximum over the lanes that
 // share a query is taken only then.
+//
+// At d = 8, where S is exact enough for the sums to show, a third level: the
+// stages of a run (1,024 keys) are added to each other and then to totals in
+// LDS, each lane's own, which cost no registers.  250 stages added one by one at
+// 16,000 keys had moved out, and through D = dO . out dQ: 8 heads, x 5.9e-7 ->
+// 3.9e-7 and dQ 2.2e-6 -> 1.3e-6 against float64 (vector kernels 7.5e-7 and
+// 2.0e-6); the pass with dropout 4,897 -> 4,911 us, in registers 4,960.
+constexpr bool run_totals(int dh) { return dh == 8; }
+template <int DH, int G>
+struct Totals {
+  static constexpr int BYTES = run_totals(DH) ? G * kBlock * 20 : 0;
+  char* lds;
+  float m[G];  // the base of the totals
+  bool any = false;
+  __device__ __forceinline__ f32x4& acc_of(int u) const {
+    return reinterpret_cast<f32x4*>(lds)[u * kBlock + tid_x()];
+  }
+  __device__ __forceinline__ float& l_of(int u) const {
+    return reinterpret_cast<float*>(lds + G * kBlock * 16)[u * kBlock + tid_x()];
+  }
+  // acc, l (base mu) += the totals
+  __device__ __forceinline__ void add_to(f32x4 (&acc)[G][out_tiles(DH)], float (&l)[G],
+                                         const float (&mu)[G]) const {
+    if (!any) return;
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const float f = m[u] == -INFINITY ? 0.f : exp_nat(m[u] - mu[u]);
+      acc[u][0] += acc_of(u) * f;
+      l[u] += l_of(u) * f;
+    }
+  }
+  // the totals += acc, l, which become zero
+  __device__ __forceinline__ void take(f32x4 (&acc)[G][out_tiles(DH)], float (&l)[G],
+                                       const float (&mu)[G]) {
+    add_to(acc, l, mu);
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      acc_of(u) = acc[u][0];
+      l_of(u) = l[u];
+      m[u] = mu[u];
+      l[u] = 0.f;
+    }
+    zero_acc(acc);
+    any = true;
+  }
+};
 template <class Ops, typename T, int DH, int G, bool DROP>
 __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z, char* lds) {
   constexpr int SB = Ops::SB, MT = out_tiles(DH);
@@ -685,6 +732,9 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     sk.load(a.k, k_begin, h, H);
     sv.load(a.v, k_begin, h, H);
   }
+  Totals<DH, G> tot;
+  tot.lds = lds + sk.BYTES + sv.BYTES;
+  int run = kRun;
   for (int kb = k_begin; kb < k_end; kb += SB) {
     __syncthreads();
     sk.store();
@@ -758,7 +808,13 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     add_acc(stage, acc);
 #pragma unroll
     for (int u = 0; u < G; ++u) l[u] += lst[u];
+    if constexpr (run_totals(DH))
+      if (--run == 0) {
+        run = kRun;
+        tot.take(acc, l, m);
+      }
   }
+  if constexpr (run_totals(DH)) tot.add_to(acc, l, m);
   Ops::finish(acc);
   const float ds = DROP && !Ops::SCALED ? a.drop_scale : 1.f;
 #pragma unroll
@@ -835,9 +891,10 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
   }
 }
 
-template <class Ops>
+template <class Ops, int DH, int G>
 constexpr int fwd_lds() {
-  return Ops::template Staged<true, false>::BYTES + Ops::template Staged<false, true>::BYTES;
+  return Ops::template Staged<true, false>::BYTES + Ops::template Staged<false, true>::BYTES +
+         Totals<DH, G>::BYTES;
 }
 
 // The forward and the column scores in one launch: grid z < n_split are
@@ -847,7 +904,7 @@ template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
   using P = PieceOps<T, DH, G>;
-  __shared__ __align__(16) char lds[max_of(fwd_lds<F>(), fwd_lds<P>())];
+  __shared__ __align__(16) char lds[max_of(fwd_lds<F, DH, G>(), fwd_lds<P, DH, G>())];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
   if (bx >= (z == a.n_split ? a.score_bx : a.fwd_bx)) return;  // block-uniform, before any barrier
   const bool plain = any_flag(a.q, a.k, a.v, h);

@@ -1,12 +1,14 @@
 """The fp32 dense kernels at the edges of their tiles: 16-row tiles, 32-row
 steps, 32/64-row stages, 64/128-row blocks, key splits, both tile counts per
 wave, every head dim, with and without dropout, against the restatement."""
+import math
+
 import pytest
 import torch
 
 from neutrongt_amd import dense_attention
 from oracle import attention as OA
-from tests._util import assert_parity
+from tests._util import assert_parity, relerr
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +85,24 @@ def test_piece_scores_are_rounded_once_at_their_size(monkeypatch, d, tiles):
     parts = 4.0 * q.double()[0, 0] * k.double()[:, 0]
     err = (ns.double().cpu() - parts.sum(-1).abs()).abs()
     assert (err <= 1.4 * 2.0 ** -24 * parts.abs().sum(-1)).all()
+
+
+@pytest.mark.parametrize("tiles,n_k", [(1, 16000), (2, 16000), (2, 1025), (2, 1024), (1, 2047)])
+def test_long_rows_are_summed_in_three_levels(monkeypatch, tiles, n_k):
+    """d = 8: out and dQ of queries over 16,000 keys in one split keep the error of
+    short rows (x 5.9e-7 and dQ 2.2e-6 with the stages added one by one); rows
+    around one run of stages."""
+    print(f"case dense f32 long rows tiles={tiles} n_k={n_k}", flush=True)
+    monkeypatch.setenv("NGT_DENSE_F32_TILES", str(tiles))
+    monkeypatch.setenv("NGT_DENSE_F32_FWD_SPLIT", "1")
+    n_q, H, d = 700, 2, 8
+    g = torch.Generator(device="cuda").manual_seed(n_k)
+    q, k, v, go = (torch.randn(n, H, d, device="cuda", generator=g) for n in (n_q, n_k, n_k, n_q))
+    t = [w.requires_grad_(True) for w in (q, k, v)]
+    x, _ = dense_attention(*t)
+    dq, = torch.autograd.grad(x, t[0], go)
+    Q, K, V = (w.detach().double().transpose(0, 1).contiguous().requires_grad_(True) for w in t)
+    y = torch.softmax((Q * math.sqrt(d)) @ K.transpose(1, 2).contiguous(), -1) @ V
+    gq, = torch.autograd.grad(y, Q, go.double().transpose(0, 1).contiguous())
+    assert relerr(x.detach(), y.detach().transpose(0, 1)) < 5e-7
+    assert relerr(dq, gq.transpose(0, 1)) < 1.7e-6
