@@ -75,7 +75,7 @@ constexpr int kStep = 32;  // streamed rows per step of a wave (two tiles)
 constexpr int kPadRows = 64;  // the images' rows come in multiples of this
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-constexpr int kRun = 16;  // stages whose sums meet before they join a total (fwd_body)
+constexpr int kRun = 16;  // stages whose sums meet before they join a total
 constexpr float kRebase = 5.5f;  // forward: P entries stay below e^5.5 (fp32 sums)
 constexpr float kHuge = 4.2535296e37f;  // 2^125: values past it take the fp32 MFMAs
 
@@ -841,8 +841,9 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
 }
 
 // Column scores part[h][j] = sum_i |S[h, i, j]|: rows = queries (staged),
-// lanes = keys.  Each stage's sum is added to the total, so a long column is
-// summed in two levels.
+// lanes = keys.  A long column is summed in three levels: the stages of a run of
+// kRun are added to each other before they join the total (8,000 queries, 4 heads
+// of 32: 7.3e-8 -> 4.7e-8 of float64).
 template <class Ops, int DH, int G>
 __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, char* lds) {
   constexpr int SB = Ops::SB;
@@ -852,16 +853,17 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
   const int n_q = a.q.n;
   int kj[G];
   typename Ops::Rows kf;
-  float sum[G];
+  float sum[G], runs[G];
 #pragma unroll
   for (int u = 0; u < G; ++u) {
     kj[u] = bx * block_rows(G) + (wave * G + u) * kT + l16;
-    sum[u] = 0.f;
+    sum[u] = runs[u] = 0.f;
     Ops::load_rows(kf, u, a.k, kj[u], h, a.H, g);
   }
   typename Ops::template Staged<true, false> sq;
   sq.lds = reinterpret_cast<decltype(sq.lds)>(lds);
   sq.load(a.q, 0, h, a.H);
+  int run = kRun;
   for (int qb = 0; qb < n_q; qb += SB) {
     __syncthreads();
     sq.store();
@@ -882,7 +884,15 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
           for (int i = 0; i < 4; ++i) st[u] += fabsf(s[t][u][i]);
     }
 #pragma unroll
-    for (int u = 0; u < G; ++u) sum[u] += st[u];
+    for (int u = 0; u < G; ++u) runs[u] += st[u];
+    if (--run == 0 || qb + SB >= n_q) {
+      run = kRun;
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        sum[u] += runs[u];
+        runs[u] = 0.f;
+      }
+    }
   }
 #pragma unroll
   for (int u = 0; u < G; ++u) {
