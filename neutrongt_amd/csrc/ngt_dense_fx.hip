@@ -45,8 +45,11 @@
 // Outputs come out transposed, 4 consecutive columns of a lane's row.
 //
 // Pieces of an infinity or a NaN would turn products with zero pieces into
-// NaN, so a head whose inputs hold one (or a value past 2^125) runs the same
-// kernels' other body, with v_mfma_f32_16x16x4_f32: plain fp32 FMA chains.
+// NaN, and below 2^-110 the third piece of an fp32 value is a bf16 subnormal
+// that no longer holds all its bits (below 2^-126 the second).  So a head whose
+// inputs hold such a value or one past 2^125, and a backward pass whose dO or v
+// is so small that dS would be there, runs the same kernels' other body, with
+// v_mfma_f32_16x16x4_f32: plain fp32 FMA chains.
 #include "ngt_common.h"
 
 #include <math.h>
@@ -77,7 +80,9 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int kRun = 16;  // stages whose sums meet before they join a total
 constexpr float kRebase = 5.5f;  // forward: P entries stay below e^5.5 (fp32 sums)
-constexpr float kHuge = 4.2535296e37f;  // 2^125: values past it take the fp32 MFMAs
+constexpr float kHuge = 4.2535296e37f;   // 2^125: values past it take the fp32 MFMAs,
+constexpr float kTiny = 7.7037198e-34f;  // 2^-110: and values below it (but zero)
+constexpr float kFaint = 9.0949470e-13f; // 2^-40: see backward_plain
 
 // Rows (queries or keys) a block owns with G tiles per wave.
 constexpr int block_rows(int G) { return kWaves * kT * G; }
@@ -178,12 +183,14 @@ struct Mat {
   const void* x;        // [n, H, d] of the element type
   const char* row_img;  // [H][padded(n)][row_bytes]
   const char* t_img;    // [H][padded(n) / 32][t_bytes]
-  const uint32_t* flag; // [H][padded(n) / 32]: nonzero where a value takes the fp32 body
+  const uint32_t* flag; // [H][padded(n) / 32]: what the step's values are (k...Value)
   int32_t n;
   float scale;          // of x (in the images of fp32 inputs already)
 };
 
 // -------------------------------------------------------------- preparation
+constexpr uint32_t kSpecialValue = 1u;  // some value has no three pieces
+constexpr uint32_t kNonzeroValue = 2u, kPlainValue = 4u;  // some value is not 0, not below 2^-40
 struct PrepJob {
   const void* x;
   char* row_img;
@@ -206,20 +213,27 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
   const int n_pad = padded(job.n);
   if (step * kStep >= n_pad) return;
   __shared__ float xs[kStep][DH + 1];
-  int bad = 0;
+  constexpr int NP = pieces<T>();
+  uint32_t mark = 0u;
   for (int e = tid_x(); e < kStep * DH; e += kBlock) {
     const int r = e / DH, c = e - r * DH;
     const int64_t row = int64_t(step) * kStep + r;
     float v = 0.f;
     if (row < job.n) v = elem<T>::load(static_cast<const T*>(job.x) + (row * H + h) * DH + c);
-    if constexpr (pieces<T>() == 3) v *= job.scale;
+    if constexpr (NP == 3) v *= job.scale;
     xs[r][c] = v;
-    // (an unordered compare on the bits: this file does not honour NaNs)
-    bad |= (__float_as_uint(v) & 0x7fffffffu) > __float_as_uint(kHuge);
+    // (compares on the bits: this file does not honour NaNs)
+    const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
+    if (u > __float_as_uint(kHuge) || (NP == 3 && u != 0u && u < __float_as_uint(kTiny)))
+      mark |= kSpecialValue;
+    if (u != 0u) mark |= kNonzeroValue;
+    if (u >= __float_as_uint(kFaint)) mark |= kPlainValue;
   }
-  bad = __syncthreads_or(bad);
-  if (tid_x() == 0) job.flag[int64_t(h) * (n_pad / kStep) + step] = bad ? 1u : 0u;
-  constexpr int NP = pieces<T>();
+  uint32_t word = 0u;
+#pragma unroll
+  for (uint32_t bit = kSpecialValue; bit <= kPlainValue; bit *= 2)
+    if (__syncthreads_or(int(mark & bit))) word |= bit;
+  if (tid_x() == 0) job.flag[int64_t(h) * (n_pad / kStep) + step] = word;
   constexpr int NB = col_blocks(DH);
   for (int e = tid_x(); e < kStep * NB; e += kBlock) {
     const int r = e / NB, cb = e - r * NB;
@@ -255,18 +269,32 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
   }
 }
 
-// Whether any step of head h of these matrices takes the fp32 body (the same
-// answer in every thread of the block).  Without images (few_scores) all do.
-__device__ __forceinline__ bool any_flag(const Mat& a, const Mat& b, const Mat& c, int h) {
+// This thread's share of the marks of head h of a matrix.
+__device__ __forceinline__ uint32_t marks(const Mat& m, int h) {
+  const int steps = padded(m.n) / kStep;
+  uint32_t w = 0u;
+  for (int t = tid_x(); t < steps; t += kBlock) w |= m.flag[int64_t(h) * steps + t];
+  return w;
+}
+// Whether head h of these matrices takes the fp32 body (the same answer in every
+// thread of the block).  Without images (few_scores) all do.
+__device__ __forceinline__ bool any_special(const Mat& a, const Mat& b, const Mat& c, int h) {
   if (!a.flag) return true;
-  int bad = 0;
-  const Mat* m[3] = {&a, &b, &c};
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const int steps = padded(m[i]->n) / kStep;
-    for (int t = tid_x(); t < steps; t += kBlock) bad |= int(m[i]->flag[int64_t(h) * steps + t]);
-  }
-  return __syncthreads_or(bad) != 0;
+  return __syncthreads_or(int((marks(a, h) | marks(b, h) | marks(c, h)) & kSpecialValue)) != 0;
+}
+// The same for the backward, whose dS = p (dO . v - D) is split into pieces too:
+// with dO or v below 2^-40 everywhere (zeros alone do no harm) it could lie below
+// 2^-110 where it counts.  With one value of each past that, the largest dS lies
+// past 2^-80 p and what the pieces drop is below 2^-133.
+__device__ __forceinline__ bool backward_plain(const Mat& q, const Mat& k, const Mat& v,
+                                               const Mat& g, int h) {
+  if (any_special(q, k, v, h)) return true;
+  const uint32_t mg = marks(g, h), mv = marks(v, h);
+  if (__syncthreads_or(int(mg & kSpecialValue))) return true;
+  auto faint = [](uint32_t m) {
+    return __syncthreads_or(int(m & kNonzeroValue)) && !__syncthreads_or(int(m & kPlainValue));
+  };
+  return faint(mg) || faint(mv);
 }
 
 // ------------------------------------------------------- fp32 MFMA products
@@ -917,7 +945,7 @@ __global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
   __shared__ __align__(16) char lds[max_of(fwd_lds<F, DH, G>(), fwd_lds<P, DH, G>())];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
   if (bx >= (z == a.n_split ? a.score_bx : a.fwd_bx)) return;  // block-uniform, before any barrier
-  const bool plain = any_flag(a.q, a.k, a.v, h);
+  const bool plain = any_special(a.q, a.k, a.v, h);
   if (z == a.n_split) {
     if (plain)
       scores_body<F, DH, G>(a, bx, h, lds);
@@ -1071,7 +1099,7 @@ __global__ __launch_bounds__(kBlock) void k_fx_bwd_q(const BwdArgs a) {
   using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(bwd_q_lds<F>(), bwd_q_lds<P>())];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
-  if (any_flag(a.q, a.k, a.v, h) || any_flag(a.g, a.g, a.g, h))
+  if (backward_plain(a.q, a.k, a.v, a.g, h))
     bwd_q_body<F, T, DH, G, DROP>(a, bx, h, z, lds);
   else
     bwd_q_body<P, T, DH, G, DROP>(a, bx, h, z, lds);
@@ -1214,7 +1242,7 @@ __global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
                int64_t(a.comb_bx) * a.H);
     return;
   }
-  if (any_flag(a.q, a.k, a.v, h) || any_flag(a.g, a.g, a.g, h))
+  if (backward_plain(a.q, a.k, a.v, a.g, h))
     bwd_kv_body<F, T, DH, G, DROP>(a, bx, h, lds, ls, ds);
   else
     bwd_kv_body<P, T, DH, G, DROP>(a, bx, h, lds, ls, ds);

@@ -122,3 +122,34 @@ def test_node_scores_of_many_queries(monkeypatch, d, n_q):
     ref = sum(((q[:, h].double() * math.sqrt(d)) @ k[:, h].double().t().contiguous()).abs().sum(0)
               for h in range(4)) / 4
     assert relerr(ns, ref) < 6.2e-8
+
+
+@pytest.mark.parametrize("d", [8, 16, 24, 32, 64])
+@pytest.mark.parametrize("shift", [dict(q=-116, k=100), dict(k=-116, q=100), dict(v=-116, go=100),
+                                   dict(go=-116), dict(go=-60, v=-58), dict(v=-30, go=-35)])
+def test_small_operands_keep_their_bits(monkeypatch, d, shift):
+    """Operands scaled by powers of two: below 2^-110 a value's third bf16 piece is
+    a subnormal, and dS = p dO v may be there where dO and v are not.  Such heads
+    take the fp32 products; the error is that of operands of ordinary size."""
+    print(f"case dense f32 small operands d={d} {shift}", flush=True)
+    monkeypatch.setenv("NGT_DENSE_F32_TILES", "2")
+    g = torch.Generator(device="cuda").manual_seed(d)
+    t = {n: torch.randn(m, 2, d, device="cuda", generator=g)
+         for n, m in (("q", 90), ("k", 170), ("v", 170), ("go", 90))}
+    t["q"] *= 0.3
+    scale = math.sqrt(d)
+    for n, e in shift.items():
+        t[n] = torch.ldexp(t[n], torch.tensor(e, device="cuda"))
+    if "k" in shift:
+        scale *= 2.0 ** 16  # the logits of the unscaled operands
+    w = [t[n].requires_grad_(True) for n in ("q", "k", "v")]
+    x, ns = dense_attention(*w, scale=scale)
+    got = (x.detach(), ns, *torch.autograd.grad(x, w, t["go"]))
+    Q, K, V = (a.detach().double().transpose(0, 1).contiguous().requires_grad_(True) for a in w)
+    S = (Q * scale) @ K.transpose(1, 2).contiguous()
+    y = torch.softmax(S, -1) @ V
+    ref = torch.autograd.grad(y, (Q, K, V), t["go"].double().transpose(0, 1).contiguous())
+    ref = (y.detach().transpose(0, 1), S.detach().abs().sum(1).mean(0),
+           *(r.transpose(0, 1) for r in ref))
+    for name, a, b in zip(("x", "node_scores", "dq", "dk", "dv"), got, ref):
+        assert relerr(a, b) < 3e-7 * d + 1e-6, name
