@@ -688,7 +688,7 @@ class CoreAttention(nn.Module):
             k = torch.cat([k, kv_ext[0].detach().to(k.dtype).reshape(1, -1, *k.shape[2:])], dim=1)
             v = torch.cat([v, kv_ext[1].detach().to(v.dtype).reshape(1, -1, *v.shape[2:])], dim=1)
         if attn_type == "sparse":
-            if type(self).sparse_attention_bias is CoreAttention.sparse_attention_bias:
+            if getattr(self.sparse_attention_bias, "__func__", None) is _SPARSE_ATTENTION_BIAS:
                 x, score = _sparse(q, k, v, edge_index, self.num_heads, self.scale,
                                    self.adjacency_cache, CLAMP_LO, CLAMP_HI, EPS, kv_ext,
                                    attn_bias, interleave_grads, True)
@@ -713,6 +713,11 @@ class CoreAttention(nn.Module):
         if x.dim() != 3 or x.shape[:2] != (batch_size, s_len):
             x = x.view(batch_size, s_len, -1)
         return x, score
+
+
+# forward calls the core behind this method itself (no view of its output), and
+# the method where a subclass, the instance or a patch has put another
+_SPARSE_ATTENTION_BIAS = CoreAttention.sparse_attention_bias
 
 
 def install(model: nn.Module, cache: AdjacencyCache = None) -> int:
