@@ -91,6 +91,8 @@ class _Attention(nn.Module):
         self.local_attn = CoreAttention(hidden_size, attention_dropout_rate, num_heads)
 
     def attend(self, x, edge_index, attn_type, kv_cache):
+        if x.dim() != 3:
+            raise ValueError(f"x must be [b, N, hidden], got {tuple(x.shape)}")
         H, d = self.num_heads, self.att_size
         lins = (self.linear_q, self.linear_k, self.linear_v)
         # one projection node, and the sparse core hands back dQ, dK, dV as

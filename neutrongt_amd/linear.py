@@ -293,7 +293,9 @@ def project(x: torch.Tensor, *lins: nn.Linear, heads: int = 0):
         ys = _ProjectionGroupFn.apply(x, *params)
     else:
         ys = tuple(l(x) for l in lins)
-    return tuple(y.view(*y.shape[:-1], heads, -1) for y in ys) if heads else ys
+    if not heads:
+        return ys
+    return tuple(y.view(*y.shape[:-1], heads, y.shape[-1] // heads) for y in ys)
 
 
 class WgradLinear(nn.Linear):
