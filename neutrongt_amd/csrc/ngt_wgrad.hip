@@ -281,6 +281,9 @@ constexpr int kBlocks = 512;
 constexpr int64_t kMaxChain = 2560;
 inline int64_t min_stages(bool wide, int64_t tiles) { return !wide ? 1 : tiles < 32 ? 2 : 4; }
 
+// A launch holds fewer than 2^32 threads.
+constexpr int64_t kMaxGrid = (int64_t(1) << 32) / kBlock - 8;
+
 struct Plan {
   bool wide;
   int32_t tiles_m, tiles_n, splits;
@@ -296,7 +299,8 @@ int make_plan(const char* fn, int64_t n_rows, int32_t n_out, int32_t n_in, Plan*
   p->tiles_m = (n_out + t - 1) / t;
   p->tiles_n = (n_in + t - 1) / t;
   const int64_t tiles = int64_t(p->tiles_m) * p->tiles_n;
-  if (tiles > (1 << 20) || n_rows > (int64_t(1) << 31))
+  const int64_t sums = (int64_t(n_out) * n_in + kRedCols - 1) / kRedCols + n_out / kRedCols + 1;
+  if (tiles > (1 << 20) || n_rows > (int64_t(1) << 31) || sums > kMaxGrid)
     return set_error(NGT_ERR_UNSUPPORTED, "%s: %lld rows, %d x %d outputs exceed the grid", fn,
                      static_cast<long long>(n_rows), n_out, n_in);
   const int64_t kb = stage_rows(t);
@@ -307,7 +311,7 @@ int make_plan(const char* fn, int64_t n_rows, int32_t n_out, int32_t n_in, Plan*
   if (splits < 1) splits = 1;
   const int64_t per = (stages + splits - 1) / splits;
   p->rows_per_split = per * kb;
-  if (per > 0 && (stages + per - 1) / per * tiles > (1 << 30))
+  if (per > 0 && (stages + per - 1) / per * tiles > kMaxGrid)
     return set_error(NGT_ERR_UNSUPPORTED, "%s: %lld rows, %d x %d outputs exceed the grid", fn,
                      static_cast<long long>(n_rows), n_out, n_in);
   p->splits = per > 0 ? static_cast<int32_t>((stages + per - 1) / per) : 0;
@@ -379,9 +383,6 @@ extern "C" int ngt_wgrad_bf16(const void* x, const void* dy, int64_t n_rows, int
   const int64_t n = int64_t(n_out) * n_in;
   const int64_t blocks_w = (n + kRedCols - 1) / kRedCols;
   const int64_t blocks_b = db ? (n_out + kRedCols - 1) / kRedCols : 0;
-  if (blocks_w + blocks_b > INT32_MAX)
-    return set_error(NGT_ERR_UNSUPPORTED, "ngt_wgrad_bf16: %d x %d outputs exceed the grid", n_out,
-                     n_in);
   const bool vec = n % 4 == 0 && n_out % 4 == 0;
   const dim3 grid(static_cast<unsigned>(blocks_w + blocks_b));
   if (vec)

@@ -256,3 +256,14 @@ def test_dense_bias_head_chunk_follows_the_budget():
     assert A.dense_bias_head_chunk(32, 4000, 4000, budget=1 << 30) == 3
     # and the softmax launches stay within 2^24 (head, query) rows
     assert A.dense_bias_head_chunk(64, 1 << 20, 1, budget=1 << 60) == 16
+
+
+def test_wgrad_refuses_launches_past_the_grid():
+    """2^32 threads are more than a launch holds: refused with a plan's sizes, not
+    by the launch."""
+    lib = _lib.load()
+    nb = C.c_size_t()
+    ok = lambda K, o, i: lib.ngt_wgrad_workspace_bytes(K, o, i, C.byref(nb))
+    assert ok(10007, 2304, 768) == 0 and ok(1 << 31, 8, 8) == 0 and ok(0, 32768, 32768 - 64) == 0
+    assert ok(1 << 31, 2048, 2048) == 2 and b"exceed the grid" in lib.ngt_last_error()
+    assert ok(16, 32768, 32768) == 2 and b"exceed the grid" in lib.ngt_last_error()
