@@ -672,6 +672,8 @@ int ngt_chunk_sum_f32(const float* in, int32_t n_chunks, int64_t n, float* out, 
  * bias, NeutronGT/models/graphormer_dist_node_level.py:130-206.
  */
 int ngt_wgrad_workspace_bytes(int64_t n_rows, int32_t n_out, int32_t n_in, size_t* bytes);
+/* 1 where ngt_wgrad_bf16 is faster than library GEMMs over row chunks, else 0. */
+int ngt_wgrad_pays(int64_t n_rows, int64_t n_out, int64_t n_in);
 int ngt_wgrad_bf16(const void* x, const void* dy, int64_t n_rows, int32_t n_out, int32_t n_in,
                    float* dw, float* db, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -135,6 +135,7 @@ SIGNATURES = {
     "ngt_colsum_bf16": [_vp, _i64, _i32, _vp, _vp, _sz, _vp],
     "ngt_chunk_sum_f32": [_vp, _i32, _i64, _vp, _vp],
     "ngt_wgrad_workspace_bytes": [_i64, _i32, _i32, _psz],
+    "ngt_wgrad_pays": [_i64, _i64, _i64],
     "ngt_wgrad_bf16": [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _sz, _vp],
     "ngt_related_workspace_bytes": [_i32, _i32, _psz],
     "ngt_merge_related_nodes": [_vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _sz, _vp],

@@ -51,6 +51,7 @@ decltype(&ngt_colsum_workspace_bytes) g_colsum_ws = nullptr;
 decltype(&ngt_colsum_bf16) g_colsum = nullptr;
 decltype(&ngt_chunk_sum_f32) g_chunk_sum = nullptr;
 decltype(&ngt_wgrad_workspace_bytes) g_wgrad_ws = nullptr;
+decltype(&ngt_wgrad_pays) g_wgrad_pays = nullptr;
 decltype(&ngt_wgrad_bf16) g_wgrad = nullptr;
 decltype(&ngt_layernorm_fwd) g_ln_fwd = nullptr;
 decltype(&ngt_layernorm_bwd_workspace_bytes) g_ln_bwd_ws = nullptr;
@@ -229,9 +230,8 @@ struct NoAutocast {
   c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
 };
 
-constexpr int64_t kChunk = 2048;  // as the limits of linear.py
+constexpr int64_t kChunk = 2048;  // as _CHUNK and _MAX_SPLITS of linear.py
 constexpr int64_t kMaxSplits = 16;
-constexpr int64_t kFusedProducts = 18000000000, kFusedRows = 3000, kFusedOutputs = 1000000;
 
 // fp32 column sums of a contiguous bf16 [K, n] matrix
 Tensor colsum(const Tensor& dy) {
@@ -265,16 +265,15 @@ Tensor library_weight_grad(const Tensor& x, const Tensor& dy) {
 }
 
 // dw = dY^T X and, where wanted, db = column sums of dY, in fp32 from
-// contiguous bf16 rows (_grads of linear.py; its _fused explains the rule).  x
-// may be undefined where dw is not wanted.
+// contiguous bf16 rows (_grads of linear.py).  x may be undefined where dw is not
+// wanted.
 void linear_grads(const Tensor& x, const Tensor& dy, Tensor* dw, Tensor* db) {
   if (!dw) {
     if (db) *db = colsum(dy);
     return;
   }
   const int64_t K = x.size(0), n_in = x.size(1), n_out = dy.size(1);
-  if (at::GradMode::is_enabled() || n_in == 0 || n_out == 0 ||
-      K * n_in * n_out > kFusedProducts || (K < kFusedRows && n_in * n_out >= kFusedOutputs)) {
+  if (at::GradMode::is_enabled() || !g_wgrad_pays(K, n_out, n_in)) {
     *dw = library_weight_grad(x, dy);
     if (db) *db = colsum(dy);
     return;
@@ -566,6 +565,7 @@ void init(const std::map<std::string, int64_t>& addr) {
   entry(g_colsum, addr, "ngt_colsum_bf16");
   entry(g_chunk_sum, addr, "ngt_chunk_sum_f32");
   entry(g_wgrad_ws, addr, "ngt_wgrad_workspace_bytes");
+  entry(g_wgrad_pays, addr, "ngt_wgrad_pays");
   entry(g_wgrad, addr, "ngt_wgrad_bf16");
   entry(g_ln_fwd, addr, "ngt_layernorm_fwd");
   entry(g_ln_bwd_ws, addr, "ngt_layernorm_bwd_workspace_bytes");

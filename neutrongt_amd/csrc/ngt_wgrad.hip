@@ -340,6 +340,42 @@ extern "C" int ngt_wgrad_workspace_bytes(int64_t n_rows, int32_t n_out, int32_t 
   return NGT_OK;
 }
 
+// Where k_wgrad beats the library's GEMMs over row chunks, chunk sum and column
+// sum (us with the bias, this / library, rows x n_out x n_in).
+// Products: the library's large tiles win once a second round of blocks is under
+// way, which the 2,560-row chains ask for: 30,000 x 768 x 768 62 / 87, 32,768 67 / 66,
+// 40,000 109 / 85; 896 x 1,024 outputs at 20,000 rows 66 / 92; 65,536 x 512 x 512
+// 61 / 68, 100,000 112 / 105.  Between 1 and 2 M outputs its tiles divide the
+// chip badly and the line is further out: 2,304 x 768 at 10,007 rows 75 / 93,
+// 12,000 111 / 109, 16,000 111 / 125, 20,000 133 / 136, 24,000 165 / 145; 1,536 x
+// 768 at 20,000 114 / 119, 32,768 138 / 134; 1,024 x 1,024 at 24,000 106 / 124,
+// 32,768 127 / 97.  3,072 x 768 at 7,600 82 / 88, 10,000 119 / 86; above, the
+// library's tiles fill it: 3,072 x 1,024 at 5,700 rows 98 / 69, 2,304 x 2,304
+// at 3,000 96 / 63.
+// Few rows: the partials cost more than the products: 896 x 1,024 at 1,000 rows
+// 23 / 21, 1,024 x 1,024 24 / 21 and at 2,000 28 / 29, 768 x 768 at 500 16 / 16.
+// Narrow on one side, wide on the other, and many rows: a tile's unused columns
+// cost as much as used ones while the rows come from memory: 47 x 768 at 32,768
+// rows 44 / 67, 131,072 155 / 138; 48 x 2,048 at 32,768 58 / 36; 48 x 256 at
+// 524,288 172 / 222.  Fuller tiles keep longer: 64 x 768 at 131,072 57 / 116, 64 x
+// 2,048 152 / 124; 100 x 768 99 / 147, 100 x 1,024 161 / 138.
+// Over 166 shapes of 8 to 2,600 columns the choice costs more than 10 % against
+// the library in one (2,308 x 191 at 35,131 rows, 260 / 195).
+extern "C" int ngt_wgrad_pays(int64_t n_rows, int64_t n_out, int64_t n_in) {
+  if (n_rows < 0 || n_out < 1 || n_in < 1 || n_out > 65536 || n_in > 65536 ||
+      n_rows > (int64_t(1) << 31))
+    return 0;
+  const int64_t outputs = n_out * n_in;
+  const int64_t narrow = n_out < n_in ? n_out : n_in, wide = n_out < n_in ? n_in : n_out;
+  const int64_t most = outputs >= 1000000 && outputs < 2000000 ? 32000000000 : 18000000000;
+  if (outputs > 2500000 || n_rows > most / outputs) return 0;
+  if (n_rows < 2000 && outputs > 750000) return 0;
+  const int64_t span = narrow < 64 ? 60000000 : narrow == 64 ? 150000000 : 120000000;
+  if ((narrow <= 64 || (narrow < 256 && narrow % 64)) && wide > 256 && n_rows * wide > span)
+    return 0;
+  return 1;
+}
+
 extern "C" int ngt_wgrad_bf16(const void* x, const void* dy, int64_t n_rows, int32_t n_out,
                               int32_t n_in, float* dw, float* db, void* workspace,
                               size_t workspace_bytes, void* stream) {

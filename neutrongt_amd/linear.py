@@ -32,8 +32,6 @@ from . import _lib
 
 _CHUNK = 2048      # rows per split of the library's weight-gradient reduction
 _MAX_SPLITS = 16   # 16 x 2048 rows measured fastest for 32,768 x 768 x 768
-_FUSED_PRODUCTS = 18_000_000_000  # the limits of _fused
-_FUSED_ROWS, _FUSED_OUTPUTS = 3000, 1_000_000
 
 
 def colsum_bf16(dy: torch.Tensor) -> torch.Tensor:
@@ -106,16 +104,11 @@ def _library_weight_grad(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
 
 
 def _fused(x: torch.Tensor, dy: torch.Tensor) -> bool:
-    """Whether linear_grads takes these rows (a gradient that will itself be
-    differentiated is torch's).  The library's large GEMM tiles are the faster
-    from about 1.8e10 products on (32,768 x 768 x 768 with the bias 65.8 us
-    against 66 to 72, 32,768 x 2,304 x 768 168 against 181; but 10,007 x 2,304 x
-    768 92 against 73), and for a million outputs over few rows, where the
-    partials weigh most (1,000 x 2,304 x 768 25.8 against 32, 3,000 rows 40.7
-    against 37.6)."""
-    rows, outputs = x.shape[0], x.shape[1] * dy.shape[1]
-    return (not torch.is_grad_enabled() and outputs > 0 and rows * outputs <= _FUSED_PRODUCTS
-            and (rows >= _FUSED_ROWS or outputs < _FUSED_OUTPUTS))
+    """Whether linear_grads takes these rows: where it is the faster (the rule is
+    ngt_wgrad_pays; the C++ nodes ask it too), and not for a gradient that will
+    itself be differentiated, which is torch's."""
+    return (not torch.is_grad_enabled()
+            and bool(_lib.load().ngt_wgrad_pays(x.shape[0], dy.shape[1], x.shape[1])))
 
 
 def _grads(x2: torch.Tensor, g2: torch.Tensor, want_w: bool, want_b: bool):

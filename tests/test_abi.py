@@ -267,3 +267,17 @@ def test_wgrad_refuses_launches_past_the_grid():
     assert ok(10007, 2304, 768) == 0 and ok(1 << 31, 8, 8) == 0 and ok(0, 32768, 32768 - 64) == 0
     assert ok(1 << 31, 2048, 2048) == 2 and b"exceed the grid" in lib.ngt_last_error()
     assert ok(16, 32768, 32768) == 2 and b"exceed the grid" in lib.ngt_last_error()
+
+
+@pytest.mark.parametrize("rows,n_out,n_in,pays", [
+    (10584, 64, 64, 1), (10007, 2304, 768, 1), (20000, 2304, 768, 0), (13000, 2304, 768, 1),
+    (32768, 2304, 768, 0), (30000, 768, 768, 1), (32768, 768, 768, 0), (5700, 3072, 1024, 0),
+    (1000, 896, 1024, 0), (32768, 47, 768, 1), (131072, 47, 768, 0), (524288, 48, 256, 1),
+    (131072, 64, 768, 1), (131072, 2048, 64, 0), (131072, 100, 768, 1), (131072, 1024, 100, 0), (0, 8, 8, 1), (8, 0, 8, 0), (8, 8, 0, 0),
+    ((1 << 31) + 1, 1, 1, 0), (-1, 8, 8, 0), (1 << 62, 1 << 40, 1 << 40, 0)])
+def test_wgrad_rule(rows, n_out, n_in, pays):
+    """The measured sides of the rule, and sizes that the kernel does not take."""
+    lib = _lib.load()
+    assert lib.ngt_wgrad_pays(rows, n_out, n_in) == pays
+    if pays:
+        assert lib.ngt_wgrad_workspace_bytes(rows, n_out, n_in, C.byref(C.c_size_t())) == 0

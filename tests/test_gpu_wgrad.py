@@ -6,7 +6,9 @@ at most 2,560 terms in a chain and then the splits, below 1e-6 in the 2-norm."""
 import pytest
 import torch
 
-from neutrongt_amd.linear import _fused, _grads, _library_weight_grad, colsum_bf16, linear_grads
+from neutrongt_amd import _lib
+from neutrongt_amd.linear import (WgradLinear, _fused, _grads, _library_weight_grad, colsum_bf16,
+                                  linear_grads)
 from tests._util import relerr
 
 pytestmark = pytest.mark.gpu
@@ -58,8 +60,10 @@ def test_infinities_and_nan_stay_in_their_row_and_column():
     assert db[:46].eq(K).all() and db[46].isnan()
 
 
-@pytest.mark.parametrize("K,n_out,n_in,fused", [(2999, 1536, 768, False), (3000, 1536, 768, True),
-                                                (1000, 768, 768, True), (32768, 768, 768, False)])
+@pytest.mark.parametrize("K,n_out,n_in,fused", [
+    (1999, 1536, 768, False), (2000, 1536, 768, True), (1000, 768, 768, True),
+    (32768, 768, 768, False), (16000, 2304, 768, True), (24000, 2304, 768, False),
+    (4000, 3072, 1024, False), (32768, 47, 768, True), (131072, 47, 768, False)])
 def test_both_routes_agree_at_the_rule(K, n_out, n_in, fused):
     print(f"case wgrad rule {K} {n_out} {n_in}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(K)
@@ -70,3 +74,10 @@ def test_both_routes_agree_at_the_rule(K, n_out, n_in, fused):
         dw, db = _grads(x, dy, True, True)
         assert relerr(dw, _library_weight_grad(x, dy).double()) < 2e-6
         assert relerr(db, colsum_bf16(dy).double()) < 2e-6
+    # the layer's node takes the same route
+    lin = WgradLinear(n_in, n_out).cuda()
+    assert _lib.node_ext() is not None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = lin(x)
+    gw, gb = torch.autograd.grad(y, (lin.weight, lin.bias), dy)
+    assert torch.equal(gw, dw) and torch.equal(gb, db)
