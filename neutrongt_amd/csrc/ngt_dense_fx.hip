@@ -1402,10 +1402,15 @@ MfSplit fx_dq_split(int n_q, int n_k, int H, int d) {
 
 // Few scores: the fp32 bodies alone, on the matrices as they are.  Their MFMAs
 // take 8 times the cycles, but up to here the two preparation launches and the
-// pieces' splits cost more.  Forward and backward in us, pieces / fp32: 8 heads
-// of 8, 406 nodes 61 / 36, 2,048 nodes 170 / 144; 8 of 16, 2,048 nodes 204 / 193;
-// 32 of 24, 1,000 nodes 279 / 240, 2,048 nodes 942 / 1,103; 8 of 64, 406 nodes
-// 127 / 115, 1,000 nodes 214 / 236.  NGT_DENSE_F32_TILES asks for the pieces.
+// pieces' splits cost more.  Forward and backward in us, pieces / fp32 (in brackets
+// with dropout): 8 heads of 8, 406 nodes 61 / 36, 2^25 scores (2,048 nodes) 191 /
+// 143 (205 / 170); 8 of 16, 2^25 205 / 187 (220 / 220), 2^26 336 / 346; 32 of 24,
+// 2^25 285 / 234, 2^27 976 / 1,102; 8 of 32, 2^25 305 / 272 (341 / 355), 4 of 32
+// 394 / 415 (398 / 451); 8 of 64, 2^22 179 / 172 (180 / 180), 2^23 232 / 241.  At
+// d = 8 and 24 the times cross one power later (2^26 272 / 225 and 463 / 404), but
+// the pieces are the more exact there (8 heads of 8, 2,500 nodes: x 3.1e-7 against
+// 5.2e-7), so the line stays at 2^25.
+// NGT_DENSE_F32_TILES asks for the pieces.
 bool few_scores(int dtype, int n_q, int n_k, int H, int d) {
   return dtype == NGT_F32 && !getenv("NGT_DENSE_F32_TILES") &&
          int64_t(n_q) * n_k <= (int64_t(1) << (d == 64 ? 22 : 25)) / std::max(H, 1);
