@@ -25,7 +25,7 @@
 // same in bf16 (one piece per operand) 1,570 / 5,870 / 2,970 -> 275 / 635 / 290.
 //
 // A preparation kernel (k_fx_prep) writes the pieces of q * scale, k, v and dO
-// once per call, in the layout the LDS stages have:
+// once per call, each matrix in the images that the pass reads:
 //   row image: per row 3 pieces x d / 8 blocks of 8 columns (16 bytes each),
 //     read as A and B operands of S and dP;
 //   transposed image: per 32 rows, one line per (piece, column) with the 32
@@ -193,8 +193,7 @@ constexpr uint32_t kSpecialValue = 1u;  // some value has no three pieces
 constexpr uint32_t kNonzeroValue = 2u, kPlainValue = 4u;  // some value is not 0, not below 2^-40
 struct PrepJob {
   const void* x;
-  char* row_img;
-  char* t_img;  // null: not wanted
+  char *row_img, *t_img;  // null: not wanted
   uint32_t* flag;
   int32_t n;
   float scale;
@@ -235,7 +234,7 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
     if (__syncthreads_or(int(mark & bit))) word |= bit;
   if (tid_x() == 0) job.flag[int64_t(h) * (n_pad / kStep) + step] = word;
   constexpr int NB = col_blocks(DH);
-  for (int e = tid_x(); e < kStep * NB; e += kBlock) {
+  for (int e = tid_x(); job.row_img && e < kStep * NB; e += kBlock) {
     const int r = e / NB, cb = e - r * NB;
     float x[8];
 #pragma unroll
@@ -1291,13 +1290,15 @@ struct Images {
   PrepJobs jobs{};
   int n_jobs = 0, max_rows = 0;
   bool none = false;  // no images: the fp32 bodies read the matrices themselves
-  Mat add(const void* x, int n, float scale, bool want_t) {
+  Mat add(const void* x, int n, float scale, bool want_row, bool want_t) {
     if (none) return Mat{x, nullptr, nullptr, nullptr, n, scale};
     PrepJob& j = jobs.j[n_jobs++];
     j.x = x;
-    j.row_img = ws;
-    ws += row_image_bytes(n, H, d, np);
-    j.t_img = nullptr;
+    j.row_img = j.t_img = nullptr;
+    if (want_row) {
+      j.row_img = ws;
+      ws += row_image_bytes(n, H, d, np);
+    }
     if (want_t) {
       j.t_img = ws;
       ws += t_image_bytes(n, H, d, np);
@@ -1420,7 +1421,7 @@ bool few_scores(int dtype, int n_q, int n_k, int H, int d) {
 size_t fx_fwd_image_bytes(int dtype, int n_q, int n_k, int H, int d) {
   if (few_scores(dtype, n_q, n_k, H, d)) return 0;
   const int np = dtype == NGT_F32 ? 3 : 1;
-  return row_image_bytes(n_q, H, d, np) + flag_bytes(n_q, H) + 2 * row_image_bytes(n_k, H, d, np) +
+  return row_image_bytes(n_q, H, d, np) + flag_bytes(n_q, H) + row_image_bytes(n_k, H, d, np) +
          t_image_bytes(n_k, H, d, np) + 2 * flag_bytes(n_k, H);
 }
 size_t fx_bwd_image_bytes(int dtype, int n_q, int n_k, int H, int d) {
@@ -1446,9 +1447,9 @@ int fx_dense_fwd(int dtype, int d, const void* q, const void* k, const void* v, 
   im.none = few_scores(dtype, n_q, n_k, H, d);
   FwdArgs a{};
   drop_terms(dm, &a.thr16, &a.drop_scale);
-  a.q = im.add(q, n_q, scale, false);
-  a.k = im.add(k, n_k, 1.f, false);
-  a.v = im.add(v, n_k, a.drop_scale, true);
+  a.q = im.add(q, n_q, scale, true, false);
+  a.k = im.add(k, n_k, 1.f, true, false);
+  a.v = im.add(v, n_k, a.drop_scale, false, true);
   a.H = H;
   if (dm) a.dm = *dm;
   a.out = out, a.out32 = out32, a.lse = lse;
@@ -1476,10 +1477,10 @@ int fx_dense_bwd(int dtype, int d, const void* q, const void* k, const void* v, 
   im.none = few_scores(dtype, n_q, n_k, H, d);
   BwdArgs a{};
   drop_terms(dm, &a.thr16, &a.drop_scale);
-  a.q = im.add(q, n_q, scale, true);
-  a.g = im.add(go, n_q, a.drop_scale, true);
-  a.k = im.add(k, n_k, 1.f, true);
-  a.v = im.add(v, n_k, 1.f, false);
+  a.q = im.add(q, n_q, scale, true, true);
+  a.g = im.add(go, n_q, a.drop_scale, true, true);
+  a.k = im.add(k, n_k, 1.f, true, true);
+  a.v = im.add(v, n_k, 1.f, true, false);
   a.H = H;
   if (dm) a.dm = *dm;
   a.out = out, a.out32 = out32, a.lse = lse, a.dsum = dsum, a.scale = scale;

@@ -281,3 +281,17 @@ def test_wgrad_rule(rows, n_out, n_in, pays):
     assert lib.ngt_wgrad_pays(rows, n_out, n_in) == pays
     if pays:
         assert lib.ngt_wgrad_workspace_bytes(rows, n_out, n_in, C.byref(C.c_size_t())) == 0
+
+
+def test_dense_fp32_forward_keeps_only_the_images_it_reads():
+    """Above 2^25 scores: rows of q and k (48 bytes each at d = 8), the transposed
+    lines of v (2,560 bytes per 32 rows) and a word per 32 rows of each."""
+    lib = _lib.load()
+    fb = C.c_size_t()
+    n_q, n_k, H = 40000, 1000, 8
+    assert lib.ngt_dense_workspace_bytes(0, n_q, n_k, H, 8, 0, C.byref(fb), None) == 0
+    a256 = lambda x: (x + 255) // 256 * 256
+    steps_q, steps_k = n_q // 32, 1024 // 32
+    assert fb.value == (a256(32 * steps_q * H * 48) + a256(32 * steps_k * H * 48)
+                        + a256(steps_k * H * 2560) + a256(steps_q * H * 4)
+                        + 2 * a256(steps_k * H * 4))
