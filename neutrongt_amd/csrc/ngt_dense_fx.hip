@@ -188,6 +188,20 @@ struct Mat {
   float scale;          // of x (in the images of fp32 inputs already)
 };
 
+// The low N bits of x, each set where some thread of the block has it; a barrier.
+template <int N>
+__device__ __forceinline__ uint32_t or_over_block(uint32_t x, uint32_t (&waves)[kWaves]) {
+  uint32_t w = 0u;
+#pragma unroll
+  for (int i = 0; i < N; ++i) w |= __ballot(x >> i & 1u) ? 1u << i : 0u;
+  waves[tid_x() >> 6] = w;  // one value, whichever lane writes last
+  __syncthreads();
+  w = waves[0];
+#pragma unroll
+  for (int i = 1; i < kWaves; ++i) w |= waves[i];
+  return w;
+}
+
 // -------------------------------------------------------------- preparation
 constexpr uint32_t kSpecialValue = 1u;  // some value has no three pieces
 constexpr uint32_t kNonzeroValue = 2u, kPlainValue = 4u;  // some value is not 0, not below 2^-40
@@ -228,10 +242,8 @@ __global__ __launch_bounds__(kBlock) void k_fx_prep(const PrepJobs jobs, int32_t
     if (u != 0u) mark |= kNonzeroValue;
     if (u >= __float_as_uint(kFaint)) mark |= kPlainValue;
   }
-  uint32_t word = 0u;
-#pragma unroll
-  for (uint32_t bit = kSpecialValue; bit <= kPlainValue; bit *= 2)
-    if (__syncthreads_or(int(mark & bit))) word |= bit;
+  __shared__ uint32_t waves[kWaves];
+  const uint32_t word = or_over_block<3>(mark, waves);
   if (tid_x() == 0) job.flag[int64_t(h) * (n_pad / kStep) + step] = word;
   constexpr int NB = col_blocks(DH);
   for (int e = tid_x(); job.row_img && e < kStep * NB; e += kBlock) {
@@ -277,23 +289,24 @@ __device__ __forceinline__ uint32_t marks(const Mat& m, int h) {
 }
 // Whether head h of these matrices takes the fp32 body (the same answer in every
 // thread of the block).  Without images (few_scores) all do.
-__device__ __forceinline__ bool any_special(const Mat& a, const Mat& b, const Mat& c, int h) {
-  if (!a.flag) return true;
-  return __syncthreads_or(int((marks(a, h) | marks(b, h) | marks(c, h)) & kSpecialValue)) != 0;
+__device__ __forceinline__ bool forward_plain(const Mat& q, const Mat& k, const Mat& v, int h,
+                                              uint32_t (&waves)[kWaves]) {
+  if (!q.flag) return true;
+  return or_over_block<1>(marks(q, h) | marks(k, h) | marks(v, h), waves) != 0u;
 }
 // The same for the backward, whose dS = p (dO . v - D) is split into pieces too:
 // with dO or v below 2^-40 everywhere (zeros alone do no harm) it could lie below
 // 2^-110 where it counts.  With one value of each past that, the largest dS lies
 // past 2^-80 p and what the pieces drop is below 2^-133.
 __device__ __forceinline__ bool backward_plain(const Mat& q, const Mat& k, const Mat& v,
-                                               const Mat& g, int h) {
-  if (any_special(q, k, v, h)) return true;
+                                               const Mat& g, int h, uint32_t (&waves)[kWaves]) {
+  if (!q.flag) return true;
   const uint32_t mg = marks(g, h), mv = marks(v, h);
-  if (__syncthreads_or(int(mg & kSpecialValue))) return true;
-  auto faint = [](uint32_t m) {
-    return __syncthreads_or(int(m & kNonzeroValue)) && !__syncthreads_or(int(m & kPlainValue));
-  };
-  return faint(mg) || faint(mv);
+  const uint32_t special = (marks(q, h) | marks(k, h) | mg | mv) & kSpecialValue;
+  const uint32_t w = or_over_block<5>(special | (mg & 6u) | (mv & 6u) << 2, waves);
+  const bool faint_g = (w & kNonzeroValue) && !(w & kPlainValue);
+  const bool faint_v = (w & kNonzeroValue << 2) && !(w & kPlainValue << 2);
+  return (w & kSpecialValue) || faint_g || faint_v;
 }
 
 // ------------------------------------------------------- fp32 MFMA products
@@ -688,30 +701,29 @@ struct FwdArgs {
 // LDS, each lane's own, which cost no registers.  250 stages added one by one at
 // 16,000 keys had moved out, and through D = dO . out dQ: 8 heads, x 5.9e-7 ->
 // 3.9e-7 and dQ 2.2e-6 -> 1.3e-6 against float64 (vector kernels 7.5e-7 and
-// 2.0e-6); the pass with dropout 4,897 -> 4,911 us, in registers 4,960.
+// 2.0e-6); the forward with dropout 1,443 -> 1,493 us (totals in registers, with
+// dQ's sums as well: 50 us more for the whole pass).
 constexpr bool run_totals(int dh) { return dh == 8; }
 template <int DH, int G>
 struct Totals {
   static constexpr int BYTES = run_totals(DH) ? G * kBlock * 20 : 0;
-  char* lds;
+  f32x4* acc_of;  // this lane's slots, kBlock apart
+  float* l_of;
   float m[G];  // the base of the totals
   bool any = false;
-  __device__ __forceinline__ f32x4& acc_of(int u) const {
-    return reinterpret_cast<f32x4*>(lds)[u * kBlock + tid_x()];
-  }
-  __device__ __forceinline__ float& l_of(int u) const {
-    return reinterpret_cast<float*>(lds + G * kBlock * 16)[u * kBlock + tid_x()];
-  }
+  __device__ __forceinline__ explicit Totals(char* lds)
+      : acc_of(reinterpret_cast<f32x4*>(lds) + tid_x()),
+        l_of(reinterpret_cast<float*>(lds + G * kBlock * 16) + tid_x()) {}
   // acc, l (base mu) += the totals
   __device__ __forceinline__ void add_to(f32x4 (&acc)[G][out_tiles(DH)], float (&l)[G],
                                          const float (&mu)[G]) const {
-    if (!any) return;
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
-      const float f = m[u] == -INFINITY ? 0.f : exp_nat(m[u] - mu[u]);
-      acc[u][0] += acc_of(u) * f;
-      l[u] += l_of(u) * f;
-    }
+    for (int u = 0; u < G; ++u)
+      if (any) {
+        const float f = m[u] == -INFINITY ? 0.f : exp_nat(m[u] - mu[u]);
+        acc[u][0] += acc_of[u * kBlock] * f;
+        l[u] += l_of[u * kBlock] * f;
+      }
   }
   // the totals += acc, l, which become zero
   __device__ __forceinline__ void take(f32x4 (&acc)[G][out_tiles(DH)], float (&l)[G],
@@ -719,8 +731,8 @@ struct Totals {
     add_to(acc, l, mu);
 #pragma unroll
     for (int u = 0; u < G; ++u) {
-      acc_of(u) = acc[u][0];
-      l_of(u) = l[u];
+      acc_of[u * kBlock] = acc[u][0];
+      l_of[u * kBlock] = l[u];
       m[u] = mu[u];
       l[u] = 0.f;
     }
@@ -759,9 +771,8 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     sk.load(a.k, k_begin, h, H);
     sv.load(a.v, k_begin, h, H);
   }
-  Totals<DH, G> tot;
-  tot.lds = lds + sk.BYTES + sv.BYTES;
-  int run = kRun;
+  Totals<DH, G> tot(lds + sk.BYTES + sv.BYTES);
+  int run = 0;  // stages since the totals were last written
   for (int kb = k_begin; kb < k_end; kb += SB) {
     __syncthreads();
     sk.store();
@@ -835,11 +846,10 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     add_acc(stage, acc);
 #pragma unroll
     for (int u = 0; u < G; ++u) l[u] += lst[u];
-    if constexpr (run_totals(DH))
-      if (--run == 0) {
-        run = kRun;
-        tot.take(acc, l, m);
-      }
+    if (run_totals(DH) && ++run == kRun && kb + SB < k_end) {
+      tot.take(acc, l, m);
+      run = 0;
+    }
   }
   if constexpr (run_totals(DH)) tot.add_to(acc, l, m);
   Ops::finish(acc);
@@ -942,9 +952,10 @@ __global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
   using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(fwd_lds<F, DH, G>(), fwd_lds<P, DH, G>())];
+  __shared__ uint32_t waves[kWaves];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
   if (bx >= (z == a.n_split ? a.score_bx : a.fwd_bx)) return;  // block-uniform, before any barrier
-  const bool plain = any_special(a.q, a.k, a.v, h);
+  const bool plain = forward_plain(a.q, a.k, a.v, h, waves);
   if (z == a.n_split) {
     if (plain)
       scores_body<F, DH, G>(a, bx, h, lds);
@@ -1097,8 +1108,9 @@ __global__ __launch_bounds__(kBlock) void k_fx_bwd_q(const BwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
   using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(bwd_q_lds<F>(), bwd_q_lds<P>())];
+  __shared__ uint32_t waves[kWaves];
   const int bx = wg_x(), h = wg_y(), z = wg_z();
-  if (backward_plain(a.q, a.k, a.v, a.g, h))
+  if (backward_plain(a.q, a.k, a.v, a.g, h, waves))
     bwd_q_body<F, T, DH, G, DROP>(a, bx, h, z, lds);
   else
     bwd_q_body<P, T, DH, G, DROP>(a, bx, h, z, lds);
@@ -1233,6 +1245,7 @@ __global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
   using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(bwd_kv_lds<F>(), bwd_kv_lds<P>())];
+  __shared__ uint32_t waves[kWaves];
   __shared__ __align__(16) float ls[64];
   __shared__ __align__(16) float ds[64];
   const int bx = wg_x(), h = wg_y();
@@ -1241,7 +1254,7 @@ __global__ __launch_bounds__(kBlock) void k_fx_bwd_kv(const BwdArgs a) {
                int64_t(a.comb_bx) * a.H);
     return;
   }
-  if (backward_plain(a.q, a.k, a.v, a.g, h))
+  if (backward_plain(a.q, a.k, a.v, a.g, h, waves))
     bwd_kv_body<F, T, DH, G, DROP>(a, bx, h, lds, ls, ds);
   else
     bwd_kv_body<P, T, DH, G, DROP>(a, bx, h, lds, ls, ds);
