@@ -142,8 +142,8 @@ def test_colsum_takes_any_width():
 
 def test_dense_workspace_query_depends_on_path_and_scores():
     """The matrix-core path (bf16, d <= 32) needs H * n_k floats of node-score
-    partials and nothing without node scores; the vector-ALU path sizes its
-    per-block partials only when node scores are wanted."""
+    partials and nothing without node scores; the fp32 one sizes its partials
+    only when node scores are wanted."""
     lib = _lib.load()
     fb, bb = C.c_size_t(), C.c_size_t()
     assert lib.ngt_dense_workspace_bytes(1, 300, 300, 8, 8, 1, C.byref(fb), C.byref(bb)) == 0

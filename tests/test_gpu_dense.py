@@ -38,7 +38,7 @@ def _qkv(n_q, n_k, H, d, dtype, seed):
     (100, 100, 8, 8, torch.bfloat16), (96, 150, 4, 16, torch.bfloat16),
     (60, 61, 2, 24, torch.bfloat16), (70, 45, 3, 32, torch.bfloat16),
     (33, 47, 2, 64, torch.bfloat16), (1, 1, 1, 8, torch.bfloat16), (130, 33, 2, 8, torch.bfloat16),
-    # long key ranges: the vector-ALU forward splits the keys over blocks
+    # long key ranges: the forward splits the keys over blocks
     # (5, 4, 2 and 3 splits, last one ragged) and combines the splits
     (100, 3000, 2, 8, torch.float32), (37, 2100, 1, 24, torch.float32),
     (64, 1300, 3, 64, torch.float32), (50, 1800, 2, 64, torch.bfloat16)])

@@ -1,9 +1,9 @@
 """A seeded sweep of random dense windows against the oracle (the
 reference's full_attention: logits q k^T sqrt(d)): sizes from 1 to 2,500
-keys, 1 to 8 heads, every head dim, fp32 (vector-ALU kernels) and bf16
-(matrix-core kernels for d <= 32, vector-ALU at 64), input scales that make
-the softmax peaked or flat, dropout, key splits, and the single-pass
-backward.  Every case is drawn from a fixed seed."""
+keys, 1 to 8 heads, every head dim, fp32 (on its own MFMAs and, where the
+tile count is asked for, on bf16 pieces) and bf16 (bf16 weights for d <= 32,
+24-bit ones at 64), input scales that make the softmax peaked or flat, dropout,
+key splits, and the single-pass backward.  Every case is drawn from a fixed seed."""
 import math
 
 import numpy as np
@@ -34,7 +34,8 @@ def _cases(n=100, seed=4242):
                         qscale=float(rng.choice([1.0, 0.25, 0.05])),
                         p=float(rng.choice([0.0, 0.0, 0.3])),
                         fwd_split=int(rng.choice([0, 0, 2, 3])), dq_split=int(rng.choice([0, 0, 2])),
-                        fused=bool(fused), seed=int(rng.integers(1 << 30))))
+                        fused=bool(fused), tiles=i % 3 if dtype == "f32" else 0,
+                        seed=int(rng.integers(1 << 30))))
     return out
 
 
@@ -42,10 +43,12 @@ def _cases(n=100, seed=4242):
 def test_random_dense_window_matches_oracle(monkeypatch, c):
     _say(f"case {c}")
     monkeypatch.setenv("NGT_DENSE_FUSED", "1" if c["fused"] else "0")
-    if c["fwd_split"]:
-        monkeypatch.setenv("NGT_MF_FWD_SPLIT", str(c["fwd_split"]))
-    if c["dq_split"]:
-        monkeypatch.setenv("NGT_MF_DQ_SPLIT", str(c["dq_split"]))
+    if c["tiles"]:
+        monkeypatch.setenv("NGT_DENSE_F32_TILES", str(c["tiles"]))
+    for family in ("MF", "DENSE_F32"):
+        for pass_ in ("fwd", "dq"):
+            if c[pass_ + "_split"]:
+                monkeypatch.setenv(f"NGT_{family}_{pass_.upper()}_SPLIT", str(c[pass_ + "_split"]))
     dtype = torch.bfloat16 if c["dtype"] == "bf16" else torch.float32
     g = torch.Generator().manual_seed(c["seed"])
     H, d, n_q, n_k, p = c["H"], c["d"], c["n_q"], c["n_k"], c["p"]

@@ -62,7 +62,7 @@ def test_sparse_graph_replay_matches_eager(H, d, dtype):
 
 @pytest.mark.parametrize("n_q,n_k,H,d,dtype", [
     (500, 500, 4, 8, torch.bfloat16),   # matrix-core kernels
-    (300, 2100, 2, 8, torch.float32),   # vector-ALU kernels, keys split over 4 blocks + combine
+    (300, 2100, 2, 8, torch.float32),   # fp32 MFMAs, keys split over blocks + combine
 ])
 def test_dense_graph_replay_matches_eager(n_q, n_k, H, d, dtype):
     print(f"case graph dense n_q={n_q} n_k={n_k} H={H} d={d} {dtype}", flush=True)
