@@ -22,6 +22,8 @@ def _both(monkeypatch, fn):
             if python:
                 m.setattr(_lib, "node_ext", lambda: None)
                 m.setattr(_lib, "autograd_ext", lambda: None)
+            else:
+                assert _lib.node_ext() is not None  # else Python would face Python
             torch.manual_seed(11)
             out.append(fn())
             torch.cuda.synchronize()
@@ -120,3 +122,16 @@ def test_parts_of_the_gradients_match_python_nodes(monkeypatch):
         return res
 
     _both(monkeypatch, run)
+
+
+def test_the_layers_run_as_cpp_nodes():
+    """Under bf16 autocast every layer's output comes from a C++ node."""
+    print("case cpp nodes", flush=True)
+    lins, ln = [_params(WgradLinear(16, 16)) for _ in range(3)], _params(FusedLayerNorm(16))
+    x = torch.randn(1, 5, 16, device=DEV, requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        outs = [lins[0](x), *project(x, *lins, heads=2), ln(x),
+                *add_dropout_layernorm(x, x, ln, torch.nn.Dropout(0.5))]
+    for y, node in zip(outs, ["Linear"] + 3 * ["Projection3"] + ["LayerNorm"] + 2 * ["AddLayerNorm"]):
+        name = y.grad_fn.name()
+        assert "CppNode" in name and node in name, name
