@@ -309,8 +309,9 @@ inline int grid_for(int64_t n) {
   return int(g);
 }
 
-int sub_prepare(bool init, int64_t n_nodes, int64_t n_items, const int64_t* set, int32_t n_set, void* ws,
-                size_t ws_bytes, hipStream_t s, int64_t* result, SubLayout* L, const char* who) {
+int sub_prepare(bool init, int64_t n_nodes, int64_t n_items, const int64_t* set, int32_t n_set,
+                void* ws, size_t ws_bytes, hipStream_t s, int64_t* result, SubLayout* L,
+                const char* who) {
   NGT_CHECK_OK(sub_layout(n_nodes, n_items, n_set, L));
   if (!ws || ws_bytes < L->total)
     return set_error(NGT_ERR_ARG, "%s: workspace too small (%zu < %zu)", who, ws_bytes, L->total);

@@ -188,8 +188,9 @@ class _ProjectionGroupFn(torch.autograd.Function):
 
     Forward: one GEMM per projection, as ``_WgradLinearFn``.  Backward: when
     the output gradients are column blocks of one [M, k * n_out] matrix (the
-    attention core's interleaved dQ/dK/dV), one GEMM each for dX (against the
-    stacked weights), dW (split-K, fp32) and db (one column sum).  Otherwise
+    attention core's interleaved dQ/dK/dV), one GEMM for dX (against the
+    stacked weights), and dW and db in fp32 from _grads: one pass over the rows
+    where _fused says so, else split-K GEMMs and a column sum.  Otherwise
     dX is accumulated by the GEMMs themselves (dX = dY_0 W_0, then dX +=
     dY_i W_i with the library's beta = 1), where separate nodes would leave
     autograd to add their bf16 dX tensors with elementwise kernels (two extra

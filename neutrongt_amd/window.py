@@ -184,12 +184,12 @@ _SUBGRAPH_ERRORS = {1: "node id out of range in the node set", 2: "duplicate nod
                     4: "edge endpoint out of range", 8: "CSR row outside col"}
 
 
-def _subgraph_job(call, n_nodes: int, n_edges: int, n_set: int, device, stream, host):
+def _subgraph_job(calls, n_nodes: int, n_edges: int, n_set: int, device, stream, host):
     """Count pass, the count copied into ``host`` (pinned) asynchronously, a
     yield, then the emit pass into an exact [2, n] tensor, from the map and
     counts that the count pass left in the workspace: a job of
-    _streams.run_in_flight.  ``call`` = (count, emit) entry points."""
-    count, emit = call
+    _streams.run_in_flight.  ``calls`` = (count, emit) entry points."""
+    count, emit = calls
     lib = _lib.load()
     nb = C.c_size_t()
     _lib.check(lib.ngt_subgraph_workspace_bytes(n_nodes, n_edges, n_set, C.byref(nb)))
@@ -224,10 +224,13 @@ def _coo_call(subset: torch.Tensor, edge_index: torch.Tensor, num_nodes: int):
     subset = subset.to(torch.int64).contiguous()
     ei = edge_index.to(torch.int64).contiguous()
     E, n_set = int(ei.shape[1]), int(subset.numel())
-    call = lambda fn: lambda out, cap, res, ws, wb, st: fn(  # noqa: E731
-        ei.data_ptr(), E, int(num_nodes), subset.data_ptr(), n_set, out, cap, res, ws, wb, st)
-    return functools.partial(_subgraph_job,
-                             (call(lib.ngt_subgraph_coo), call(lib.ngt_subgraph_coo_emit)), int(num_nodes), E, n_set, subset.device)
+
+    def run(fn, *rest):  # rest: out, cap, result, workspace, its bytes, stream
+        return fn(ei.data_ptr(), E, int(num_nodes), subset.data_ptr(), n_set, *rest)
+
+    calls = tuple(functools.partial(run, fn)
+                  for fn in (lib.ngt_subgraph_coo, lib.ngt_subgraph_coo_emit))
+    return functools.partial(_subgraph_job, calls, int(num_nodes), E, n_set, subset.device)
 
 
 def _csr_call(node_set: torch.Tensor, rowptr: torch.Tensor, col: torch.Tensor):
@@ -240,11 +243,14 @@ def _csr_call(node_set: torch.Tensor, rowptr: torch.Tensor, col: torch.Tensor):
     n_nodes, n_set = int(rowptr.numel()) - 1, int(node_set.numel())
     if n_nodes < 0:
         raise ValueError("subgraph_from_csr: rowptr must have n_nodes + 1 entries")
-    call = lambda fn: lambda out, cap, res, ws, wb, st: fn(  # noqa: E731
-        rowptr.data_ptr(), col.data_ptr(), int(col.numel()), n_nodes, node_set.data_ptr(), n_set,
-        out, cap, res, ws, wb, st)
-    return functools.partial(_subgraph_job,
-                             (call(lib.ngt_subgraph_csr), call(lib.ngt_subgraph_csr_emit)), n_nodes, int(col.numel()), n_set,
+
+    def run(fn, *rest):  # rest: out, cap, result, workspace, its bytes, stream
+        return fn(rowptr.data_ptr(), col.data_ptr(), int(col.numel()), n_nodes,
+                  node_set.data_ptr(), n_set, *rest)
+
+    calls = tuple(functools.partial(run, fn)
+                  for fn in (lib.ngt_subgraph_csr, lib.ngt_subgraph_csr_emit))
+    return functools.partial(_subgraph_job, calls, n_nodes, int(col.numel()), n_set,
                              node_set.device)
 
 
