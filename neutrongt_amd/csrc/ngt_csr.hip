@@ -84,7 +84,9 @@ hipError_t sort_with(void* temp, size_t& bytes, uint32_t* key_in, uint32_t* key_
 // Radix passes clear their counters with memsets, which replays of a captured
 // graph do not repeat reliably: under capture every sort is a merge sort, kernels
 // only.  (The library's default takes radix passes above a million entries, and
-// the row sort below holds both sides' rows.)
+// the row sort below holds both sides' rows.)  That costs a captured build, eager
+// against replay: 0.67 M edges of 16,384 nodes 242 / 391 us, 1.8 M of 32,768 387 /
+// 612, 3.6 M of 65,000 551 / 791.
 using KernelsOnly = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
                                                rocprim::default_config, (size_t(1) << 32)>;
 bool capturing(hipStream_t st) {
