@@ -701,45 +701,14 @@ struct FwdArgs {
 // LDS, each lane's own, which cost no registers.  250 stages added one by one at
 // 16,000 keys had moved out, and through D = dO . out dQ: 8 heads, x 5.9e-7 ->
 // 3.9e-7 and dQ 2.2e-6 -> 1.3e-6 against float64 (vector kernels 7.5e-7 and
-// 2.0e-6); the forward with dropout 1,443 -> 1,493 us (totals in registers, with
-// dQ's sums as well: 50 us more for the whole pass).
+// 2.0e-6); the forward with dropout 1,408 -> 1,449 us.  With the totals in
+// registers it took 134 of them for 111 and the whole pass 50 us more; as a
+// struct's members passed by reference 1,480 us.
 constexpr bool run_totals(int dh) { return dh == 8; }
 template <int DH, int G>
-struct Totals {
-  static constexpr int BYTES = run_totals(DH) ? G * kBlock * 20 : 0;
-  f32x4* acc_of;  // this lane's slots, kBlock apart
-  float* l_of;
-  float m[G];  // the base of the totals
-  bool any = false;
-  __device__ __forceinline__ explicit Totals(char* lds)
-      : acc_of(reinterpret_cast<f32x4*>(lds) + tid_x()),
-        l_of(reinterpret_cast<float*>(lds + G * kBlock * 16) + tid_x()) {}
-  // acc, l (base mu) += the totals
-  __device__ __forceinline__ void add_to(f32x4 (&acc)[G][out_tiles(DH)], float (&l)[G],
-                                         const float (&mu)[G]) const {
-#pragma unroll
-    for (int u = 0; u < G; ++u)
-      if (any) {
-        const float f = m[u] == -INFINITY ? 0.f : exp_nat(m[u] - mu[u]);
-        acc[u][0] += acc_of[u * kBlock] * f;
-        l[u] += l_of[u * kBlock] * f;
-      }
-  }
-  // the totals += acc, l, which become zero
-  __device__ __forceinline__ void take(f32x4 (&acc)[G][out_tiles(DH)], float (&l)[G],
-                                       const float (&mu)[G]) {
-    add_to(acc, l, mu);
-#pragma unroll
-    for (int u = 0; u < G; ++u) {
-      acc_of[u * kBlock] = acc[u][0];
-      l_of[u * kBlock] = l[u];
-      m[u] = mu[u];
-      l[u] = 0.f;
-    }
-    zero_acc(acc);
-    any = true;
-  }
-};
+constexpr int totals_bytes() {
+  return run_totals(DH) ? G * kBlock * 20 : 0;
+}
 template <class Ops, typename T, int DH, int G, bool DROP>
 __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z, char* lds) {
   constexpr int SB = Ops::SB, MT = out_tiles(DH);
@@ -771,8 +740,22 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
     sk.load(a.k, k_begin, h, H);
     sv.load(a.v, k_begin, h, H);
   }
-  Totals<DH, G> tot(lds + sk.BYTES + sv.BYTES);
+  // this lane's slots of the totals, kBlock apart, and their base
+  f32x4* const tot = reinterpret_cast<f32x4*>(lds + sk.BYTES + sv.BYTES) + tid_x();
+  float* const tot_l =
+      reinterpret_cast<float*>(lds + sk.BYTES + sv.BYTES + G * kBlock * 16) + tid_x();
+  float m_tot[G];
+  auto add_totals = [&](bool any) {  // acc, l += the totals
+#pragma unroll
+    for (int u = 0; u < G; ++u)
+      if (any) {
+        const float f = m_tot[u] == -INFINITY ? 0.f : exp_nat(m_tot[u] - m[u]);
+        acc[u][0] += tot[u * kBlock] * f;
+        l[u] += tot_l[u * kBlock] * f;
+      }
+  };
   int run = 0;  // stages since the totals were last written
+  bool any = false;
   for (int kb = k_begin; kb < k_end; kb += SB) {
     __syncthreads();
     sk.store();
@@ -847,11 +830,20 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
 #pragma unroll
     for (int u = 0; u < G; ++u) l[u] += lst[u];
     if (run_totals(DH) && ++run == kRun && kb + SB < k_end) {
-      tot.take(acc, l, m);
+      add_totals(any);
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        tot[u * kBlock] = acc[u][0];
+        tot_l[u * kBlock] = l[u];
+        m_tot[u] = m[u];
+        l[u] = 0.f;
+      }
+      zero_acc(acc);
       run = 0;
+      any = true;
     }
   }
-  if constexpr (run_totals(DH)) tot.add_to(acc, l, m);
+  if constexpr (run_totals(DH)) add_totals(any);
   Ops::finish(acc);
   const float ds = DROP && !Ops::SCALED ? a.drop_scale : 1.f;
 #pragma unroll
@@ -941,7 +933,7 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
 template <class Ops, int DH, int G>
 constexpr int fwd_lds() {
   return Ops::template Staged<true, false>::BYTES + Ops::template Staged<false, true>::BYTES +
-         Totals<DH, G>::BYTES;
+         totals_bytes<DH, G>();
 }
 
 // The forward and the column scores in one launch: grid z < n_split are
