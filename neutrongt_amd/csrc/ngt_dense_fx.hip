@@ -19,10 +19,10 @@
 // pieces and, with dropout, the hash.
 // Measured (us per launch, forward with node scores / dK/dV / dQ; the earlier
 // one-row-per-lane vector kernels -> these): 16,000 nodes, 8 heads, d = 8
-// 1,720 / 2,490 / 1,680 -> 1,060 / 1,780 / 1,030, with dropout 0.5 2,150 /
-// 2,810 / 1,980 -> 1,400 / 2,215 / 1,370; all-fp32 MFMAs 1,390 / 1,900 /
+// 1,720 / 2,490 / 1,680 -> 1,080 / 1,545 / 970, with dropout 0.5 2,150 /
+// 2,810 / 1,980 -> 1,420 / 2,100 / 1,370; all-fp32 MFMAs 1,390 / 1,900 /
 // 1,300.  5,000 nodes, 8 heads, d = 64: 8,400 in all -> 650 / 1,210 / 555; the
-// same in bf16 (one piece per operand) 1,570 / 5,870 / 2,970 -> 275 / 635 / 290.
+// same in bf16 (one piece per operand) 1,570 / 5,870 / 2,970 -> 275 / 630 / 290.
 //
 // A preparation kernel (k_fx_prep) writes the pieces of q * scale, k, v and dO
 // once per call, each matrix in the images that the pass reads:
