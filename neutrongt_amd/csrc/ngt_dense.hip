@@ -40,13 +40,14 @@ int mfma_dense_bwd(int d, const void* q, const void* k, const void* v, const voi
                    MfSplit sq, float* part_dq, int fused_blocks, hipStream_t st);
 // fp32 (and bf16, d = 64) matrix-core kernels (ngt_dense_fx.hip).
 MfSplit fx_fwd_split(int n_q, int n_k, int H, int d, bool node_scores);
+MfSplit fx_score_split(int n_q, MfSplit keys);
 MfSplit fx_dq_split(int n_q, int n_k, int H, int d);
 size_t fx_fwd_image_bytes(int dtype, int n_q, int n_k, int H, int d);
 size_t fx_bwd_image_bytes(int dtype, int n_q, int n_k, int H, int d);
 int fx_dense_fwd(int dtype, int d, const void* q, const void* k, const void* v, int n_q, int n_k,
                  int H, float scale, const DropoutMask* dm, void* out, float* out32, float* lse,
-                 float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
-                 hipStream_t st);
+                 float* part, MfSplit sp, MfSplit scores, float* part_ml, float* part_acc,
+                 char* images, hipStream_t st);
 int fx_dense_bwd(int dtype, int d, const void* q, const void* k, const void* v, const void* go,
                  const void* out, const float* out32, const float* lse, float* dsum, int n_q,
                  int n_k, int H, float scale, const DropoutMask* dm, void* gq, void* gk, void* gv,
@@ -92,11 +93,14 @@ __global__ __launch_bounds__(kBlock) void k_dense_combine(
 
 // node_score[j] = sum over rows of ns_part[:, j] / H.  A block of 1024
 // threads takes 64 keys (lane = key) and splits the rows over its 16 waves
-// (wave w: rows w, w + 16, ...); the waves' sums are added in wave order.
+// (wave w: rows w, w + 16, ...); the waves' sums are added in wave order, or with
+// PAIRS, where the rows are many (query splits), by halves: 8,000 queries in 32
+// splits, 4 heads of 32, 6.6e-8 -> 4.0e-8 of float64.
 // One thread per key down all rows (2,000 at 16,000 nodes, 8 heads) left the
 // loads' latency exposed: 466 us for 128 MB.
 constexpr int kScoreThreads = 1024;
 constexpr int kScoreWaves = kScoreThreads / kWave;
+template <bool PAIRS>
 __global__ __launch_bounds__(kScoreThreads) void k_dense_scores(
     const float* __restrict__ part, int32_t rows, int32_t n_k, int32_t H, float* __restrict__ ns) {
   __shared__ float red[kScoreWaves][kWave];
@@ -111,10 +115,19 @@ __global__ __launch_bounds__(kScoreThreads) void k_dense_scores(
   red[w][lane] = s;
   __syncthreads();
   if (w == 0 && j < n_k) {
-    float t = red[0][lane];
+    float t[kScoreWaves];
 #pragma unroll
-    for (int u = 1; u < kScoreWaves; ++u) t += red[u][lane];
-    ns[j] = t / float(H);
+    for (int u = 0; u < kScoreWaves; ++u) t[u] = red[u][lane];
+    if (PAIRS) {
+#pragma unroll
+      for (int n = kScoreWaves / 2; n > 0; n /= 2)
+#pragma unroll
+        for (int u = 0; u < n; ++u) t[u] += t[u + n];
+    } else {
+#pragma unroll
+      for (int u = 1; u < kScoreWaves; ++u) t[0] += t[u];
+    }
+    ns[j] = t[0] / float(H);
   }
 }
 
@@ -137,18 +150,19 @@ int check_args(const char* fn, int dtype, int n_q, int n_k, int H, int d) {
 // ngt_dense_fx.hip.
 bool use_bf16(int dtype, int d) { return dtype == NGT_BF16 && mfma_dense_supported(d); }
 
-// Forward workspace: [node-score partials H * n_k (with node scores)][split
+// Forward workspace: [node-score partials, per query split H * n_k][split
 // states (m, l) and unnormalised outputs (with a key split)][the operands'
 // pieces (ngt_dense_fx.hip)].
 struct FwdLayout {
   size_t ml, acc, images, total;
-  MfSplit sp;
+  MfSplit sp, scores;  // of the keys; of the node scores' queries
 };
 FwdLayout fwd_layout(int dtype, int32_t n_q, int32_t n_k, int32_t H, int32_t d, bool node_scores) {
   FwdLayout L{};
   const bool b16 = use_bf16(dtype, d);
   L.sp = b16 ? mfma_fwd_split(n_q, n_k, H, node_scores) : fx_fwd_split(n_q, n_k, H, d, node_scores);
-  size_t off = node_scores ? align256(size_t(H) * n_k * 4) : 0;
+  L.scores = b16 ? MfSplit{1, n_q} : fx_score_split(n_q, L.sp);
+  size_t off = node_scores ? align256(size_t(L.scores.n_split) * H * n_k * 4) : 0;
   if (L.sp.n_split > 1) {
     L.ml = off;
     off += align256(size_t(L.sp.n_split) * n_q * H * 8);
@@ -264,15 +278,16 @@ extern "C" int ngt_dense_fwd(int dtype, const void* q, const void* k, const void
                         L.sp, part_ml, part_acc, st);
   else
     rc = fx_dense_fwd(dtype, head_dim, q, k, v, n_q, n_k, n_heads, scale, dm, out, out_f32, lse,
-                      part, L.sp, part_ml, part_acc, ws + L.images, st);
+                      part, L.sp, L.scores, part_ml, part_acc, ws + L.images, st);
   if (rc != NGT_OK) return rc;
   if (L.sp.n_split > 1)
     NGT_CHECK_OK((dtype == NGT_F32 ? launch_combine<float> : launch_combine<bf16_t>)(
         head_dim, part_ml, part_acc, L.sp.n_split, n_q, n_heads, out, out_f32, lse, st));
   if (!node_score || n_k == 0) return NGT_OK;
   KernelTimer timer_("dense_scores", st);
-  hipLaunchKernelGGL(k_dense_scores, dim3((n_k + kWave - 1) / kWave), dim3(kScoreThreads), 0, st,
-                     part, n_heads, n_k, n_heads, node_score);
+  hipLaunchKernelGGL(L.scores.n_split > 1 ? k_dense_scores<true> : k_dense_scores<false>,
+                     dim3((n_k + kWave - 1) / kWave), dim3(kScoreThreads), 0, st, part,
+                     L.scores.n_split * n_heads, n_k, n_heads, node_score);
   NGT_HIP_CHECK(hipGetLastError());
   return NGT_OK;
 }

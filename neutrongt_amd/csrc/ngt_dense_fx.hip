@@ -686,8 +686,10 @@ struct FwdArgs {
   float *out32, *lse;
   int32_t split_keys;
   float *part_ml, *part_acc;
-  int32_t n_split, fwd_bx, score_bx;
-  float* part;
+  int32_t n_split, fwd_bx, score_bx, score_splits;
+  int32_t grid_x;      // blocks are numbered y * grid_x + x
+  int32_t score_rows;  // queries per split of the column scores
+  float* part;         // [split][H][n_k]
 };
 
 // One block: block_rows(G) queries of head h, keys of split z.  S^T = K Q^T
@@ -869,17 +871,18 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
   }
 }
 
-// Column scores part[h][j] = sum_i |S[h, i, j]|: rows = queries (staged),
-// lanes = keys.  A long column is summed in three levels: the stages of a run of
+// Column scores part[z][h][j] = sum |S[h, i, j]| over the queries of split z:
+// rows = queries (staged), lanes = keys.  A long column is summed in three levels: the stages of a run of
 // kRun are added to each other before they join the total (8,000 queries, 4 heads
 // of 32: 7.3e-8 -> 4.7e-8 of float64).
 template <class Ops, int DH, int G>
-__device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, char* lds) {
+__device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, int z, char* lds) {
   constexpr int SB = Ops::SB;
   const int lane = tid_x() & (kWave - 1);
   const int wave = tid_x() >> 6;
   const int g = lane >> 4, l16 = lane & 15;
-  const int n_q = a.q.n;
+  const int q_begin = z * a.score_rows;
+  const int q_end = min(a.q.n, q_begin + a.score_rows);
   int kj[G];
   typename Ops::Rows kf;
   float sum[G], runs[G];
@@ -891,17 +894,17 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
   }
   typename Ops::template Staged<true, false> sq;
   sq.lds = reinterpret_cast<decltype(sq.lds)>(lds);
-  sq.load(a.q, 0, h, a.H);
+  sq.load(a.q, q_begin, h, a.H);
   int run = kRun;
-  for (int qb = 0; qb < n_q; qb += SB) {
+  for (int qb = q_begin; qb < q_end; qb += SB) {
     __syncthreads();
     sq.store();
     __syncthreads();
-    if (qb + SB < n_q) sq.load(a.q, qb + SB, h, a.H);
+    if (qb + SB < q_end) sq.load(a.q, qb + SB, h, a.H);
     float st[G];
 #pragma unroll
     for (int u = 0; u < G; ++u) st[u] = 0.f;
-    for (int r0 = 0; r0 < SB && qb + r0 < n_q; r0 += kStep) {  // rows past n_q are zero
+    for (int r0 = 0; r0 < SB && qb + r0 < q_end; r0 += kStep) {  // rows past n_q are zero
       f32x4 s[2][G];
       sq.products(r0, g, l16, kf, s);
       if constexpr (!Ops::SCALED) times(s, a.q.scale);
@@ -914,7 +917,7 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
     }
 #pragma unroll
     for (int u = 0; u < G; ++u) runs[u] += st[u];
-    if (--run == 0 || qb + SB >= n_q) {
+    if (--run == 0 || qb + SB >= q_end) {
       run = kRun;
 #pragma unroll
       for (int u = 0; u < G; ++u) {
@@ -926,7 +929,7 @@ __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, cha
 #pragma unroll
   for (int u = 0; u < G; ++u) {
     const float t = sum_rows(sum[u]);
-    if (g == 0 && kj[u] < a.k.n) a.part[int64_t(h) * a.k.n + kj[u]] = t;
+    if (g == 0 && kj[u] < a.k.n) a.part[(int64_t(z) * a.H + h) * a.k.n + kj[u]] = t;
   }
 }
 
@@ -936,23 +939,30 @@ constexpr int fwd_lds() {
          totals_bytes<DH, G>();
 }
 
-// The forward and the column scores in one launch: grid z < n_split are
-// forward blocks, the last slice holds the score blocks, which fill the CUs
-// that the forward's last round leaves idle.
+// The forward and the column scores in one launch: first the forward blocks (block
+// of queries, head, key split), then the score blocks (block of keys, head, query
+// split), which fill the CUs that the forward's last round leaves idle.
 template <typename T, int DH, int G, bool DROP>
 __global__ __launch_bounds__(kBlock) void k_fx_fwd(const FwdArgs a) {
   using F = Fp32Ops<T, DH, G>;
   using P = PieceOps<T, DH, G>;
   __shared__ __align__(16) char lds[max_of(fwd_lds<F, DH, G>(), fwd_lds<P, DH, G>())];
   __shared__ uint32_t waves[kWaves];
-  const int bx = wg_x(), h = wg_y(), z = wg_z();
-  if (bx >= (z == a.n_split ? a.score_bx : a.fwd_bx)) return;  // block-uniform, before any barrier
+  int64_t id = int64_t(wg_y()) * a.grid_x + wg_x();
+  const int64_t fwd_blocks = int64_t(a.fwd_bx) * a.H * a.n_split;
+  const bool scores = id >= fwd_blocks;
+  if (scores) id -= fwd_blocks;
+  // block-uniform, before any barrier
+  if (scores && id >= int64_t(a.score_bx) * a.H * a.score_splits) return;
+  const uint32_t nx = scores ? a.score_bx : a.fwd_bx;
+  const uint32_t rest = uint32_t(id) / nx, bx = uint32_t(id) % nx;
+  const int h = rest % a.H, z = rest / a.H;
   const bool plain = forward_plain(a.q, a.k, a.v, h, waves);
-  if (z == a.n_split) {
+  if (scores) {
     if (plain)
-      scores_body<F, DH, G>(a, bx, h, lds);
+      scores_body<F, DH, G>(a, bx, h, z, lds);
     else
-      scores_body<P, DH, G>(a, bx, h, lds);
+      scores_body<P, DH, G>(a, bx, h, z, lds);
   } else if (plain) {
     fwd_body<F, T, DH, G, DROP>(a, bx, h, z, lds);
   } else {
@@ -1273,7 +1283,10 @@ MfSplit split_keys_for(int n_q, int n_k, int H, int d, int target_waves, int64_t
   const int64_t room = std::max<int64_t>(target_waves - shared_waves, 0);
   int want = base > 0 ? int((room + base / 2) / base) : 1;
   if (const char* e = getenv(env)) want = atoi(e);
-  want = std::max(1, std::min({want, 8, std::max(1, n_k / 256)}));
+  // more than 8 only where those would not give 1,024 waves (few queries: 4 heads
+  // of 32, one query, 16,000 keys, forward 73 -> 22 us)
+  const int most = base > 0 ? int(std::min<int64_t>(std::max<int64_t>(1024 / base, 8), 32)) : 8;
+  want = std::max(1, std::min({want, most, std::max(1, n_k / 256)}));
   if (want <= 1 || n_k <= 0) return {1, std::max(n_k, 1)};
   int keys = (n_k + want - 1) / want;
   keys = (keys + kPadRows - 1) / kPadRows * kPadRows;
@@ -1331,7 +1344,13 @@ template <typename T, int DH, int G>
 int fx_fwd(FwdArgs a, const DropoutMask* dm, hipStream_t st) {
   a.fwd_bx = blocks_of(a.q.n, block_rows(G));
   a.score_bx = a.part && a.k.n > 0 ? blocks_of(a.k.n, block_rows(G)) : 0;
-  const dim3 grid(std::max(a.fwd_bx, a.score_bx), a.H, a.n_split + (a.score_bx > 0 ? 1 : 0));
+  a.score_splits = a.score_bx > 0 ? blocks_of(a.q.n, a.score_rows) : 0;
+  const int64_t blocks = (int64_t(a.fwd_bx) * a.n_split + int64_t(a.score_bx) * a.score_splits) * a.H;
+  if (blocks > INT32_MAX)
+    return set_error(NGT_ERR_UNSUPPORTED, "dense: %d x %d x %d scores exceed the grid", a.q.n, a.k.n,
+                     a.H);
+  a.grid_x = int(std::min<int64_t>(blocks, 1 << 20));
+  const dim3 grid(a.grid_x, unsigned((blocks + a.grid_x - 1) / a.grid_x));
   KernelTimer timer_("dense_fwd", st);
   if (dm)
     hipLaunchKernelGGL((k_fx_fwd<T, DH, G, true>), grid, dim3(kBlock), 0, st, a);
@@ -1399,8 +1418,22 @@ int fx_backward(const BwdArgs& a, const Images& im, const DropoutMask* dm, hipSt
 
 MfSplit fx_fwd_split(int n_q, int n_k, int H, int d, bool node_scores) {
   const int rows = block_rows(tiles_per_wave(n_k, H, d));
-  const int64_t score_waves = node_scores ? int64_t(blocks_of(n_k, rows)) * H * kWaves : 0;
+  // the score blocks' waves weigh as their rows do against the forward's
+  const double weight = node_scores && n_k > 0 ? double(std::min(n_q, n_k)) / n_k : 0.0;
+  const int64_t score_waves = int64_t(weight * blocks_of(n_k, rows) * H * kWaves);
   return split_keys_for(n_q, n_k, H, d, 6144, score_waves, "NGT_DENSE_F32_FWD_SPLIT");
+}
+// Queries per block of the column scores: about the rows that a forward block
+// streams, so that neither outlasts the other, and at least 256.  With all
+// queries in one block a forward over few keys waited for it (us, vector kernels /
+// one block / so): 8 heads of 8, 30,000 queries, 64 keys 40 / 394 / 28; 16,000 and
+// 1,000 143 / 260 / 103; 2,500 and 2,500 67 / 79 / 66.  Of the 28, numbering the
+// blocks without gaps is worth 39 (empty ones exited at once, 220,000 of them).
+MfSplit fx_score_split(int n_q, MfSplit keys) {
+  const int rows = std::max(256, keys.split_keys);
+  const int want = std::min(std::max(blocks_of(n_q, rows), 1), 1024);
+  const int per = blocks_of(blocks_of(n_q, want), kPadRows) * kPadRows;
+  return {std::max(blocks_of(n_q, per), 1), std::max(per, kPadRows)};
 }
 MfSplit fx_dq_split(int n_q, int n_k, int H, int d) {
   return split_keys_for(n_q, n_k, H, d, 6144, 0, "NGT_DENSE_F32_DQ_SPLIT");
@@ -1416,10 +1449,16 @@ MfSplit fx_dq_split(int n_q, int n_k, int H, int d) {
 // d = 8 and 24 the times cross one power later (2^26 272 / 225 and 463 / 404), but
 // the pieces are the more exact there (8 heads of 8, 2,500 nodes: x 3.1e-7 against
 // 5.2e-7), so the line stays at 2^25.
+// Up to 128 rows on one side an image's row is read by a block or two, and the
+// preparation of the other side's is most of the work: 32 heads of 24, 23,170
+// queries, 128 keys, forward 256 / 189 (forward and backward 2,209 / 1,568); 128
+// queries, 23,170 keys 405 / 187 (1,177 / 659); 8 of 8, 92,681 and 128 135 / 99; at
+// 256 173 / 174 and 101 / 89.
 // NGT_DENSE_F32_TILES asks for the pieces.
 bool few_scores(int dtype, int n_q, int n_k, int H, int d) {
   return dtype == NGT_F32 && !getenv("NGT_DENSE_F32_TILES") &&
-         int64_t(n_q) * n_k <= (int64_t(1) << (d == 64 ? 22 : 25)) / std::max(H, 1);
+         (std::min(n_q, n_k) <= 128 ||
+          int64_t(n_q) * n_k <= (int64_t(1) << (d == 64 ? 22 : 25)) / std::max(H, 1));
 }
 
 // Bytes of the images and flags that the two directions keep in the workspace.
@@ -1446,8 +1485,8 @@ static void drop_terms(const DropoutMask* dm, uint32_t* thr16, float* scale) {
 
 int fx_dense_fwd(int dtype, int d, const void* q, const void* k, const void* v, int n_q, int n_k,
                  int H, float scale, const DropoutMask* dm, void* out, float* out32, float* lse,
-                 float* part, MfSplit sp, float* part_ml, float* part_acc, char* images,
-                 hipStream_t st) {
+                 float* part, MfSplit sp, MfSplit scores, float* part_ml, float* part_acc,
+                 char* images, hipStream_t st) {
   Images im{images, H, d, dtype == NGT_F32 ? 3 : 1};
   im.none = few_scores(dtype, n_q, n_k, H, d);
   FwdArgs a{};
@@ -1460,6 +1499,7 @@ int fx_dense_fwd(int dtype, int d, const void* q, const void* k, const void* v, 
   a.out = out, a.out32 = out32, a.lse = lse;
   a.split_keys = sp.split_keys;
   a.n_split = sp.n_split;
+  a.score_rows = scores.split_keys;
   if (sp.n_split > 1) a.part_ml = part_ml, a.part_acc = part_acc;
   a.part = part;
   if (dtype == NGT_BF16 && d == 64) return fx_forward<bf16_t, 64>(a, im, dm, st);

@@ -283,6 +283,27 @@ def test_wgrad_rule(rows, n_out, n_in, pays):
         assert lib.ngt_wgrad_workspace_bytes(rows, n_out, n_in, C.byref(C.c_size_t())) == 0
 
 
+@pytest.mark.parametrize("dtype,H,d", [(0, 8, 8), (0, 1, 64), (1, 8, 64)])
+def test_dense_forward_is_split_for_lopsided_windows(dtype, H, d):
+    """Few keys under many queries: the node scores' queries over several blocks;
+    few queries: the keys, with node scores as without."""
+    lib = _lib.load()
+    fb = C.c_size_t()
+
+    def size(n_q, n_k, scores):
+        assert lib.ngt_dense_workspace_bytes(dtype, n_q, n_k, H, d, scores, C.byref(fb), None) == 0
+        return fb.value
+
+    assert size(30000, 64, 1) - size(30000, 64, 0) >= 16 * H * 64 * 4
+    states = 8 * H * 8 + 8 * H * d * 4  # 8 splits' (m, l) and outputs of one query
+    assert size(1, 16000, 1) - size(1, 16000, 0) <= H * 16000 * 4 + 256
+    assert size(1, 16000, 0) >= states
+    if dtype == 0:  # up to 128 rows on a side: no images
+        split = lambda n: (n * H * 8 + 255) // 256 * 256 + (n * H * d * 4 + 255) // 256 * 256
+        assert size(128, 1 << 20, 0) in [split(128 * s) for s in range(1, 33)]
+        assert size(129, 1 << 20, 0) > split(129 * 32)
+
+
 def test_dense_fp32_forward_keeps_only_the_images_it_reads():
     """Above 2^25 scores: rows of q and k (48 bytes each at d = 8), the transposed
     lines of v (2,560 bytes per 32 rows) and a word per 32 rows of each."""

@@ -193,3 +193,20 @@ def test_small_operands_keep_their_bits(monkeypatch, d, shift):
            *(r.transpose(0, 1) for r in ref))
     for name, a, b in zip(("x", "node_scores", "dq", "dk", "dv"), got, ref):
         assert relerr(a, b) < 3e-7 * d + 1e-6, name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n_q,n_k", [(257, 3), (512, 64), (5001, 70), (30000, 64), (1, 2000), (700, 2500)])
+def test_node_scores_of_split_queries(dtype, n_q, n_k):
+    """d = 64: the node scores' queries over several blocks of 256 or more, the
+    last one ragged; fp32 sums."""
+    print(f"case dense node score splits {dtype} n_q={n_q} n_k={n_k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n_q)
+    q, k = (torch.randn(n, 3, 64, device="cuda", generator=g).to(dtype) for n in (n_q, n_k))
+    x, ns = dense_attention(q, k, k)
+    again, ns2 = dense_attention(q, k, k)
+    assert torch.equal(ns, ns2) and torch.equal(x, again)
+    Q, K = (t.double().transpose(0, 1).contiguous() for t in (q, k))
+    S = 8.0 * Q @ K.transpose(1, 2).contiguous()
+    assert relerr(ns, S.abs().sum(1).mean(0)) < 1e-7
+    assert relerr(x, (torch.softmax(S, -1) @ K).transpose(0, 1)) < (2e-5 if dtype == torch.float32 else 2e-2)

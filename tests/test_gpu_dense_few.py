@@ -1,5 +1,6 @@
 """fp32 dense attention where its products change: fp32 MFMAs on the matrices
-themselves up to 2^25 scores (2^22 at d = 64), bf16 pieces above."""
+themselves up to 2^25 scores (2^22 at d = 64) or 128 rows on one side, bf16
+pieces above."""
 import math
 
 import pytest
@@ -32,7 +33,10 @@ def _run(n_q, n_k, H, d, seed=0):
 # relative error of p: 1.5e-6 at d = 8 to 2e-5 at d = 64.
 @pytest.mark.parametrize("n_q,n_k,H,d", [(2048, 2048, 8, 8), (2048, 2049, 8, 8), (1023, 1025, 32, 24),
                                          (1025, 1024, 32, 24), (724, 724, 8, 64), (724, 725, 8, 64),
-                                         (1, 3, 1, 16), (4100, 33, 2, 32)])
+                                         (1, 3, 1, 16), (4100, 33, 2, 32),
+                                         # one side of 128 rows and of 129; few queries: more splits
+                                         (33000, 128, 8, 24), (33000, 129, 8, 24), (128, 33000, 8, 16),
+                                         (129, 33000, 8, 16), (40, 16000, 2, 32), (1000, 16000, 1, 8)])
 def test_both_sides_of_the_rule(n_q, n_k, H, d):
     print(f"case dense few n_q={n_q} n_k={n_k} H={H} d={d}", flush=True)
     got, ref, floors = _run(n_q, n_k, H, d)
