@@ -273,7 +273,9 @@ void linear_grads(const Tensor& x, const Tensor& dy, Tensor* dw, Tensor* db) {
     return;
   }
   const int64_t K = x.size(0), n_in = x.size(1), n_out = dy.size(1);
-  if (at::GradMode::is_enabled() || !g_wgrad_pays(K, n_out, n_in)) {
+  // (a vmapped backward's tensors have no storage: torch's GEMMs take them)
+  if (at::GradMode::is_enabled() || !x.has_storage() || !dy.has_storage() ||
+      !g_wgrad_pays(K, n_out, n_in)) {
     *dw = library_weight_grad(x, dy);
     if (db) *db = colsum(dy);
     return;

@@ -106,8 +106,9 @@ def _library_weight_grad(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
 def _fused(x: torch.Tensor, dy: torch.Tensor) -> bool:
     """Whether linear_grads takes these rows: where it is the faster (the rule is
     ngt_wgrad_pays; the C++ nodes ask it too), and not for a gradient that will
-    itself be differentiated, which is torch's."""
-    return (not torch.is_grad_enabled()
+    itself be differentiated or is taken under vmap (tensors without storage),
+    which is torch's."""
+    return (not torch.is_grad_enabled() and torch._C._has_storage(x) and torch._C._has_storage(dy)
             and bool(_lib.load().ngt_wgrad_pays(x.shape[0], dy.shape[1], x.shape[1])))
 
 

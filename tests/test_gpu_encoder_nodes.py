@@ -135,3 +135,22 @@ def test_the_layers_run_as_cpp_nodes():
     for y, node in zip(outs, ["Linear"] + 3 * ["Projection3"] + ["LayerNorm"] + 2 * ["AddLayerNorm"]):
         name = y.grad_fn.name()
         assert "CppNode" in name and node in name, name
+
+
+@pytest.mark.parametrize("python", [False, True])
+def test_batched_gradients_of_layers_without_a_bias(monkeypatch, python):
+    """torch.autograd.grad(is_grads_batched=True): weight and input gradients over a
+    batch of output gradients, as one at a time."""
+    print(f"case batched gradients python={python}", flush=True)
+    if python:
+        monkeypatch.setattr(_lib, "node_ext", lambda: None)
+    lins = [_params(WgradLinear(16, 24, bias=False)) for _ in range(3)]
+    x = torch.randn(50, 16, device=DEV, requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y, ys = lins[0](x), project(x, *lins)
+    for out, ins in ((y, [x, lins[0].weight]), (ys[1], [x, lins[1].weight])):
+        g = torch.randn(3, *out.shape, device=DEV).bfloat16()
+        got = torch.autograd.grad(out, ins, g, is_grads_batched=True, retain_graph=True)
+        for i in range(3):
+            for a, b in zip(got, torch.autograd.grad(out, ins, g[i], retain_graph=True)):
+                assert (a[i].double() - b.double()).norm() <= 2e-3 * b.double().norm()
