@@ -361,14 +361,15 @@ int ngt_dense_abs_colsum(int32_t n_heads, int32_t n_q, int32_t n_k, const float*
  * alone moves dQ by percents.
  * workspace: fwd_bytes / bwd_bytes from ngt_dense_workspace_bytes for the
  * same dtype, sizes and node_scores (non-zero when node_score will be passed).
- * The forward uses it for node-score partials (H * n_k floats), for per-split
- * softmax states when it splits the keys of a large window over several blocks
- * and, in fp32 above 2^25 scores n_q * n_k * H (2^22 at head_dim 64) and in bf16
- * at head_dim 64, for images of the operands in bf16 pieces, the largest part: q
- * and k by rows, v transposed, 48 to 400 and 80 to 480 bytes per row and head in
- * fp32, a third of that in bf16.  A size of 0 means none is needed.  The backward
- * uses it for D per query and head, the partial dQ of its key splits and the
- * images of q, dO and k (both kinds) and v (rows).
+ * The forward uses it for node-score partials (H * n_k floats per split of the
+ * queries), for per-split softmax states when it splits the keys over several
+ * blocks and, in fp32 above 2^25 scores n_q * n_k * H (2^22 at head_dim 64) with
+ * more than 128 rows on both sides, and in bf16 at head_dim 64, for images of the
+ * operands in bf16 pieces, the largest part: q and k by rows, v transposed, 48 to
+ * 400 and 80 to 480 bytes per row and head in fp32, a third of that in bf16.  A
+ * size of 0 means none is needed.  The backward uses it for D per query and head,
+ * the partial dQ of its key splits and the images of q, dO and k (both kinds) and
+ * v (rows).
  * seed_dev (may be NULL): a device uint64 the kernels read the seed from when
  * they start, instead of `seed`; a captured HIP graph that rewrites it before
  * each replay draws a new mask per replay.  Forward and backward must see the
