@@ -1427,8 +1427,8 @@ MfSplit fx_fwd_split(int n_q, int n_k, int H, int d, bool node_scores) {
 // streams, so that neither outlasts the other, and at least 256.  With all
 // queries in one block a forward over few keys waited for it (us, vector kernels /
 // one block / so): 8 heads of 8, 30,000 queries, 64 keys 40 / 394 / 28; 16,000 and
-// 1,000 143 / 260 / 103; 2,500 and 2,500 67 / 79 / 66.  Of the 28, numbering the
-// blocks without gaps is worth 39 (empty ones exited at once, 220,000 of them).
+// 1,000 143 / 260 / 103; 2,500 and 2,500 67 / 79 / 66.  (On a 3-d grid padded with
+// 220,000 blocks that exit at once the first took 67.)
 MfSplit fx_score_split(int n_q, MfSplit keys) {
   const int rows = std::max(256, keys.split_keys);
   const int want = std::min(std::max(blocks_of(n_q, rows), 1), 1024);
