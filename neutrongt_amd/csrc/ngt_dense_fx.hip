@@ -872,9 +872,9 @@ __device__ __forceinline__ void fwd_body(const FwdArgs& a, int bx, int h, int z,
 }
 
 // Column scores part[z][h][j] = sum |S[h, i, j]| over the queries of split z:
-// rows = queries (staged), lanes = keys.  A long column is summed in three levels: the stages of a run of
-// kRun are added to each other before they join the total (8,000 queries, 4 heads
-// of 32: 7.3e-8 -> 4.7e-8 of float64).
+// rows = queries (staged), lanes = keys.  A long column is summed in three levels:
+// the stages of a run of kRun are added to each other before they join the total
+// (8,000 queries, 4 heads of 32: 7.3e-8 -> 4.7e-8 of float64).
 template <class Ops, int DH, int G>
 __device__ __forceinline__ void scores_body(const FwdArgs& a, int bx, int h, int z, char* lds) {
   constexpr int SB = Ops::SB;
